@@ -9,8 +9,9 @@
 // KV head through LDS in blocks of 64 or 128, and folds every block into a
 // running (max, sum, output) per query, so the scores never leave the chip.
 //
-// f16 with a head size that is a multiple of 32 (32..128) takes the matrix
-// cores (v_mfma_f32_32x32x16_f16, f32 accumulation): per wave 32 queries,
+// f16 with a head size that is a multiple of 32 (32..128; padded, of 8 up to
+// 256) takes the matrix cores
+// (v_mfma_f32_32x32x16_f16, f32 accumulation): per wave 32 queries,
 // S^T = K Q^T so that each lane owns one query column and its row statistics
 // need one cross-lane exchange; the keys of a 32-key tile are read in an
 // order that swaps bits 2 and 3 of the key index, which leaves each lane
@@ -23,7 +24,8 @@
 // f32 with the same head sizes takes v_mfma_f32_32x32x2_f32 in the same
 // tiling (its own key order, f32 probabilities).  Decode steps (few query
 // rows per KV head) split the keys over many workgroups; other head sizes
-// (up to 512) take a one-wave-per-query kernel on the vector ALUs.
+// (f16 off the multiples of 8 or above 256, f32 off those of 32, up to 512)
+// take a one-wave-per-query kernel on the vector ALUs.
 //
 // Arithmetic (both kernels): scores are f32 dot products of the (widened)
 // inputs; x * scale in f32 and masking as attention_scale_mask.metal:21-41
@@ -92,7 +94,7 @@ template <int NT>
 __device__ inline uint32_t lds_swizzle(uint32_t r) {
     if constexpr (NT == 1) return (r >> 2) & 3u;
     else if constexpr (NT == 2) return ((r & 2u) << 1) | ((r >> 2) & 3u);
-    else if constexpr (NT == 4) return ((r & 3u) << 2) | ((r >> 2) & 3u);
+    else if constexpr (NT == 4 || NT == 8) return ((r & 3u) << 2) | ((r >> 2) & 3u);
     else return 0u;
 }
 
@@ -131,46 +133,113 @@ __device__ inline void dma_to_lds(i32x4 rsrc, uint32_t lds_addr, uint32_t voffse
 // below 2^3, well inside f16 and f32 range.
 constexpr float kRescaleSlack = 3.0f;
 
+// One query row by one wave with plain f32 products, as k_attention_rows
+// computes it: for rows whose output the split products leave non-finite
+// (inf - inf and 0 * inf between the parts of an infinite operand or value),
+// so that infinities and NaN come out as in unsplit arithmetic.  Lane = key
+// for the scores, lane = head elements lane + 64 t for the values; no LDS.
+// D <= 32 NT.
+template <typename T, int NT>
+__device__ inline void exact_row(const T* __restrict__ qrow, const T* __restrict__ kh,
+                                 const T* __restrict__ vh, T* __restrict__ orow, uint32_t D,
+                                 uint32_t key_end, float scale) {
+    constexpr int DT = (NT + 1) / 2;
+    const uint32_t lane = threadIdx.x % 64;
+    float o[DT];
+#pragma unroll
+    for (int t = 0; t < DT; ++t) o[t] = 0.0f;
+    float m = -INFINITY, l = 0.0f;
+    for (uint32_t base = 0; base < key_end; base += 64) {
+        float s = -INFINITY;
+        if (base + lane < key_end) {
+            const T* krow = kh + uint64_t(base + lane) * D;
+            float dot = 0.0f;
+            for (uint32_t d = 0; d < D; ++d) dot += to_float(qrow[d]) * to_float(krow[d]);
+            s = dot * scale;
+        }
+        const float m_new = fmaxf(m, wave_max_dpp(s));
+        const float alpha = m_new > m ? exp_fast(m - m_new) : 1.0f;
+        m = m_new;
+        const float e = s == -INFINITY ? 0.0f : exp_fast(s - m);
+        l = l * alpha + e;
+#pragma unroll
+        for (int t = 0; t < DT; ++t) o[t] *= alpha;
+        const uint32_t n = min(64u, key_end - base);
+        for (uint32_t j = 0; j < n; ++j) {
+            const float pj = __shfl(e, int(j), 64);
+            const T* vrow = vh + uint64_t(base + j) * D;
+#pragma unroll
+            for (int t = 0; t < DT; ++t) {
+                const uint32_t d = lane + 64 * t;
+                if (d < D) o[t] += pj * to_float(vrow[d]);
+            }
+        }
+    }
+    const float inv = 1.0f / wave_sum_dpp(l);
+#pragma unroll
+    for (int t = 0; t < DT; ++t) {
+        const uint32_t d = lane + 64 * t;
+        if (d < D) orow[d] = from_float<T>(o[t] * inv);
+    }
+}
+
+// Added to the exponent of a probability that is split into two f16 parts:
+// with kRescaleSlack its largest value is 2^15, below f16's 65504.
+constexpr float kAnyShift = 12.0f;
+
 // QW waves of 32 queries each; KSPLIT groups of such waves split the key
 // blocks of the tile between them (group g takes blocks g, g + KSPLIT, ...)
 // and merge their partial (max, sum, output) through LDS at the end.
 //
-// DMA: K and V blocks go from memory straight into LDS (buffer_load ... lds,
-// no registers), two stages deep, so the next blocks stream in while this
-// one is computed; rows are unpadded with the chunk order of lds_swizzle.
-// Otherwise blocks pass through registers into rows padded for the bank
-// layout (head size 96, whose 12 chunks a row do not swizzle onto 64 banks),
-// one block at a time.
-template <int NT, int QW, int KSPLIT, int BN, bool DMA, bool PARTIAL = false>
+// K and V blocks go from memory straight into LDS (buffer_load ... lds, no
+// registers), two stages deep, so the next blocks stream in while this one is
+// computed; rows are in the chunk order of lds_swizzle, at a power of two of
+// chunks (head sizes 65 .. 96 take 16: 12 chunks a row do not spread over the
+// 64 banks; the chunks past the head size are loads past the buffer, zeros
+// without memory traffic.  Staged through registers in rows of 12 chunks, one
+// block at a time, head size 96 took 74.6 us against 69.0 for 15 heads x
+// [4096, 4096], one MI355X).
+//
+// ANY: a head size that is a multiple of 8 but has no kernel of its own (D is
+// then the next multiple of 32, or 192 or 256 above 128): rows are read and
+// written at the run-time size, the padding is zeros in registers and LDS.
+// Those head sizes take f32 probabilities (k_attention_rows did): P enters
+// the second product as the sum of two f16 parts, hi + lo, of 2^(t - m + 12)
+// -- 22 bits, and the factor 2^12 (kAnyShift), which cancels in the division
+// by the sum, keeps lo's own bits above the f16 subnormals down to
+// probabilities of 2^-15 of the largest.  A query whose output is not finite
+// is computed again by exact_row, whose products are not split.  One MI355X,
+// 8 heads x [1021, 1021], head size 80: 475 us on k_attention_rows (a dot
+// product a lane on the vector ALUs, uncoalesced key rows), 24.4 us here; 32
+// heads x [4096, 4096]: 12.0 ms, 0.18 ms; head size 256, 8 heads x [570, 570]:
+// 645 us, 39.7 us.
+template <int NT, int QW, int KSPLIT, int BN, bool PARTIAL = false, bool ANY = false>
 __global__ __launch_bounds__(64 * QW * KSPLIT) void k_flash_attention(
     const half_t* __restrict__ q, const half_t* __restrict__ k, const half_t* __restrict__ v,
     half_t* __restrict__ out, AttnParams p) {
     constexpr int D = 32 * NT;          // head size
     constexpr int DC = D / 16;          // 16-wide slices of a head (MFMA depth)
     constexpr int KT = BN / 32;         // 32-key tiles per block
-    static_assert(!DMA || NT != 3, "no bank-spreading chunk order for 12-chunk rows");
-    // LDS rows: with DMA unpadded and swizzled; otherwise K at a stride of
-    // D + 8 halves (the 16-byte reads of 16 consecutive rows hit distinct
-    // banks), V at v_stride_tr(D).
-    constexpr int KS = DMA ? D : D + 8;
-    constexpr int VS = DMA ? D : v_stride_tr(D);
-    constexpr int NSTAGE = DMA ? 2 : 1;
+    static_assert(!ANY || !PARTIAL, "padded head sizes do not split a tile's keys over workgroups");
+    const uint32_t hd = ANY ? p.head_dim : uint32_t(D);  // elements of a row in memory
+    constexpr int RD = NT == 3 ? 128 : D;  // elements of an LDS row
+    constexpr int SW = RD / 32;            // its chunk order (lds_swizzle)
     constexpr int THREADS = 64 * QW * KSPLIT;
     constexpr int TILE_Q = 32 * QW;                    // queries per tile
-    constexpr int BLOCK_CHUNKS = BN * D / 8;           // 16-byte chunks of one K (or V) block
+    constexpr int BLOCK_CHUNKS = BN * RD / 8;          // 16-byte chunks of one K (or V) block
     constexpr int LOADS = BLOCK_CHUNKS * KSPLIT / THREADS;
-    constexpr int DMA_LOADS = 2 * LOADS;               // K and V chunks per lane (DMA)
+    constexpr int DMA_LOADS = 2 * LOADS;               // K and V chunks per lane
     constexpr int WAVES = THREADS / 64;
     constexpr int ROUNDS = BLOCK_CHUNKS / (64 * WAVES);  // DMA instructions per region
-    constexpr int ROW_CHUNKS = D / 8;
-    constexpr int KV_HALVES = BN * KS + BN * VS;       // one block of K and V
+    constexpr int ROW_CHUNKS = RD / 8;
+    constexpr int KV_HALVES = 2 * BN * RD;             // one block of K and V
     constexpr int STAGE_BYTES = KSPLIT * KV_HALVES * 2;
     constexpr int MERGE = NT * 16 + 2;                 // floats a lane hands over
-    constexpr int LDS_BYTES = NSTAGE * STAGE_BYTES > (KSPLIT - 1) * QW * 64 * MERGE * 4
-                                  ? NSTAGE * STAGE_BYTES
+    constexpr int LDS_BYTES = 2 * STAGE_BYTES > (KSPLIT - 1) * QW * 64 * MERGE * 4
+                                  ? 2 * STAGE_BYTES
                                   : (KSPLIT - 1) * QW * 64 * MERGE * 4;
     static_assert((BLOCK_CHUNKS * KSPLIT) % THREADS == 0, "blocks must split evenly");
-    static_assert(!DMA || BLOCK_CHUNKS % (64 * WAVES) == 0,
+    static_assert(BLOCK_CHUNKS % (64 * WAVES) == 0,
                   "every wave's DMA instructions cover whole regions");
     __shared__ __align__(16) unsigned char lds[LDS_BYTES];
     half_t* const kv_lds = reinterpret_cast<half_t*>(lds);
@@ -202,7 +271,7 @@ __global__ __launch_bounds__(64 * QW * KSPLIT) void k_flash_attention(
     uint32_t koff[DC];
 #pragma unroll
     for (int c = 0; c < DC; ++c)
-        koff[c] = col * KS + 8 * ((2 * c + hs) ^ (DMA ? lds_swizzle<NT>(col) : 0u));
+        koff[c] = col * RD + 8 * ((2 * c + hs) ^ lds_swizzle<SW>(col));
     uint32_t voff[2][NT];
 #pragma unroll
     for (int e2 = 0; e2 < 2; ++e2) {
@@ -210,10 +279,10 @@ __global__ __launch_bounds__(64 * QW * KSPLIT) void k_flash_attention(
 #pragma unroll
         for (int t = 0; t < NT; ++t) {
             const uint32_t ch = 2 * ((lane / 16) % 2) + (lane % 4) / 2 + 4 * t;
-            voff[e2][t] = row * VS + 8 * (ch ^ (DMA ? lds_swizzle<NT>(row) : 0u)) + 4 * (lane % 2);
+            voff[e2][t] = row * RD + 8 * (ch ^ lds_swizzle<SW>(row)) + 4 * (lane % 2);
         }
     }
-    // DMA: a stage holds, per key group, the K block then the V block
+    // A stage holds, per key group, the K block then the V block
     // (regions of BLOCK_CHUNKS 16-byte chunks).  Instruction li of a wave
     // fills 64 chunks (lane order) of region li / ROUNDS, so the region --
     // which block, K or V -- is a compile-time fact of li; the lane picks the
@@ -225,12 +294,16 @@ __global__ __launch_bounds__(64 * QW * KSPLIT) void k_flash_attention(
         const bool is_v = (li / ROUNDS) % 2;
         const uint32_t cf = ((li % ROUNDS) * WAVES + wave) * 64 + lane;  // chunk in the region
         const uint32_t r = cf / ROW_CHUNKS;
-        const uint32_t ch = (cf % ROW_CHUNKS) ^ lds_swizzle<NT>(r);
+        const uint32_t ch = (cf % ROW_CHUNKS) ^ lds_swizzle<SW>(r);
         const uint32_t key = is_v ? r : ((r & ~31u) | perm32(r & 31u));
-        dma_off[li] = key * (D * 2) + ch * 16;
+        dma_off[li] = key * (hd * 2) + ch * 16;
+        // the padding of a row: an offset past any key's, which loads zeros
+        // (use_flash_any keeps those offsets below 2^31; the padding of head
+        // size 96, 12 chunks of 16, is not read)
+        if (RD > D || ANY) dma_off[li] = ch * 8 < hd ? dma_off[li] : 0x80000000u;
     }
-    const i32x4 k_rsrc = raw_buffer(kh, p.kv_len * (D * 2));
-    const i32x4 v_rsrc = raw_buffer(vh, p.kv_len * (D * 2));
+    const i32x4 k_rsrc = raw_buffer(kh, p.kv_len * (hd * 2));
+    const i32x4 v_rsrc = raw_buffer(vh, p.kv_len * (hd * 2));
     const uint32_t lds_base = uint32_t(
         reinterpret_cast<uintptr_t>((__attribute__((address_space(3))) unsigned char*)(lds)));
 
@@ -263,10 +336,10 @@ __global__ __launch_bounds__(64 * QW * KSPLIT) void k_flash_attention(
         // too, so their arithmetic stays finite; never stored).
         const uint32_t key_limit = min(p.start + qi, p.kv_len - 1);
         h8 qf[DC];
-        const half_t* qrow = q + (uint64_t(bh) * p.q_len + (q_valid ? qi : 0)) * D + 8 * hs;
+        const half_t* qrow = q + (uint64_t(bh) * p.q_len + (q_valid ? qi : 0)) * hd + 8 * hs;
 #pragma unroll
         for (int c = 0; c < DC; ++c) {
-            if (q_valid) {
+            if (q_valid && (!ANY || 16 * c + 8 * hs < hd)) {
                 qf[c] = *reinterpret_cast<const h8*>(qrow + 16 * c);
             } else {
 #pragma unroll
@@ -280,45 +353,6 @@ __global__ __launch_bounds__(64 * QW * KSPLIT) void k_flash_attention(
         for (int t = 0; t < NT; ++t)
 #pragma unroll
             for (int r = 0; r < 16; ++r) o[t][r] = 0.0f;
-
-        h8 kreg[LOADS], vreg[LOADS];
-        bool vlive[LOADS];
-        auto load_step = [&](uint32_t step) {
-#pragma unroll
-            for (int li = 0; li < LOADS; ++li) {
-                const uint32_t chunk = threadIdx.x + THREADS * li;
-                const uint32_t blk = step * KSPLIT + chunk / BLOCK_CHUNKS;
-                const uint32_t c = chunk % BLOCK_CHUNKS;
-                const uint32_t key = blk * BN + c / ROW_CHUNKS;
-                const uint32_t d0 = (c % ROW_CHUNKS) * 8;
-                // Rows past kv_len are never read (they may hold anything): a
-                // key past the end loads row kv_len - 1 instead; its score is
-                // masked (selected to -inf) and its value row zeroed, so it
-                // adds nothing even if that row is not finite.  (The zeroing
-                // happens at the LDS store, after the compute: a select here
-                // would make the wave wait for the load now.)
-                const uint32_t row = min(key, p.kv_len - 1);
-                kreg[li] = *reinterpret_cast<const h8*>(kh + uint64_t(row) * D + d0);
-                vreg[li] = *reinterpret_cast<const h8*>(vh + uint64_t(row) * D + d0);
-                vlive[li] = key < p.kv_len;
-            }
-        };
-        auto store_step = [&](uint32_t stage) {
-#pragma unroll
-            for (int li = 0; li < LOADS; ++li) {
-                const uint32_t chunk = threadIdx.x + THREADS * li;
-                const uint32_t c = chunk % BLOCK_CHUNKS;
-                half_t* kdst = kv_lds + (stage * KSPLIT + chunk / BLOCK_CHUNKS) * KV_HALVES;
-                half_t* vdst = kdst + BN * KS;
-                const uint32_t key = c / ROW_CHUNKS;
-                const uint32_t d0 = (c % ROW_CHUNKS) * 8;
-                // K row `key` goes to LDS row perm32(key): the S^T operand of
-                // lane i is then LDS row i.
-                *reinterpret_cast<h8*>(kdst + perm32(key) * KS + d0) = kreg[li];
-                const h8 zero = {};
-                *reinterpret_cast<h8*>(vdst + key * VS + d0) = vlive[li] ? vreg[li] : zero;
-            }
-        };
 
         // DMA of one step's blocks into stage step % 2.  Keys past kv_len
         // read as zeros (the buffer ends at row kv_len): their scores are
@@ -336,33 +370,21 @@ __global__ __launch_bounds__(64 * QW * KSPLIT) void k_flash_attention(
                 const uint32_t region = li / ROUNDS, round = li % ROUNDS;
                 dma_to_lds(is_v ? v_rsrc : k_rsrc,
                            wave_lds + 16 * (region * BLOCK_CHUNKS + round * WAVES * 64),
-                           dma_off[li] + blk * (BN * D * 2));
+                           dma_off[li] + blk * (BN * hd * 2));
             }
         };
 
-        if constexpr (DMA) {
-            if (s_begin < s_end) issue_step(s_begin);
-            __builtin_amdgcn_s_waitcnt(0);
-            __syncthreads();
-        } else {
-            load_step(s_begin);
-            __syncthreads();  // the previous tile's LDS use is over
-            store_step(0);
-            __syncthreads();
-        }
+        if (s_begin < s_end) issue_step(s_begin);
+        __builtin_amdgcn_s_waitcnt(0);
+        __syncthreads();
 
-        // DMA: the blocks of step j + 1 stream into the other stage while
-        // step j is computed (one barrier per step).  Otherwise they wait in
-        // registers and are stored after the step's compute.
+        // The blocks of step j + 1 stream into the other stage while step j
+        // is computed (one barrier per step).
         for (uint32_t step = s_begin; step < s_end; ++step) {
-            if constexpr (DMA) {
-                if (step + 1 < s_end) issue_step(step + 1);  // nothing past the last block
-            } else {
-                if (step + 1 < s_end) load_step(step + 1);
-            }
+            if (step + 1 < s_end) issue_step(step + 1);  // nothing past the last block
             const uint32_t blk = step * KSPLIT + sub;
-            const half_t* ks = kv_lds + ((step % NSTAGE) * KSPLIT + sub) * KV_HALVES;
-            const half_t* vs = ks + BN * KS;
+            const half_t* ks = kv_lds + ((step % 2) * KSPLIT + sub) * KV_HALVES;
+            const half_t* vs = ks + BN * RD;
             if (blk < blocks && blk * BN < wave_keys) {
                 // S^T = K Q^T, 32 keys per tile
                 f32x16 s[KT];
@@ -372,7 +394,7 @@ __global__ __launch_bounds__(64 * QW * KSPLIT) void k_flash_attention(
                     for (int r = 0; r < 16; ++r) s[kt][r] = 0.0f;
 #pragma unroll
                     for (int c = 0; c < DC; ++c) {
-                        const h8 ka = *reinterpret_cast<const h8*>(ks + kt * 32 * KS + koff[c]);
+                        const h8 ka = *reinterpret_cast<const h8*>(ks + kt * 32 * RD + koff[c]);
                         s[kt] = __builtin_amdgcn_mfma_f32_32x32x16_f16(ka, qf[c], s[kt], 0, 0, 0);
                     }
                 }
@@ -411,16 +433,27 @@ __global__ __launch_bounds__(64 * QW * KSPLIT) void k_flash_attention(
                 }
                 // p = 2^(s * scale * log2 e - m); a query that has seen no
                 // key yet (m = -inf) has only -inf scores here, and p = 0.
-                const float neg_m = m == -INFINITY ? 0.0f : -m;
+                const float neg_m = (m == -INFINITY ? 0.0f : -m) + (ANY ? kAnyShift : 0.0f);
                 // P as the f16 operand of the P V product: lane half hs
                 // supplies keys 16c + 8hs .. +7, which it holds in registers
                 // 8(c%2) .. +7 of tile c/2.  The running sum adds the same f16
                 // probabilities the product uses (v_dot2_f32_f16 against
                 // ones, f32 accumulation).
                 const h2 ones = {half_t(1.0f), half_t(1.0f)};
-                h8 pb[BN / 16];
+                h8 pb[BN / 16], pl[ANY ? BN / 16 : 1];
 #pragma unroll
                 for (int c = 0; c < BN / 16; ++c) {
+                    if constexpr (ANY) {
+#pragma unroll
+                        for (int e = 0; e < 8; ++e) {
+                            const float x = __builtin_amdgcn_exp2f(
+                                __builtin_fmaf(s[c >> 1][8 * (c & 1) + e], p.scale_log2, neg_m));
+                            l += x;
+                            pb[c][e] = half_t(x);
+                            pl[c][e] = half_t(x - float(pb[c][e]));
+                        }
+                        continue;
+                    }
 #pragma unroll
                     for (int e = 0; e < 8; ++e)
                         pb[c][e] = half_t(__builtin_amdgcn_exp2f(
@@ -434,19 +467,16 @@ __global__ __launch_bounds__(64 * QW * KSPLIT) void k_flash_attention(
                 for (int c = 0; c < BN / 16; ++c) {
 #pragma unroll
                     for (int t = 0; t < NT; ++t) {
-                        const h4 lo = lds_read_transposed(vs + 16 * c * VS + voff[0][t]);
-                        const h4 hi = lds_read_transposed(vs + 16 * c * VS + voff[1][t]);
+                        const h4 lo = lds_read_transposed(vs + 16 * c * RD + voff[0][t]);
+                        const h4 hi = lds_read_transposed(vs + 16 * c * RD + voff[1][t]);
                         const h8 va = {lo[0], lo[1], lo[2], lo[3], hi[0], hi[1], hi[2], hi[3]};
+                        if constexpr (ANY)
+                            o[t] = __builtin_amdgcn_mfma_f32_32x32x16_f16(va, pl[c], o[t], 0, 0, 0);
                         o[t] = __builtin_amdgcn_mfma_f32_32x32x16_f16(va, pb[c], o[t], 0, 0, 0);
                     }
                 }
             }
-            if constexpr (DMA) {
-                __builtin_amdgcn_s_waitcnt(0);  // this wave's DMA has landed
-            } else {
-                __syncthreads();
-                if (step + 1 < s_end) store_step(0);
-            }
+            __builtin_amdgcn_s_waitcnt(0);  // this wave's DMA has landed
             __syncthreads();
         }
 
@@ -504,18 +534,36 @@ __global__ __launch_bounds__(64 * QW * KSPLIT) void k_flash_attention(
             }
         } else if (sub == 0) {
             const float inv = 1.0f / (l + __shfl_xor(l, 32, 64));  // both halves of the query
+            bool finite = true;  // ANY: every output of this lane
             if (q_valid) {
                 // register r of tile t: element 32t + 8(r / 4) + 4hs + r % 4
-                half_t* orow = out + (uint64_t(bh) * p.q_len + qi) * D + 4 * hs;
+                half_t* orow = out + (uint64_t(bh) * p.q_len + qi) * hd + 4 * hs;
 #pragma unroll
                 for (int t = 0; t < NT; ++t) {
 #pragma unroll
                     for (int g = 0; g < 4; ++g) {
+                        if (ANY && 32 * t + 8 * g >= int(hd)) continue;  // padding
                         h4 w;
 #pragma unroll
-                        for (int e = 0; e < 4; ++e) w[e] = half_t(o[t][4 * g + e] * inv);
+                        for (int e = 0; e < 4; ++e) {
+                            w[e] = half_t(o[t][4 * g + e] * inv);
+                            if constexpr (ANY) finite &= fabsf(o[t][4 * g + e] * inv) < INFINITY;
+                        }
                         *reinterpret_cast<h4*>(orow + t * 32 + 8 * g) = w;
                     }
+                }
+            }
+            if constexpr (ANY) {
+                // queries with an output that is not finite, in turn, by the
+                // whole wave (after its stores above: same wave, in order)
+                uint64_t redo = __ballot(!finite);
+                redo = (redo | redo >> 32) & 0xffffffffu;
+                while (redo != 0) {
+                    const uint32_t c = __builtin_ctzll(redo);
+                    redo &= redo - 1;
+                    const uint64_t row = uint64_t(bh) * p.q_len + qw0 + c;
+                    exact_row<half_t, NT>(q + row * hd, kh, vh, out + row * hd, hd,
+                                          min(p.kv_len, p.start + qw0 + c + 1), p.scale);
                 }
             }
         }
@@ -1600,7 +1648,8 @@ uint32_t flash_key_chunks(uint64_t heads, uint64_t q_len, uint64_t kv_len, uint6
 
 // The matrix-core kernels by head size: f16 in key blocks of 128 (head
 // size up to 64 with 128-query tiles) or 64 (32 for head size 128 with
-// 32-query tiles), from DMA-fed LDS except head size 96; f32 in blocks of
+// 32-query tiles; head size 96 as 128, its LDS rows being as long); f32 in
+// blocks of
 // 64 (up to 64, 128-query tiles) or 32.
 template <int QW, int KS>
 void launch_flash(rl_context* ctx, dim3 g, uint32_t nt, const half_t* q, const half_t* k,
@@ -1609,14 +1658,14 @@ void launch_flash(rl_context* ctx, dim3 g, uint32_t nt, const half_t* q, const h
     constexpr int BN4 = KS == 4 ? 32 : 64;
     const dim3 b(64 * QW * KS);
     if (nt == 1) {
-        RL_LAUNCH(ctx, (k_flash_attention<1, QW, KS, BN, true>), g, b, q, k, v, o, p);
+        RL_LAUNCH(ctx, (k_flash_attention<1, QW, KS, BN>), g, b, q, k, v, o, p);
     } else if (nt == 2) {
-        RL_LAUNCH(ctx, (k_flash_attention<2, QW, KS, BN, true>), g, b, q, k, v, o, p);
+        RL_LAUNCH(ctx, (k_flash_attention<2, QW, KS, BN>), g, b, q, k, v, o, p);
     } else if constexpr (!(QW == 1 && KS == 2)) {  // that shape only for head sizes <= 64
         if (nt == 3) {
-            RL_LAUNCH(ctx, (k_flash_attention<3, QW, KS, 64, false>), g, b, q, k, v, o, p);
+            RL_LAUNCH(ctx, (k_flash_attention<3, QW, KS, BN4>), g, b, q, k, v, o, p);
         } else {
-            RL_LAUNCH(ctx, (k_flash_attention<4, QW, KS, BN4, true>), g, b, q, k, v, o, p);
+            RL_LAUNCH(ctx, (k_flash_attention<4, QW, KS, BN4>), g, b, q, k, v, o, p);
         }
     }
 }
@@ -1626,16 +1675,16 @@ void launch_flash_split(rl_context* ctx, uint64_t heads, uint32_t nt, const half
     const dim3 g(static_cast<unsigned>(heads * p.pairs * p.kchunks)), b(64 * 4 * 2);
     const dim3 gc(static_cast<unsigned>(heads * p.tiles * (128 / kCombineRows))), bc(256);
     if (nt == 1) {
-        RL_LAUNCH(ctx, (k_flash_attention<1, 4, 2, 128, true, true>), g, b, q, k, v, o, p);
+        RL_LAUNCH(ctx, (k_flash_attention<1, 4, 2, 128, true>), g, b, q, k, v, o, p);
         RL_LAUNCH(ctx, (k_flash_combine<32, 128>), gc, bc, o, p);
     } else if (nt == 2) {
-        RL_LAUNCH(ctx, (k_flash_attention<2, 4, 2, 128, true, true>), g, b, q, k, v, o, p);
+        RL_LAUNCH(ctx, (k_flash_attention<2, 4, 2, 128, true>), g, b, q, k, v, o, p);
         RL_LAUNCH(ctx, (k_flash_combine<64, 128>), gc, bc, o, p);
     } else if (nt == 3) {
-        RL_LAUNCH(ctx, (k_flash_attention<3, 4, 2, 64, false, true>), g, b, q, k, v, o, p);
+        RL_LAUNCH(ctx, (k_flash_attention<3, 4, 2, 64, true>), g, b, q, k, v, o, p);
         RL_LAUNCH(ctx, (k_flash_combine<96, 128>), gc, bc, o, p);
     } else {
-        RL_LAUNCH(ctx, (k_flash_attention<4, 4, 2, 64, true, true>), g, b, q, k, v, o, p);
+        RL_LAUNCH(ctx, (k_flash_attention<4, 4, 2, 64, true>), g, b, q, k, v, o, p);
         RL_LAUNCH(ctx, (k_flash_combine<128, 128>), gc, bc, o, p);
     }
 }
@@ -1658,10 +1707,54 @@ void launch_flash(rl_context* ctx, dim3 g, uint32_t nt, const float* q, const fl
     }
 }
 
+// The f16 kernel for padded head sizes (ANY), blocks and staging as above;
+// 64-query tiles of two key shares above head size 128, whose two DMA stages
+// of 32-key blocks take 128 KB of LDS.
+template <int QW, int KS, int NT, int BN>
+void launch_flash_any(rl_context* ctx, dim3 g, const half_t* q, const half_t* k, const half_t* v,
+                      half_t* o, const AttnParams& p) {
+    RL_LAUNCH(ctx, (k_flash_attention<NT, QW, KS, BN, false, true>), g,
+              dim3(64 * QW * KS), q, k, v, o, p);
+}
+rl_status launch_flash_any(rl_context* ctx, uint64_t heads, const half_t* q, const half_t* k,
+                           const half_t* v, half_t* o, AttnParams p) {
+    const uint32_t nt = (p.head_dim + 31) / 32;
+    const bool wide =
+        nt <= 4 && flash_shape(heads, p.q_len, 32 * nt, kFlashFillBlocksF16) == FlashShape::kWide;
+    p.tiles = uint32_t(ceil_div(p.q_len, wide ? 128 : nt > 4 ? 64 : 32));
+    p.pairs = (p.tiles + 1) / 2;
+    const uint64_t grid = heads * p.pairs;
+    if (grid > UINT32_MAX) return fail(RL_ERR_INVALID_SHAPE, "attention grid exceeds u32");
+    const dim3 g(static_cast<unsigned>(grid));
+    if (nt > 4) {
+        launch_flash_any<2, 2, 8, 32>(ctx, g, q, k, v, o, p);
+    } else if (wide) {
+        if (nt == 1) launch_flash_any<4, 2, 1, 128>(ctx, g, q, k, v, o, p);
+        else if (nt == 2) launch_flash_any<4, 2, 2, 128>(ctx, g, q, k, v, o, p);
+        else if (nt == 3) launch_flash_any<4, 2, 3, 64>(ctx, g, q, k, v, o, p);
+        else launch_flash_any<4, 2, 4, 64>(ctx, g, q, k, v, o, p);
+    } else {
+        if (nt == 1) launch_flash_any<1, 4, 1, 64>(ctx, g, q, k, v, o, p);
+        else if (nt == 2) launch_flash_any<1, 4, 2, 64>(ctx, g, q, k, v, o, p);
+        else if (nt == 3) launch_flash_any<1, 4, 3, 32>(ctx, g, q, k, v, o, p);
+        else launch_flash_any<1, 4, 4, 32>(ctx, g, q, k, v, o, p);
+    }
+    return RL_OK;
+}
+
 // Which kernel a shape takes: the MFMA kernels for a head size of 32, 64,
 // 96 or 128 and 16-byte aligned buffers (f16: also byte offsets into one KV
 // head, a block past its end included, that fit the 32-bit buffer offsets
-// of its loads); the row kernel otherwise (head sizes up to 512).
+// of its loads); in f16 the padded matrix-core kernel (ANY) for the other
+// multiples of 8 up to 256 (rows of whole 16-byte pieces); the row kernel
+// otherwise (head sizes up to 512).
+bool use_flash_any(const AttnShape& s, const void* q, const void* k, const void* v,
+                   const void* o) {
+    const uint64_t span = (s.kv_len + uint64_t(kFlashMaxBlockKeys) * kFlashMaxKeySplit) *
+                          s.head_dim * sizeof(half_t);
+    return s.head_dim % 8 == 0 && s.head_dim <= 256 && span < (uint64_t(1) << 31) &&
+           aligned_to(q, 16) && aligned_to(k, 16) && aligned_to(v, 16) && aligned_to(o, 16);
+}
 template <typename T>
 bool use_flash(const AttnShape& s, const void* q, const void* k, const void* v, const void* o) {
     const bool shape = s.head_dim % 32 == 0 && s.head_dim <= 128 && aligned_to(q, 16) &&
@@ -1898,6 +1991,12 @@ rl_status attention_entry(rl_context* ctx, const char* name, const rl_buffer* q,
         else if (shape == FlashShape::kNarrow2) launch_flash<1, 2>(ctx, g, nt, qd, kd, vd, od, p);
         else launch_flash<1, 4>(ctx, g, nt, qd, kd, vd, od, p);
         return after_launch(ctx, name);
+    }
+    if constexpr (std::is_same<T, half_t>::value) {
+        if (use_flash_any(s, qd, kd, vd, od)) {
+            if (rl_status st = launch_flash_any(ctx, heads, qd, kd, vd, od, p)) return st;
+            return after_launch(ctx, name);
+        }
     }
     const dim3 g(static_cast<unsigned>(rows)), b(64);
     if (s.head_dim <= 64) {

@@ -384,3 +384,69 @@ def test_attention_in_a_graph_matches_eager(ctx, dtype):
         ctx.attention(bufs[1][4], bufs[1][5], bufs[1][6], 0.125, dshape[7], dshape[4])  # eager work
         ctx.finish()
     ctx.graph_destroy(graph)
+
+
+# ------------------------------- f16 head sizes without a kernel of their own
+
+# Padded to the next multiple of 32 (192 and up: to 256); the last of each
+# wide/narrow pair has enough heads and queries for the 128-query tiles.
+PADDED_SHAPES = [
+    (1, 2, 1, 33, 40, 48, 8, 7),
+    (1, 3, 1, 65, 130, 130, 24, 65),
+    (1, 8, 4, 129, 129, 160, 40, 0),
+    (1, 32, 8, 700, 700, 700, 48, 0),     # 128-query tiles, padded to 64
+    (1, 8, 8, 1021, 1021, 1024, 80, 0),
+    (1, 32, 8, 700, 713, 720, 80, 13),    # 128-query tiles, padded to 96
+    (2, 4, 2, 31, 95, 100, 112, 64),
+    (1, 32, 8, 641, 641, 641, 120, 0),    # 128-query tiles, padded to 128
+    (1, 48, 8, 500, 500, 500, 16, 0),     # 128-query tiles, padded to 32
+    (1, 4, 2, 70, 1000, 1024, 136, 930),
+    (1, 4, 1, 127, 127, 127, 200, 0),
+    (1, 8, 8, 500, 500, 512, 256, 0),
+    (1, 2, 2, 1, 33, 64, 256, 32),
+]
+
+
+@pytest.mark.parametrize("shape", PADDED_SHAPES)
+def test_attention_padded_head_sizes(ctx, shape):
+    """f32 bound plus the output's f16 rounding: the probabilities enter the
+    second product as two f16 parts (22 bits: within the f32 bound's 8 u)."""
+    b, qh, kvh, ql, kl, cap, hd, start = shape
+    q = synth.normal(synth.seed_for("pad-q", *shape), (b, qh, ql, hd)).astype(np.float16)
+    k = cache(synth.seed_for("pad-k", *shape), b, kvh, cap, hd, kl, np.float16)
+    v = cache(synth.seed_for("pad-v", *shape), b, kvh, cap, hd, kl, np.float16)
+    scale = 1.0 / np.sqrt(hd)
+    got = run_attention(ctx, q, k, v, scale, start, kl)
+    exact, bound = attention_bound(q, k, v, scale, start, kl, "f32")
+    err = np.abs(got.astype(np.float64) - exact)
+    bound = bound + ulp16(exact) * 0.5001
+    worst = np.unravel_index(np.argmax(err / bound), err.shape)
+    assert np.all(err <= bound), f"{shape}: {err[worst]:.3g} > {bound[worst]:.3g} at {worst}"
+
+
+@pytest.mark.parametrize("hd,ql", [(80, 70), (48, 300), (256, 70)])
+def test_attention_padded_head_sizes_infinities(ctx, hd, ql):
+    """Infinities and NaN as unsplit arithmetic gives them: an infinite value
+    column is infinite from its key on, a key of score -inf drops out, and a
+    NaN key or value behind a query's causal limit does not reach it."""
+    q = np.abs(synth.normal(41, (1, 2, ql, hd))).astype(np.float16)
+    k = synth.normal(42, (1, 1, ql, hd)).astype(np.float16)
+    v = synth.normal(43, (1, 1, ql, hd)).astype(np.float16)
+    scale = 1.0 / np.sqrt(hd)
+    keep = np.array([j for j in range(ql) if j != 5])
+    k[0, 0, 5] = -np.inf      # scores -inf: never contributes to queries >= 6
+    v[0, 0, 20, 3] = np.inf
+    k[0, 0, ql - 2] = np.nan
+    v[0, 0, ql - 2] = np.nan
+    got = run_attention(ctx, q, k, v, scale, 0, ql).astype(np.float64)
+    assert np.isnan(got[:, :, ql - 2:]).all()
+    assert np.isposinf(got[:, :, 20:ql - 2, 3]).all()
+    clean_v = v.copy()
+    clean_v[0, 0, 20, 3] = 0
+    n = ql - 2
+    exact, bound = attention_bound(q[:, :, 6:n], k[:, :, keep[:n - 1]], clean_v[:, :, keep[:n - 1]],
+                                   scale, 5, n - 1, "f32")
+    err = np.abs(got[:, :, 6:n] - exact)
+    cols = [c for c in range(hd) if c != 3]
+    assert np.all(err[..., cols] <= (bound + ulp16(exact))[..., cols])
+    assert np.isfinite(got[:, :, :5]).all()
