@@ -52,12 +52,14 @@ constexpr float kLn2 = 0.693147180559945309417f;
 
 struct AttnParams {
     uint32_t q_heads;      // query heads per batch entry
+    uint32_t kv_heads;     // KV heads per batch entry
+    uint32_t heads;        // query heads of all batch entries
     uint32_t group;        // query heads per KV head
     uint32_t q_len;
     uint32_t kv_len;
     uint32_t start;        // absolute position of query 0
     uint32_t tiles;        // query tiles per head (MFMA kernel)
-    uint32_t pairs;        // workgroups per head (MFMA kernel)
+    uint32_t pairs;        // workgroups per head (MFMA kernel): tile pairs, or tiles
     uint32_t head_dim;
     uint64_t kv_head_stride;  // elements between KV heads (kv_capacity * head_dim)
     float scale;           // attention scale
@@ -248,10 +250,14 @@ __global__ __launch_bounds__(64 * QW * KSPLIT) void k_flash_attention(
     // (the chunks of one pair are neighbours in the grid: one KV head)
     const uint32_t chunk = PARTIAL ? blockIdx.x % p.kchunks : 0u;
     const uint32_t unit_blk = PARTIAL ? blockIdx.x / p.kchunks : blockIdx.x;
-    const uint32_t bh = unit_blk / p.pairs;
-    const uint32_t pair = unit_blk % p.pairs;
-    const uint32_t kv_heads = p.q_heads / p.group;
-    const uint32_t kv_head = (bh / p.q_heads) * kv_heads + (bh % p.q_heads) / p.group;
+    // one tile a workgroup: tile by tile over all heads, longest first
+    const bool by_tile = !PARTIAL && p.pairs == p.tiles;
+    const uint32_t per = by_tile ? p.heads : p.pairs;
+    const uint32_t major = unit_blk / per, minor = unit_blk - major * per;
+    const uint32_t bh = by_tile ? minor : major;
+    const uint32_t pair = by_tile ? major : minor;
+    const uint32_t batch = bh / p.q_heads;
+    const uint32_t kv_head = batch * p.kv_heads + (bh - batch * p.q_heads) / p.group;
     const half_t* kh = k + uint64_t(kv_head) * p.kv_head_stride;
     const half_t* vh = v + uint64_t(kv_head) * p.kv_head_stride;
 
@@ -308,10 +314,11 @@ __global__ __launch_bounds__(64 * QW * KSPLIT) void k_flash_attention(
         reinterpret_cast<uintptr_t>((__attribute__((address_space(3))) unsigned char*)(lds)));
 
     // The causal tiles of a head are paired (t, tiles - 1 - t) so that every
-    // workgroup streams about the same number of key blocks.
+    // workgroup streams about the same number of key blocks; where pairs ==
+    // tiles a workgroup takes one tile (flash_pairs).
     for (int which = 0; which < 2; ++which) {
         const uint32_t tile = which == 0 ? p.tiles - 1 - pair : pair;
-        if (which == 1 && tile >= p.tiles - 1 - pair) break;
+        if (which == 1 && (p.pairs == p.tiles || tile >= p.tiles - 1 - pair)) break;
 
         const uint32_t q_first = tile * TILE_Q;
         const uint32_t q_last = min(p.q_len, q_first + TILE_Q) - 1;
@@ -657,10 +664,13 @@ __global__ __launch_bounds__(64 * QW * KSPLIT) void k_flash_attention_f32(
     static_assert((BLOCK_CHUNKS * KSPLIT) % THREADS == 0, "blocks must split evenly");
     __shared__ __align__(16) float lds[LDS_FLOATS];
 
-    const uint32_t bh = blockIdx.x / p.pairs;
-    const uint32_t pair = blockIdx.x % p.pairs;
-    const uint32_t kv_heads = p.q_heads / p.group;
-    const uint32_t kv_head = (bh / p.q_heads) * kv_heads + (bh % p.q_heads) / p.group;
+    const bool by_tile = p.pairs == p.tiles;  // as in k_flash_attention
+    const uint32_t per = by_tile ? p.heads : p.pairs;
+    const uint32_t major = blockIdx.x / per, minor = blockIdx.x - major * per;
+    const uint32_t bh = by_tile ? minor : major;
+    const uint32_t pair = by_tile ? major : minor;
+    const uint32_t batch = bh / p.q_heads;
+    const uint32_t kv_head = batch * p.kv_heads + (bh - batch * p.q_heads) / p.group;
     const float* kh = k + uint64_t(kv_head) * p.kv_head_stride;
     const float* vh = v + uint64_t(kv_head) * p.kv_head_stride;
     const uint32_t wave = threadIdx.x / 64;
@@ -672,7 +682,7 @@ __global__ __launch_bounds__(64 * QW * KSPLIT) void k_flash_attention_f32(
 
     for (int which = 0; which < 2; ++which) {
         const uint32_t tile = which == 0 ? p.tiles - 1 - pair : pair;
-        if (which == 1 && tile >= p.tiles - 1 - pair) break;
+        if (which == 1 && (p.pairs == p.tiles || tile >= p.tiles - 1 - pair)) break;
         const uint32_t q_first = tile * TILE_Q;
         const uint32_t q_last = min(p.q_len, q_first + TILE_Q) - 1;
         const uint32_t keys = min(p.kv_len, p.start + q_last + 1);
@@ -898,8 +908,8 @@ __global__ __launch_bounds__(64) void k_attention_rows(const T* __restrict__ q,
     const uint32_t row = blockIdx.x;  // (b * QH + h) * q_len + qi
     const uint32_t bh = row / p.q_len;
     const uint32_t qi = row % p.q_len;
-    const uint32_t kv_heads = p.q_heads / p.group;
-    const uint32_t kv_head = (bh / p.q_heads) * kv_heads + (bh % p.q_heads) / p.group;
+    const uint32_t batch = bh / p.q_heads;
+    const uint32_t kv_head = batch * p.kv_heads + (bh - batch * p.q_heads) / p.group;
     const uint32_t D = p.head_dim;
     const T* kh = k + uint64_t(kv_head) * p.kv_head_stride;
     const T* vh = v + uint64_t(kv_head) * p.kv_head_stride;
@@ -1135,9 +1145,8 @@ __global__ __launch_bounds__(64 * kSplitWaves) void k_attention_split(
     const uint32_t lane = threadIdx.x % 64;
     const uint32_t kvb = blockIdx.x / splits;  // b * kv_heads + kv head
     const uint32_t split = blockIdx.x % splits;
-    const uint32_t kv_heads = p.q_heads / p.group;
-    const uint32_t b = kvb / kv_heads;
-    const uint32_t first_head = (kvb % kv_heads) * p.group;
+    const uint32_t b = kvb / p.kv_heads;
+    const uint32_t first_head = (kvb - b * p.kv_heads) * p.group;
     const uint32_t R = p.group * p.q_len;
     const uint32_t D = p.head_dim;
     const T* kh = k + uint64_t(kvb) * p.kv_head_stride;
@@ -1396,9 +1405,8 @@ __global__ __launch_bounds__(64 * kSplitWaves) void k_attention_split_mfma(
     const uint32_t g = lane / 16;
     const uint32_t kvb = blockIdx.x / splits;  // b * kv_heads + kv head
     const uint32_t split = blockIdx.x % splits;
-    const uint32_t kv_heads = p.q_heads / p.group;
-    const uint32_t b = kvb / kv_heads;
-    const uint32_t first_head = (kvb % kv_heads) * p.group;
+    const uint32_t b = kvb / p.kv_heads;
+    const uint32_t first_head = (kvb - b * p.kv_heads) * p.group;
     const uint32_t R = p.group * p.q_len;
     const half_t* kh = k + uint64_t(kvb) * p.kv_head_stride;
     const half_t* vh = v + uint64_t(kvb) * p.kv_head_stride;
@@ -1620,6 +1628,22 @@ FlashShape flash_shape(uint64_t heads, uint64_t q_len, uint64_t head_dim, uint64
     return FlashShape::kNarrow2;
 }
 
+// Workgroups per head: one per pair of tiles (equal shares of a causal
+// square) where the pairs fill the CUs -- at one workgroup a CU, in whole
+// rounds -- to at least 4/5, else one per tile, handed out longest first over
+// all heads.  One MI355X, pairs against tiles: f16, 8 heads of 80 x [1021,
+// 1021] (128 pairs) 24.3 / 18.8 us; 15 of 64 x [512, 512] (120) 10.9 / 7.5;
+// 32 of 64 x 100 queries after 1000 keys (64) 21.0 / 11.3; 15 of 64 x [1500,
+// 1500] (360) 22.8 / 19.7; f32, 15 of 64 x [3001, 3001] (180) 238 / 211;
+// 32 of 64 x 200 after 2000 (128) 128 / 66.  Filled: f16, 15 of 64 x [4096,
+// 4096] (240) 53.2 / 54.4, 32 x [2048, 2048] (256) 32.0 / 32.9, 15 x [900,
+// 900] (225) 14.2 / 14.4.
+uint32_t flash_pairs(const rl_context* ctx, uint64_t heads, uint32_t tiles) {
+    const uint64_t cus = uint64_t(ctx->num_cus);
+    const uint32_t pairs = (tiles + 1) / 2;
+    return heads * pairs * 5 >= ceil_div(heads * pairs, cus) * cus * 4 ? pairs : tiles;
+}
+
 // Key chunks per 128-query tile for the f16 kernel (1 = no split), W the
 // wide tile pairs, steps the longest tile's key steps (two blocks each).
 // One workgroup a CU fits (its LDS), so chunks beyond 256 / W workgroups
@@ -1722,7 +1746,7 @@ rl_status launch_flash_any(rl_context* ctx, uint64_t heads, const half_t* q, con
     const bool wide =
         nt <= 4 && flash_shape(heads, p.q_len, 32 * nt, kFlashFillBlocksF16) == FlashShape::kWide;
     p.tiles = uint32_t(ceil_div(p.q_len, wide ? 128 : nt > 4 ? 64 : 32));
-    p.pairs = (p.tiles + 1) / 2;
+    p.pairs = flash_pairs(ctx, heads, p.tiles);
     const uint64_t grid = heads * p.pairs;
     if (grid > UINT32_MAX) return fail(RL_ERR_INVALID_SHAPE, "attention grid exceeds u32");
     const dim3 g(static_cast<unsigned>(grid));
@@ -1889,6 +1913,8 @@ rl_status attention_entry(rl_context* ctx, const char* name, const rl_buffer* q,
 
     AttnParams p{};
     p.q_heads = uint32_t(s.q_heads);
+    p.kv_heads = uint32_t(s.kv_heads);
+    p.heads = uint32_t(heads);
     p.group = uint32_t(s.q_heads / s.kv_heads);
     p.q_len = uint32_t(s.q_len);
     p.kv_len = uint32_t(s.kv_len);
@@ -1982,7 +2008,7 @@ rl_status attention_entry(rl_context* ctx, const char* name, const rl_buffer* q,
             flash_shape(heads, s.q_len, s.head_dim,
                         sizeof(T) == 2 ? kFlashFillBlocksF16 : kFlashFillBlocks);
         p.tiles = uint32_t(ceil_div(s.q_len, shape == FlashShape::kWide ? 128 : 32));
-        p.pairs = (p.tiles + 1) / 2;
+        p.pairs = flash_pairs(ctx, heads, p.tiles);
         const uint64_t grid = heads * p.pairs;
         if (grid > UINT32_MAX) return fail(RL_ERR_INVALID_SHAPE, "attention grid exceeds u32");
         const dim3 g(static_cast<unsigned>(grid));

@@ -450,3 +450,20 @@ def test_attention_padded_head_sizes_infinities(ctx, hd, ql):
     cols = [c for c in range(hd) if c != 3]
     assert np.all(err[..., cols] <= (bound + ulp16(exact))[..., cols])
     assert np.isfinite(got[:, :, :5]).all()
+
+
+# One tile a workgroup (pairs would leave CUs idle) and pairs, on both
+# sides of the rule: odd and even tile counts, one and several rounds of CUs.
+TILE_ORDER_SHAPES = [
+    (1, 7, 7, 32, 32, 32, 64, 0),       # one tile a head
+    (1, 5, 5, 300, 300, 300, 64, 0),    # 10 tiles a head, longest first
+    (3, 4, 2, 97, 500, 512, 32, 403),   # batch 3: heads of several batches
+    (1, 15, 5, 900, 900, 900, 64, 0),   # 225 pairs
+    (1, 15, 5, 1500, 1500, 1500, 64, 0),  # 705 tiles
+]
+
+
+@pytest.mark.parametrize("dtype", [np.float32, np.float16])
+@pytest.mark.parametrize("shape", TILE_ORDER_SHAPES)
+def test_attention_tile_order(ctx, dtype, shape):
+    test_attention_within_float64_bound(ctx, dtype, shape)
