@@ -12,6 +12,7 @@ method per op; ``DeviceBuffer`` owns one rl_buffer from the context's pool.
 from __future__ import annotations
 
 import ctypes
+import functools
 import os
 from typing import Sequence
 
@@ -214,7 +215,7 @@ def last_error_fields() -> tuple[int, dict]:
 
 
 def check(status: int) -> None:
-    if status != RL_OK:
+    if status:  # RL_OK is 0
         code, fields = last_error_fields()
         raise RustLLMError(status, last_error(), fields if code == status else None)
 
@@ -224,11 +225,30 @@ def device_count() -> int:
 
 
 _DTYPES = {np.dtype(np.float32): 4, np.dtype(np.float16): 2}
+_F16 = np.dtype(np.float16)
+
+
+@functools.lru_cache(maxsize=256)
+def _u64_array_of(values: tuple):
+    return (ctypes.c_uint64 * max(1, len(values)))(*[int(v) for v in values])
 
 
 def _u64_array(values: Sequence[int]):
-    arr = (ctypes.c_uint64 * max(1, len(values)))(*[int(v) for v in values])
-    return arr
+    """`values` as a C array, by value (the library only reads it): the views
+    of a model's layers have the same few dims and strides on every call."""
+    return _u64_array_of(tuple(values))
+
+
+# (op, is f16) -> the library's function, so that no name is built and looked
+# up per call.
+_FUNCTIONS: dict = {}
+
+
+def _function(lib, op: str, f16: bool):
+    fn = _FUNCTIONS.get((op, f16))
+    if fn is None:
+        fn = _FUNCTIONS[op, f16] = getattr(lib, f"rl_{op}_{'f16' if f16 else 'f32'}")
+    return fn
 
 
 class DeviceBuffer:
@@ -241,12 +261,21 @@ class DeviceBuffer:
         self.shape = tuple(int(s) for s in shape)
 
     @property
+    def raw(self) -> RlBuffer:
+        return self._raw
+
+    @raw.setter
+    def raw(self, raw: RlBuffer) -> None:
+        self._raw = raw
+        self._as_parameter_ = ctypes.byref(raw)  # what ctypes passes for a DeviceBuffer
+
+    @property
     def len(self) -> int:
-        return int(self.raw.len)
+        return self._raw.len
 
     @property
     def byte_len(self) -> int:
-        return int(self.raw.byte_len)
+        return self._raw.byte_len
 
     @property
     def ptr(self) -> int:
@@ -382,17 +411,14 @@ class Context:
         self.lib.rl_graph_destroy(graph)
 
     # ---------------------------------------------------------- ops
-    @staticmethod
-    def _sfx(buf: DeviceBuffer) -> str:
-        return "f16" if buf.dtype == np.float16 else "f32"
-
-    def _call(self, name: str, *args) -> None:
-        conv = [ctypes.byref(a.raw) if isinstance(a, DeviceBuffer) else a for a in args]
-        check(getattr(self.lib, name)(self.handle, *conv))
+    def _call(self, op: str, typed: DeviceBuffer, *args) -> None:
+        """The op of `typed`'s element type on this context.  DeviceBuffers
+        pass themselves (_as_parameter_)."""
+        check(_function(self.lib, op, typed.dtype == _F16)(self.handle, *args))
 
     def _binary(self, op: str, a: DeviceBuffer, b: DeviceBuffer, out=None) -> DeviceBuffer:
         out = out or self.empty(a.shape, a.dtype)
-        self._call(f"rl_{op}_{self._sfx(a)}", a, b, out)
+        self._call(op, a, a, b, out)
         return out
 
     def add(self, a, b, out=None):
@@ -406,81 +432,80 @@ class Context:
 
     def silu(self, x, out=None):
         out = out or self.empty(x.shape, x.dtype)
-        self._call(f"rl_silu_{self._sfx(x)}", x, out)
+        self._call("silu", x, x, out)
         return out
 
     def cast(self, x, dtype, out=None):
         dtype = np.dtype(dtype)
         out = out or self.empty(x.shape, dtype)
-        name = "rl_cast_f32_to_f16" if dtype == np.float16 else "rl_cast_f16_to_f32"
-        self._call(name, x, out)
+        name = "rl_cast_f32_to_f16" if dtype == _F16 else "rl_cast_f16_to_f32"
+        check(getattr(self.lib, name)(self.handle, x, out))
         return out
 
     def add_broadcast(self, x, bias, out=None):
         out = out or self.empty(x.shape, x.dtype)
         cols = bias.len
-        self._call(f"rl_add_broadcast_{self._sfx(x)}", x, bias, x.len // max(cols, 1), cols,
+        self._call("add_broadcast", x, x, bias, x.len // max(cols, 1), cols,
                    out)
         return out
 
     def contiguous(self, src, dims, strides, out=None):
         out = out or self.empty(dims, src.dtype)
         d, s = _u64_array(dims), _u64_array(strides)
-        self._call(f"rl_contiguous_{self._sfx(src)}", src, d, s, len(dims), out)
+        self._call("contiguous", src, src, d, s, len(dims), out)
         return out
 
     def repeat_kv(self, x, repeats: int, out=None):
         b, kvh, s, d = x.shape
         out = out or self.empty((b, kvh * repeats, s, d), x.dtype)
-        self._call(f"rl_repeat_kv_{self._sfx(x)}", x, b, kvh, s, d, repeats, out)
+        self._call("repeat_kv", x, x, b, kvh, s, d, repeats, out)
         return out
 
     def rmsnorm(self, x, weight, eps: float, out=None):
         out = out or self.empty(x.shape, x.dtype)
         hidden = weight.len
-        self._call(f"rl_rmsnorm_{self._sfx(x)}", x, weight, x.len // hidden, hidden,
-                   ctypes.c_float(eps), out)
+        self._call("rmsnorm", x, x, weight, x.len // hidden, hidden, eps, out)
         return out
 
     def add_rmsnorm(self, x, residual, weight, eps: float, sum_out=None, norm_out=None):
         sum_out = sum_out or self.empty(x.shape, x.dtype)
         norm_out = norm_out or self.empty(x.shape, x.dtype)
         hidden = weight.len
-        self._call(f"rl_add_rmsnorm_{self._sfx(x)}", x, residual, weight, x.len // hidden,
-                   hidden, ctypes.c_float(eps), sum_out, norm_out)
+        self._call("add_rmsnorm", x, x, residual, weight, x.len // hidden,
+                   hidden, eps, sum_out, norm_out)
         return sum_out, norm_out
 
     def softmax(self, x, out=None):
         out = out or self.empty(x.shape, x.dtype)
         width = x.shape[-1]
-        self._call(f"rl_softmax_{self._sfx(x)}", x, x.len // width, width, out)
+        self._call("softmax", x, x, x.len // width, width, out)
         return out
 
     def scale_mask(self, x, scale: float, start: int, out=None):
         out = out or self.empty(x.shape, x.dtype)
         q, k = x.shape[-2], x.shape[-1]
-        self._call(f"rl_attention_scale_mask_{self._sfx(x)}", x, ctypes.c_float(scale), q, k,
+        self._call("attention_scale_mask", x, x, scale, q, k,
                    start, out)
         return out
 
     def attention_softmax(self, x, scale: float, start: int, out=None):
         out = out or self.empty(x.shape, x.dtype)
         q, k = x.shape[-2], x.shape[-1]
-        self._call(f"rl_attention_softmax_{self._sfx(x)}", x, ctypes.c_float(scale), q, k,
+        self._call("attention_softmax", x, x, scale, q, k,
                    start, out)
         return out
 
     def rope(self, x, cos, sin, start: int, out=None):
         out = out or self.empty(x.shape, x.dtype)
         s, d = x.shape[-2], x.shape[-1]
-        self._call(f"rl_rope_{self._sfx(x)}", x, cos, sin, s, d, start, out)
+        self._call("rope", x, x, cos, sin, s, d, start, out)
         return out
 
     def rope_strided(self, src, dims, strides, cos, sin, start: int, out=None):
         out = out or self.empty(dims, src.dtype)
         d, s = _u64_array(dims), _u64_array(strides)
         table_rows = cos.shape[0]
-        self._call(f"rl_rope_strided_{self._sfx(src)}", src, d, s, len(dims), cos, sin,
+        self._call("rope_strided", src, src, d, s, len(dims), cos, sin,
                    table_rows, start, out)
         return out
 
@@ -490,17 +515,17 @@ class Context:
         [1, H, max, D] `cache` (in place)."""
         _, heads, max_seq, head_dim = cache.shape
         seq = source.shape[2]
-        self._call(f"rl_kv_cache_write_{self._sfx(cache)}", cache, heads, max_seq, head_dim,
+        self._call("kv_cache_write", cache, cache, heads, max_seq, head_dim,
                    source, seq, start)
 
     def kv_cache_write_strided(self, src, dims, strides, cache, start: int) -> None:
         d, s = _u64_array(dims), _u64_array(strides)
-        self._call(f"rl_kv_cache_write_strided_{self._sfx(cache)}", src, d, s, len(dims), cache,
+        self._call("kv_cache_write_strided", cache, src, d, s, len(dims), cache,
                    cache.shape[2], start)
 
     def rope_kv_cache_write(self, src, dims, strides, cos, sin, start: int, cache) -> None:
         d, s = _u64_array(dims), _u64_array(strides)
-        self._call(f"rl_rope_kv_cache_write_{self._sfx(cache)}", src, d, s, len(dims), cos, sin,
+        self._call("rope_kv_cache_write", cache, src, d, s, len(dims), cos, sin,
                    cos.shape[0], start, cache, cache.shape[2])
 
     def qkv_rope_kv_append(self, q, k, v, cos, sin, start: int, k_cache, v_cache, q_out=None):
@@ -508,7 +533,7 @@ class Context:
         rotated contiguous Q; K (rotated) and V land in the caches at start."""
         (qb, qd, qs), (kb, kd, ks), (vb, vd, vs) = q, k, v
         q_out = q_out or self.empty(qd, qb.dtype)
-        self._call(f"rl_qkv_rope_kv_append_{self._sfx(qb)}", qb, _u64_array(qd), _u64_array(qs),
+        self._call("qkv_rope_kv_append", qb, qb, _u64_array(qd), _u64_array(qs),
                    kb, _u64_array(kd), _u64_array(ks), vb, _u64_array(vd), _u64_array(vs), cos,
                    sin, cos.shape[0], start, q_out, k_cache, v_cache, k_cache.shape[2])
         return q_out
@@ -523,7 +548,7 @@ class Context:
         rep_shape = (kd[0], kd[1] * max(n_rep, 1), start + kd[2], kd[3])
         k_rep = k_rep or self.empty(rep_shape, kb.dtype)
         v_rep = v_rep or self.empty(rep_shape, vb.dtype)
-        self._call(f"rl_qkv_rope_kv_append_repeat_{self._sfx(qb)}", qb, _u64_array(qd),
+        self._call("qkv_rope_kv_append_repeat", qb, qb, _u64_array(qd),
                    _u64_array(qs), kb, _u64_array(kd), _u64_array(ks), vb, _u64_array(vd),
                    _u64_array(vs), cos, sin, cos.shape[0], start, q_out, k_cache, v_cache,
                    k_cache.shape[2], n_rep, k_rep, v_rep)
@@ -536,8 +561,8 @@ class Context:
         kvh, cap = k.shape[1], k.shape[2]
         kv_len = cap if kv_len is None else kv_len
         out = out or self.empty(q.shape, q.dtype)
-        self._call(f"rl_attention_{self._sfx(q)}", q, k, v, b, qh, kvh, ql, kv_len, hd, cap,
-                   ctypes.c_float(scale), start, out)
+        self._call("attention", q, q, k, v, b, qh, kvh, ql, kv_len, hd, cap, scale,
+                   start, out)
         return out
 
     def attention_noalloc(self, q, k, v, scale: float, start: int, kv_len=None, out=None):
@@ -548,8 +573,8 @@ class Context:
         kvh, cap = k.shape[1], k.shape[2]
         kv_len = cap if kv_len is None else kv_len
         out = out or self.empty(q.shape, q.dtype)
-        self._call("rl_attention_f16_noalloc", q, k, v, b, qh, kvh, ql, kv_len, hd, cap,
-                   ctypes.c_float(scale), start, out)
+        check(self.lib.rl_attention_f16_noalloc(self.handle, q, k, v, b, qh, kvh, ql, kv_len, hd,
+                                                cap, scale, start, out))
         return out
 
     def gqa_qk(self, q, k, kv_len=None, out=None):
@@ -558,7 +583,7 @@ class Context:
         kvh, cap = k.shape[1], k.shape[2]
         kv_len = cap if kv_len is None else kv_len
         out = out or self.empty((b, qh, ql, kv_len), q.dtype)
-        self._call(f"rl_gqa_qk_matmul_{self._sfx(q)}", q, k, b, qh, kvh, ql, kv_len, hd, cap, out)
+        self._call("gqa_qk_matmul", q, q, k, b, qh, kvh, ql, kv_len, hd, cap, out)
         return out
 
     def gqa_pv(self, probs, v, out=None):
@@ -566,7 +591,7 @@ class Context:
         b, qh, ql, kv_len = probs.shape
         kvh, cap, hd = v.shape[1], v.shape[2], v.shape[3]
         out = out or self.empty((b, qh, ql, hd), probs.dtype)
-        self._call(f"rl_gqa_pv_matmul_{self._sfx(probs)}", probs, v, b, qh, kvh, ql, kv_len, hd,
+        self._call("gqa_pv_matmul", probs, probs, v, b, qh, kvh, ql, kv_len, hd,
                    cap, out)
         return out
 
@@ -574,6 +599,6 @@ class Context:
         ids = np.ascontiguousarray(token_ids, dtype=np.uint32)
         vocab, hidden = weight.shape
         out = out or self.empty((ids.size, hidden), weight.dtype)
-        self._call(f"rl_embedding_{self._sfx(weight)}", weight, vocab, hidden,
+        self._call("embedding", weight, weight, vocab, hidden,
                    ids.ctypes.data_as(ctypes.POINTER(ctypes.c_uint32)), ids.size, out)
         return out
