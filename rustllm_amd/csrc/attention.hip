@@ -21,8 +21,9 @@
 // transposed operand comes from the LDS transpose read (ds_read_b64_tr_b16).
 // K and V blocks travel from memory to LDS by DMA (buffer loads into LDS,
 // two stages deep), so the next block streams in during this one's compute.
-// f32 with the same head sizes takes v_mfma_f32_32x32x2_f32 in the same
-// tiling (its own key order, f32 probabilities).  Decode steps (few query
+// f32 with the multiples of 32 up to 128 takes the bf16 matrix cores in the
+// same tiling, each f32 operand as three bf16 parts (f32 probabilities).
+// Decode steps (few query
 // rows per KV head) split the keys over many workgroups; other head sizes
 // (f16 off the multiples of 8 or above 256, f32 off those of 32, up to 512)
 // take a one-wave-per-query kernel on the vector ALUs.
@@ -632,37 +633,57 @@ __global__ __launch_bounds__(256) void k_flash_combine(half_t* __restrict__ out,
     }
 }
 
-// ------------------------------------------------- f32 on the matrix cores
+// ------------------------------------ f32 on the bf16 matrix cores
 
-// f32 takes v_mfma_f32_32x32x2_f32 (two head elements per step, exact f32
-// products) with K rows in the key_row32 order, so each lane's probabilities
-// are the B operand of the P V step as they stand; K rows at a stride of
-// 2 mod 64 floats and V rows at 32 mod 64 (f32_stride) keep the operand
-// reads on 64 distinct banks.
-// Same tiling as k_flash_attention (QW waves of 32 queries, KSPLIT key
-// shares merged through LDS, causal tiles paired), blocks staged through
-// registers; scores, probabilities and the running sum stay in f32.
+// The tiling of k_flash_attention with every f32 product made of bf16 parts
+// (Bf16x3): the queries are split once into registers; a block of K and V
+// passes through registers, is split there and stored as three planes each
+// (K in the perm32 key order, rows in the chunk order of lds_swizzle); the
+// probabilities are split 16 keys at a time.  Scores, probabilities and sums
+// are f32 throughout.  Two LDS stages where they fit (a step's block is split
+// and stored before the previous one's products, one barrier a step), else one.
+// A query whose output is not finite, or has an element too small for its
+// values' low parts (the matrix cores take bf16 subnormals as zero), is
+// computed again unsplit (exact_row), and so is a query with elements outside
+// 2^-64 .. 2^64, so that the parts lost from a score are below 2^-61 of one.
+// Bound by matrix and vector work in turn (they do not overlap: 35 % matrix,
+// 34 % vector, ~19 vector operations a score, at 69 % balance of the tiles
+// over the CUs).  One MI355X against v_mfma_f32_32x32x2_f32 in the same
+// tiling (which it replaces): 15 heads of 64 x [3001, 3001] 213 -> 120 us, relative
+// error against 64 bits 3.6e-7 -> 3.0e-7; 32 of 64 x 500 queries after 3000
+// keys 306 -> 99 us; 12 of 128 x [1900, 1900] 185 -> 136 us; 9 x [64, 64]
+// 10.5 -> 8.0 us.  Software-pipelined over the blocks (the next block's scores
+// beside this one's exponentials), or with the two waves of a SIMD splitting at
+// different ends of a step, it was no faster (124 and 133 us for 119).
 template <int NT, int QW, int KSPLIT, int BN>
-__global__ __launch_bounds__(64 * QW * KSPLIT) void k_flash_attention_f32(
+__global__ __launch_bounds__(64 * QW * KSPLIT) void k_flash_attention_bf16x3(
     const float* __restrict__ q, const float* __restrict__ k, const float* __restrict__ v,
     float* __restrict__ out, AttnParams p) {
     constexpr int D = 32 * NT;
-    constexpr int DS = D / 2;  // MFMA steps over the head
-    constexpr int KT = BN / 32;
-    constexpr int KS = f32_stride(D, 2);
-    constexpr int VS = f32_stride(D, 32);
+    constexpr int DC = D / 16;             // 16-wide slices of a head
+    constexpr int KT = BN / 32;            // 32-key tiles per block
+    constexpr int RD = NT == 3 ? 128 : D;  // elements of an LDS row
+    constexpr int SW = RD / 32;            // its chunk order (lds_swizzle)
     constexpr int THREADS = 64 * QW * KSPLIT;
     constexpr int TILE_Q = 32 * QW;
-    constexpr int ROW_CHUNKS = D / 4;                   // 16-byte chunks of a row
+    constexpr int ROW_CHUNKS = RD / 8;     // 8-element chunks of a row
     constexpr int BLOCK_CHUNKS = BN * ROW_CHUNKS;
     constexpr int LOADS = BLOCK_CHUNKS * KSPLIT / THREADS;
-    constexpr int KV_FLOATS = BN * KS + BN * VS;        // one block of K and V
-    constexpr int MERGE = NT * 16 + 2;
-    constexpr int LDS_FLOATS = KSPLIT * KV_FLOATS > (KSPLIT - 1) * QW * 64 * MERGE
-                                   ? KSPLIT * KV_FLOATS
-                                   : (KSPLIT - 1) * QW * 64 * MERGE;
+    constexpr int PLANE = BN * RD;         // one part of a K or V block
+    constexpr int STAGE = KSPLIT * 6 * PLANE;
+    constexpr int NSTAGE = 2 * STAGE * 2 <= 128 * 1024 ? 2 : 1;
+    constexpr int MERGE = NT * 16 + 2;     // floats a lane hands over
+    // Four waves have the registers to sum the smaller products apart, one
+    // rounding of the large sum a slice instead of six: with two key shares
+    // the chains are long (32 heads of 128 x 500 queries after 2500 keys, error
+    // against 64 bits: 6.7e-7 in one chain, 4.1e-7 apart; f32 products 6.3e-7).
+    constexpr bool APART = QW * KSPLIT == 4;
+    constexpr int LDS_BYTES = NSTAGE * STAGE * 2 > (KSPLIT - 1) * QW * 64 * MERGE * 4
+                                  ? NSTAGE * STAGE * 2
+                                  : (KSPLIT - 1) * QW * 64 * MERGE * 4;
     static_assert((BLOCK_CHUNKS * KSPLIT) % THREADS == 0, "blocks must split evenly");
-    __shared__ __align__(16) float lds[LDS_FLOATS];
+    __shared__ __align__(16) unsigned char lds[LDS_BYTES];
+    __bf16* const kv_lds = reinterpret_cast<__bf16*>(lds);
 
     const bool by_tile = p.pairs == p.tiles;  // as in k_flash_attention
     const uint32_t per = by_tile ? p.heads : p.pairs;
@@ -680,9 +701,24 @@ __global__ __launch_bounds__(64 * QW * KSPLIT) void k_flash_attention_f32(
     const uint32_t col = lane % 32;
     const uint32_t hs = lane / 32;
 
+    // operand offsets, as in k_flash_attention
+    uint32_t koff[DC];
+#pragma unroll
+    for (int c = 0; c < DC; ++c) koff[c] = col * RD + 8 * ((2 * c + hs) ^ lds_swizzle<SW>(col));
+    uint32_t voff[2][NT];
+#pragma unroll
+    for (int e2 = 0; e2 < 2; ++e2) {
+        const uint32_t row = 8 * (lane / 32) + (lane % 16) / 4 + 4 * e2;
+#pragma unroll
+        for (int t = 0; t < NT; ++t) {
+            const uint32_t ch = 2 * ((lane / 16) % 2) + (lane % 4) / 2 + 4 * t;
+            voff[e2][t] = row * RD + 8 * (ch ^ lds_swizzle<SW>(row)) + 4 * (lane % 2);
+        }
+    }
+
     for (int which = 0; which < 2; ++which) {
         const uint32_t tile = which == 0 ? p.tiles - 1 - pair : pair;
-        if (which == 1 && (p.pairs == p.tiles || tile >= p.tiles - 1 - pair)) break;
+        if (which == 1 && (by_tile || tile >= p.tiles - 1 - pair)) break;
         const uint32_t q_first = tile * TILE_Q;
         const uint32_t q_last = min(p.q_len, q_first + TILE_Q) - 1;
         const uint32_t keys = min(p.kv_len, p.start + q_last + 1);
@@ -692,95 +728,123 @@ __global__ __launch_bounds__(64 * QW * KSPLIT) void k_flash_attention_f32(
         const bool wave_active = qw0 < p.q_len;
         const uint32_t wave_keys =
             wave_active ? min(p.kv_len, p.start + min(qw0 + 31, p.q_len - 1) + 1) : 0;
-
-        // B operand of S^T = K Q^T: lane (col, hs) holds elements 2j + hs of
-        // its query for every step j.
         const uint32_t qi = qw0 + col;
         const bool q_valid = qi < p.q_len;
         const uint32_t key_limit = min(p.start + qi, p.kv_len - 1);
-        float qf[DS];
-        const float* qrow = q + (uint64_t(bh) * p.q_len + (q_valid ? qi : 0)) * D + hs;
-#pragma unroll
-        for (int j = 0; j < DS; ++j) qf[j] = q_valid ? qrow[2 * j] : 0.0f;
 
-        f32x16 o[NT];
-#pragma unroll
-        for (int t = 0; t < NT; ++t)
-#pragma unroll
-            for (int r = 0; r < 16; ++r) o[t][r] = 0.0f;
-        float m = -INFINITY, l = 0.0f;
-
-        float4 kreg[LOADS], vreg[LOADS];
-        bool vlive[LOADS];
+        // 8 consecutive elements of a row per chunk; rows past kv_len are not
+        // read (they may hold anything): a key past the end loads row
+        // kv_len - 1, its score is masked and its value row zeroed
+        f32x8 kreg[LOADS], vreg[LOADS];
         auto load_step = [&](uint32_t step) {
 #pragma unroll
             for (int li = 0; li < LOADS; ++li) {
                 const uint32_t chunk = threadIdx.x + THREADS * li;
-                const uint32_t blk = step * KSPLIT + chunk / BLOCK_CHUNKS;
                 const uint32_t c = chunk % BLOCK_CHUNKS;
-                const uint32_t key = blk * BN + c / ROW_CHUNKS;
-                const uint32_t d0 = (c % ROW_CHUNKS) * 4;
-                // rows past kv_len are not read (they may hold anything): a
-                // key past the end loads row kv_len - 1, its score is masked
-                // and its value row zeroed at the LDS store
-                const uint32_t row = min(key, p.kv_len - 1);
-                kreg[li] = *reinterpret_cast<const float4*>(kh + uint64_t(row) * D + d0);
-                vreg[li] = *reinterpret_cast<const float4*>(vh + uint64_t(row) * D + d0);
-                vlive[li] = key < p.kv_len;
+                const uint32_t key = (step * KSPLIT + chunk / BLOCK_CHUNKS) * BN + c / ROW_CHUNKS;
+                const uint32_t ch = c % ROW_CHUNKS;
+                if (RD > D && ch >= D / 8) continue;  // head size 96: 12 of 16 chunks
+                const uint64_t at = uint64_t(min(key, p.kv_len - 1)) * D + ch * 8;
+                const f32x4 k0 = *reinterpret_cast<const f32x4*>(kh + at);
+                const f32x4 k1 = *reinterpret_cast<const f32x4*>(kh + at + 4);
+                const f32x4 v0 = *reinterpret_cast<const f32x4*>(vh + at);
+                const f32x4 v1 = *reinterpret_cast<const f32x4*>(vh + at + 4);
+                kreg[li] = __builtin_shufflevector(k0, k1, 0, 1, 2, 3, 4, 5, 6, 7);
+                vreg[li] = __builtin_shufflevector(v0, v1, 0, 1, 2, 3, 4, 5, 6, 7);
             }
         };
-        auto store_step = [&]() {
+        auto store_step = [&](uint32_t step) {
+            __bf16* stage = kv_lds + (step % NSTAGE) * STAGE;
 #pragma unroll
             for (int li = 0; li < LOADS; ++li) {
                 const uint32_t chunk = threadIdx.x + THREADS * li;
                 const uint32_t c = chunk % BLOCK_CHUNKS;
-                float* kdst = lds + (chunk / BLOCK_CHUNKS) * KV_FLOATS;
-                float* vdst = kdst + BN * KS;
-                const uint32_t key = c / ROW_CHUNKS;
-                const uint32_t d0 = (c % ROW_CHUNKS) * 4;
-                // K rows at the rotated order, 8-byte aligned (stride 2 mod 64)
-                float* kr = kdst + ((key & ~31u) | key_row32(key & 31u)) * KS + d0;
-                *reinterpret_cast<float2*>(kr) = float2{kreg[li].x, kreg[li].y};
-                *reinterpret_cast<float2*>(kr + 2) = float2{kreg[li].z, kreg[li].w};
-                // per-component selects: a select of two float4 structs goes
-                // through private memory
-                const bool live = vlive[li];
-                *reinterpret_cast<float4*>(vdst + key * VS + d0) =
-                    float4{live ? vreg[li].x : 0.0f, live ? vreg[li].y : 0.0f,
-                           live ? vreg[li].z : 0.0f, live ? vreg[li].w : 0.0f};
+                const uint32_t share = chunk / BLOCK_CHUNKS;
+                const uint32_t r = c / ROW_CHUNKS, ch = c % ROW_CHUNKS;
+                if (RD > D && ch >= D / 8) continue;
+                __bf16* ks = stage + share * 6 * PLANE;
+                __bf16* vs = ks + 3 * PLANE;
+                const uint32_t kr = (r & ~31u) | perm32(r & 31u);
+                const uint32_t kat = kr * RD + 8 * (ch ^ lds_swizzle<SW>(kr));
+                const uint32_t vat = r * RD + 8 * (ch ^ lds_swizzle<SW>(r));
+                const bool live = (step * KSPLIT + share) * BN + r < p.kv_len;
+                f32x8 vx = vreg[li];
+#pragma unroll
+                for (int e = 0; e < 8; ++e) vx[e] = live ? vx[e] : 0.0f;
+                const Bf16x3 kp = split_bf16(kreg[li]), vp = split_bf16(vx);
+#pragma unroll
+                for (int i = 0; i < 3; ++i) {
+                    *reinterpret_cast<b8*>(ks + i * PLANE + kat) = kp.part[i];
+                    *reinterpret_cast<b8*>(vs + i * PLANE + vat) = vp.part[i];
+                }
             }
         };
-
         load_step(0);
-        __syncthreads();  // the previous tile's LDS use is over
-        store_step();
+
+        // B operand of S^T = K Q^T: lane (col, hs) holds elements
+        // 16c + 8hs .. + 7 of its query for every slice c
+        Bf16x3 qf[DC];
+        const float* qrow = q + (uint64_t(bh) * p.q_len + (q_valid ? qi : 0)) * D + 8 * hs;
+#pragma unroll
+        for (int c = 0; c < DC; ++c) {
+            const f32x4 x0 = *reinterpret_cast<const f32x4*>(qrow + 16 * c);
+            const f32x4 x1 = *reinterpret_cast<const f32x4*>(qrow + 16 * c + 4);
+            f32x8 x = __builtin_shufflevector(x0, x1, 0, 1, 2, 3, 4, 5, 6, 7);
+#pragma unroll
+            for (int e = 0; e < 8; ++e) x[e] = q_valid ? x[e] : 0.0f;
+            qf[c] = split_bf16(x);
+        }
+        f32x16 o[NT], low[APART ? NT : 1];
+#pragma unroll
+        for (int t = 0; t < NT; ++t)
+#pragma unroll
+            for (int r = 0; r < 16; ++r) {
+                o[t][r] = 0.0f;
+                low[APART ? t : 0][r] = 0.0f;
+            }
+        float m = -INFINITY, l = 0.0f;
+
+        store_step(0);  // the previous tile's LDS use ended with a barrier
+        if (NSTAGE == 2 && steps > 1) load_step(1);
         __syncthreads();
         for (uint32_t step = 0; step < steps; ++step) {
-            if (step + 1 < steps) load_step(step + 1);
+            if constexpr (NSTAGE == 2) {
+                if (step + 1 < steps) {
+                    store_step(step + 1);
+                    if (step + 2 < steps) load_step(step + 2);
+                }
+            } else {
+                if (step + 1 < steps) load_step(step + 1);
+            }
             const uint32_t blk = step * KSPLIT + sub;
-            const float* ks = lds + sub * KV_FLOATS;
-            const float* vs = ks + BN * KS;
+            const __bf16* ks = kv_lds + (step % NSTAGE) * STAGE + sub * 6 * PLANE;
+            const __bf16* vs = ks + 3 * PLANE;
             if (blk < blocks && blk * BN < wave_keys) {
                 f32x16 s[KT];
 #pragma unroll
                 for (int kt = 0; kt < KT; ++kt) {
 #pragma unroll
                     for (int r = 0; r < 16; ++r) s[kt][r] = 0.0f;
-                    const float* krow = ks + (kt * 32 + col) * KS + hs;
 #pragma unroll
-                    for (int j = 0; j < DS; ++j)
-                        s[kt] = __builtin_amdgcn_mfma_f32_32x32x2f32(krow[2 * j], qf[j], s[kt], 0,
-                                                                      0, 0);
+                    for (int c = 0; c < DC; ++c) {
+                        Bf16x3 ka;
+#pragma unroll
+                        for (int i = 0; i < 3; ++i)
+                            ka.part[i] = *reinterpret_cast<const b8*>(ks + i * PLANE +
+                                                                      kt * 32 * RD + koff[c]);
+                        s[kt] = mfma_bf16x3(ka, qf[c], s[kt]);
+                    }
                 }
-                // register r of tile kt holds key kbase + 32 kt + 2r + hs
+                // register r of tile kt holds key
+                // kbase + 32 kt + 16 (r / 8) + 8 hs + r % 8
                 const uint32_t kbase = blk * BN;
                 if (kbase + BN - 1 > p.start + qw0 || kbase + BN > p.kv_len) {
-                    const int lim = int(key_limit) - int(kbase + hs);
+                    const int lim = int(key_limit) - int(kbase + 8 * hs);
 #pragma unroll
                     for (int kt = 0; kt < KT; ++kt)
 #pragma unroll
                         for (int r = 0; r < 16; ++r)
-                            if (kt * 32 + 2 * r > lim) s[kt][r] = -INFINITY;
+                            if (kt * 32 + 16 * (r >> 3) + (r & 7) > lim) s[kt][r] = -INFINITY;
                 }
                 // scores in log2 units first, so that the largest one's
                 // probability is exactly 1 (2^(t - m) with t == m)
@@ -806,45 +870,68 @@ __global__ __launch_bounds__(64 * QW * KSPLIT) void k_flash_attention_f32(
 #pragma unroll
                     for (int t = 0; t < NT; ++t)
 #pragma unroll
-                        for (int r = 0; r < 16; ++r) o[t][r] *= alpha;
+                        for (int r = 0; r < 16; ++r) {
+                            o[t][r] *= alpha;
+                            if constexpr (APART) low[t][r] *= alpha;
+                        }
                 }
-                // p = 2^(t - m), in place; a query that has seen no key yet
-                // (m = -inf) has only -inf scores, and p = 0
+                // p = 2^(t - m); a query that has seen no key yet (m = -inf)
+                // has only -inf scores, and p = 0
                 const float neg_m = m == -INFINITY ? 0.0f : -m;
                 float la = 0.0f, lb = 0.0f;
 #pragma unroll
-                for (int kt = 0; kt < KT; ++kt)
+                for (int c = 0; c < BN / 16; ++c) {
+                    f32x8 x;
 #pragma unroll
-                    for (int r = 0; r < 16; r += 2) {
-                        s[kt][r] = __builtin_amdgcn_exp2f(s[kt][r] + neg_m);
-                        s[kt][r + 1] = __builtin_amdgcn_exp2f(s[kt][r + 1] + neg_m);
-                        la += s[kt][r];
-                        lb += s[kt][r + 1];
+                    for (int e = 0; e < 8; e += 2) {
+                        x[e] = __builtin_amdgcn_exp2f(s[c >> 1][8 * (c & 1) + e] + neg_m);
+                        x[e + 1] = __builtin_amdgcn_exp2f(s[c >> 1][8 * (c & 1) + e + 1] + neg_m);
+                        la += x[e];
+                        lb += x[e + 1];
                     }
+                    const Bf16x3 pb = split_bf16(x);
+                    // O^T += V^T P^T over these 16 keys
+#pragma unroll
+                    for (int t = 0; t < NT; ++t) {
+                        Bf16x3 va;
+#pragma unroll
+                        for (int i = 0; i < 3; ++i) {
+                            const half_t* plane =
+                                reinterpret_cast<const half_t*>(vs + i * PLANE + 16 * c * RD);
+                            const h4 lo = lds_read_transposed(plane + voff[0][t]);
+                            const h4 hi = lds_read_transposed(plane + voff[1][t]);
+                            const h8 w = {lo[0], lo[1], lo[2], lo[3], hi[0], hi[1], hi[2], hi[3]};
+                            va.part[i] = __builtin_bit_cast(b8, w);
+                        }
+                        if constexpr (APART) {
+                            low[t] = mfma_bf16x3_low(va, pb, low[t]);
+                            o[t] = __builtin_amdgcn_mfma_f32_32x32x16_bf16(va.part[0], pb.part[0],
+                                                                           o[t], 0, 0, 0);
+                        } else {
+                            o[t] = mfma_bf16x3(va, pb, o[t]);
+                        }
+                    }
+                }
                 l += la + lb;
-                // O^T += V^T P^T over keys 2r, 2r + 1 of each tile: lane
-                // (col, hs) supplies V[2r + hs][32t + col] and P of its query
-                // at key 2r + hs (register r).
-#pragma unroll
-                for (int kt = 0; kt < KT; ++kt)
-#pragma unroll
-                    for (int r = 0; r < 16; ++r) {
-                        const float* vrow = vs + (kt * 32 + 2 * r + hs) * VS + col;
-#pragma unroll
-                        for (int t = 0; t < NT; ++t)
-                            o[t] = __builtin_amdgcn_mfma_f32_32x32x2f32(vrow[32 * t], s[kt][r],
-                                                                         o[t], 0, 0, 0);
-                    }
             }
             __syncthreads();
-            if (step + 1 < steps) store_step();
-            __syncthreads();
+            if constexpr (NSTAGE == 1) {
+                if (step + 1 < steps) store_step(step + 1);
+                __syncthreads();
+            }
         }
 
+        if constexpr (APART) {
+#pragma unroll
+            for (int t = 0; t < NT; ++t)
+#pragma unroll
+                for (int r = 0; r < 16; ++r) o[t][r] += low[t][r];
+        }
         if constexpr (KSPLIT > 1) {
             // Groups 1.. hand their (max, sum, output) to group 0 through LDS.
+            float* mg = reinterpret_cast<float*>(lds);
             if (sub > 0) {
-                float* dst = lds + ((sub - 1) * QW * 64 + qw * 64 + lane) * MERGE;
+                float* dst = mg + ((sub - 1) * QW * 64 + qw * 64 + lane) * MERGE;
                 dst[0] = m;
                 dst[1] = l;
 #pragma unroll
@@ -856,7 +943,7 @@ __global__ __launch_bounds__(64 * QW * KSPLIT) void k_flash_attention_f32(
             if (sub == 0) {
 #pragma unroll
                 for (int h = 1; h < KSPLIT; ++h) {
-                    const float* src = lds + ((h - 1) * QW * 64 + qw * 64 + lane) * MERGE;
+                    const float* src = mg + ((h - 1) * QW * 64 + qw * 64 + lane) * MERGE;
                     const float m2 = src[0];
                     const float m_tot = fmaxf(m, m2);
                     const float a1 = m_tot > m ? __builtin_amdgcn_exp2f(m - m_tot) : 1.0f;
@@ -875,16 +962,41 @@ __global__ __launch_bounds__(64 * QW * KSPLIT) void k_flash_attention_f32(
 
         if (sub == 0) {
             const float inv = 1.0f / (l + __shfl_xor(l, 32, 64));  // both halves of the query
+            bool exact = false;  // this lane's half of a query needs exact_row
+            if (q_valid) {
+#pragma unroll
+                for (int c = 0; c < DC; ++c)
+#pragma unroll
+                    for (int e = 0; e < 8; ++e) {
+                        const float a = fabsf(qrow[16 * c + e]);
+                        exact |= a != 0.0f && !(a > 0x1p-64f && a < 0x1p64f);
+                    }
+            }
             if (q_valid) {
                 // register r of tile t: element 32t + 8(r / 4) + 4hs + r % 4
                 float* orow = out + (uint64_t(bh) * p.q_len + qi) * D + 4 * hs;
 #pragma unroll
                 for (int t = 0; t < NT; ++t)
 #pragma unroll
-                    for (int g = 0; g < 4; ++g)
-                        *reinterpret_cast<float4*>(orow + 32 * t + 8 * g) =
-                            float4{o[t][4 * g] * inv, o[t][4 * g + 1] * inv,
-                                   o[t][4 * g + 2] * inv, o[t][4 * g + 3] * inv};
+                    for (int g = 0; g < 4; ++g) {
+                        f32x4 w;
+#pragma unroll
+                        for (int e = 0; e < 4; ++e) {
+                            w[e] = o[t][4 * g + e] * inv;
+                            const float a = fabsf(w[e]);
+                            exact |= a != 0.0f && !(a > 0x1p-96f && a < INFINITY);
+                        }
+                        *reinterpret_cast<f32x4*>(orow + 32 * t + 8 * g) = w;
+                    }
+            }
+            uint64_t redo = __ballot(exact);
+            redo = (redo | redo >> 32) & 0xffffffffu;
+            while (redo != 0) {
+                const uint32_t c = __builtin_ctzll(redo);
+                redo &= redo - 1;
+                const uint64_t row = uint64_t(bh) * p.q_len + qw0 + c;
+                exact_row<float, NT>(q + row * D, kh, vh, out + row * D, D,
+                                     min(p.kv_len, p.start + qw0 + c + 1), p.scale);
             }
         }
     }
@@ -1606,14 +1718,10 @@ rl_status validate_attention(const rl_buffer* q, const rl_buffer* k, const rl_bu
 // K and V then take 64, 128 and 128 KB of LDS for head sizes 32, 64, 128).
 constexpr int kFlashMaxBlockKeys = 128;
 constexpr int kFlashMaxKeySplit = 4;
-// f32 (one MI355X, all launches inside the events): the 32-query tiles win up to
-// at least 128 pairs (8 heads x [4096, 4096]: 203 against 308 us), the wide
-// tiles at 180 (15 heads x [3072, 3072]: 240 against 281 us)
-constexpr uint64_t kFlashFillBlocks = 180;
-constexpr uint64_t kFlashFillBlocksF16 = 96;    // f16: wide tiles from here on
+constexpr uint64_t kFlashFillBlocks = 96;  // wide tiles from here on
 
-// Workgroup shape: 4 query waves x 2 key shares (128-query tiles) while that
-// gives enough workgroups (`fill`); otherwise 32-query tiles, so that short
+// f16 workgroup shape: 4 query waves x 2 key shares (128-query tiles) while that
+// gives enough workgroups (kFlashFillBlocks pairs); otherwise 32-query tiles, so that short
 // or few-head prefills spread over more CUs: 1 query wave x 2 key shares, or
 // x 4 when the workgroups are still few or the head is large (96, 128: more
 // waves per workgroup keep all four SIMDs busy).  f16, one MI355X, all
@@ -1622,8 +1730,8 @@ constexpr uint64_t kFlashFillBlocksF16 = 96;    // f16: wide tiles from here on
 // 71.8 -> 37.0, 8 heads x [4096, 4096] 52.1 -> 44.8) and lose below 64
 // (15 heads x [1024, 1024]: 19.1 against 14.2 us for 32-query tiles).
 enum class FlashShape { kWide, kNarrow2, kNarrow4 };
-FlashShape flash_shape(uint64_t heads, uint64_t q_len, uint64_t head_dim, uint64_t fill) {
-    if (heads * ((ceil_div(q_len, 128) + 1) / 2) >= fill) return FlashShape::kWide;
+FlashShape flash_shape(uint64_t heads, uint64_t q_len, uint64_t head_dim) {
+    if (heads * ((ceil_div(q_len, 128) + 1) / 2) >= kFlashFillBlocks) return FlashShape::kWide;
     if (head_dim >= 96 || heads * ((ceil_div(q_len, 32) + 1) / 2) < 256) return FlashShape::kNarrow4;
     return FlashShape::kNarrow2;
 }
@@ -1664,7 +1772,7 @@ uint32_t flash_key_chunks(uint64_t heads, uint64_t q_len, uint64_t kv_len, uint6
     const uint64_t bn = head_dim <= 64 ? 128 : 64;
     const uint64_t keys = std::min<uint64_t>(kv_len, start + q_len);  // the longest tile's
     const uint64_t steps = ceil_div(ceil_div(keys, bn), 2);
-    if (wide >= kFlashFillBlocksF16) return wide <= 128 && steps >= 16 ? 2 : 1;
+    if (wide >= kFlashFillBlocks) return wide <= 128 && steps >= 16 ? 2 : 1;
     if (start == 0 || steps < 16) return 1;
     const uint64_t chunks = std::min<uint64_t>({256 / wide, 8, steps / 2});
     return uint32_t(std::max<uint64_t>(chunks, 1));
@@ -1713,22 +1821,44 @@ void launch_flash_split(rl_context* ctx, uint64_t heads, uint32_t nt, const half
     }
 }
 
-template <int QW, int KS>
-void launch_flash(rl_context* ctx, dim3 g, uint32_t nt, const float* q, const float* k,
-                  const float* v, float* o, const AttnParams& p) {
-    constexpr int BN = QW == 4 ? 64 : 32;
-    const dim3 b(64 * QW * KS);
-    if (nt == 1) {
-        RL_LAUNCH(ctx, (k_flash_attention_f32<1, QW, KS, BN>), g, b, q, k, v, o, p);
-    } else if (nt == 2) {
-        RL_LAUNCH(ctx, (k_flash_attention_f32<2, QW, KS, BN>), g, b, q, k, v, o, p);
-    } else if constexpr (!(QW == 1 && KS == 2)) {  // that shape only for head sizes <= 64
-        if (nt == 3) {
-            RL_LAUNCH(ctx, (k_flash_attention_f32<3, QW, KS, 32>), g, b, q, k, v, o, p);
-        } else {
-            RL_LAUNCH(ctx, (k_flash_attention_f32<4, QW, KS, 32>), g, b, q, k, v, o, p);
-        }
+// f32: 128-query tiles of two key shares from kWideF32 tile pairs, else
+// 64-query tiles of four shares (two for head sizes 96 and 128, whose blocks
+// leave no LDS for more, and for at most 128 keys); blocks of 32 keys (64 for
+// head size 32 with 128-query tiles).
+template <int NT, int QW, int KS, int BN>
+void launch_flash_f32(rl_context* ctx, dim3 g, const float* q, const float* k, const float* v,
+                      float* o, const AttnParams& p) {
+    RL_LAUNCH(ctx, (k_flash_attention_bf16x3<NT, QW, KS, BN>), g, dim3(64 * QW * KS), q, k, v, o,
+              p);
+}
+// 128-query tiles against 64 (one MI355X): 15 heads of 64 x [3001, 3001] (180
+// pairs) 124 / 140 us, 32 of 96 x [1200, 1200] (160) 81 / 106; 32 of 64 x [1000,
+// 1000] (128) 44.7 / 38.9, 15 x [2000, 2000] (120) 77.5 / 63.9.
+constexpr uint64_t kWideF32 = 150;
+rl_status launch_flash_f32(rl_context* ctx, uint64_t heads, const float* q, const float* k,
+                           const float* v, float* o, AttnParams p) {
+    const uint32_t nt = p.head_dim / 32;
+    const bool wide = heads * ((ceil_div(p.q_len, 128) + 1) / 2) >= kWideF32;
+    p.tiles = uint32_t(ceil_div(p.q_len, wide ? 128 : 64));
+    p.pairs = flash_pairs(ctx, heads, p.tiles);
+    const uint64_t grid = heads * p.pairs;
+    if (grid > UINT32_MAX) return fail(RL_ERR_INVALID_SHAPE, "attention grid exceeds u32");
+    const dim3 g(static_cast<unsigned>(grid));
+    if (wide) {
+        if (nt == 1) launch_flash_f32<1, 4, 2, 64>(ctx, g, q, k, v, o, p);
+        else if (nt == 2) launch_flash_f32<2, 4, 2, 32>(ctx, g, q, k, v, o, p);
+        else if (nt == 3) launch_flash_f32<3, 4, 2, 32>(ctx, g, q, k, v, o, p);
+        else launch_flash_f32<4, 4, 2, 32>(ctx, g, q, k, v, o, p);
+    } else if (nt <= 2 && std::min<uint64_t>(p.kv_len, uint64_t(p.start) + p.q_len) > 128) {
+        if (nt == 1) launch_flash_f32<1, 2, 4, 32>(ctx, g, q, k, v, o, p);
+        else launch_flash_f32<2, 2, 4, 32>(ctx, g, q, k, v, o, p);
+    } else {
+        if (nt == 1) launch_flash_f32<1, 2, 2, 32>(ctx, g, q, k, v, o, p);
+        else if (nt == 2) launch_flash_f32<2, 2, 2, 32>(ctx, g, q, k, v, o, p);
+        else if (nt == 3) launch_flash_f32<3, 2, 2, 32>(ctx, g, q, k, v, o, p);
+        else launch_flash_f32<4, 2, 2, 32>(ctx, g, q, k, v, o, p);
     }
+    return RL_OK;
 }
 
 // The f16 kernel for padded head sizes (ANY), blocks and staging as above;
@@ -1744,7 +1874,7 @@ rl_status launch_flash_any(rl_context* ctx, uint64_t heads, const half_t* q, con
                            const half_t* v, half_t* o, AttnParams p) {
     const uint32_t nt = (p.head_dim + 31) / 32;
     const bool wide =
-        nt <= 4 && flash_shape(heads, p.q_len, 32 * nt, kFlashFillBlocksF16) == FlashShape::kWide;
+        nt <= 4 && flash_shape(heads, p.q_len, 32 * nt) == FlashShape::kWide;
     p.tiles = uint32_t(ceil_div(p.q_len, wide ? 128 : nt > 4 ? 64 : 32));
     p.pairs = flash_pairs(ctx, heads, p.tiles);
     const uint64_t grid = heads * p.pairs;
@@ -2004,18 +2134,21 @@ rl_status attention_entry(rl_context* ctx, const char* name, const rl_buffer* q,
                 return st;
             }
         }
-        const FlashShape shape =
-            flash_shape(heads, s.q_len, s.head_dim,
-                        sizeof(T) == 2 ? kFlashFillBlocksF16 : kFlashFillBlocks);
-        p.tiles = uint32_t(ceil_div(s.q_len, shape == FlashShape::kWide ? 128 : 32));
-        p.pairs = flash_pairs(ctx, heads, p.tiles);
-        const uint64_t grid = heads * p.pairs;
-        if (grid > UINT32_MAX) return fail(RL_ERR_INVALID_SHAPE, "attention grid exceeds u32");
-        const dim3 g(static_cast<unsigned>(grid));
-        const uint32_t nt = uint32_t(s.head_dim / 32);
-        if (shape == FlashShape::kWide) launch_flash<4, 2>(ctx, g, nt, qd, kd, vd, od, p);
-        else if (shape == FlashShape::kNarrow2) launch_flash<1, 2>(ctx, g, nt, qd, kd, vd, od, p);
-        else launch_flash<1, 4>(ctx, g, nt, qd, kd, vd, od, p);
+        if constexpr (std::is_same<T, half_t>::value) {
+            const FlashShape shape = flash_shape(heads, s.q_len, s.head_dim);
+            p.tiles = uint32_t(ceil_div(s.q_len, shape == FlashShape::kWide ? 128 : 32));
+            p.pairs = flash_pairs(ctx, heads, p.tiles);
+            const uint64_t grid = heads * p.pairs;
+            if (grid > UINT32_MAX)
+                return fail(RL_ERR_INVALID_SHAPE, "attention grid exceeds u32");
+            const dim3 g(static_cast<unsigned>(grid));
+            const uint32_t nt = uint32_t(s.head_dim / 32);
+            if (shape == FlashShape::kWide) launch_flash<4, 2>(ctx, g, nt, qd, kd, vd, od, p);
+            else if (shape == FlashShape::kNarrow2) launch_flash<1, 2>(ctx, g, nt, qd, kd, vd, od, p);
+            else launch_flash<1, 4>(ctx, g, nt, qd, kd, vd, od, p);
+        } else {
+            if (rl_status st = launch_flash_f32(ctx, heads, qd, kd, vd, od, p)) return st;
+        }
         return after_launch(ctx, name);
     }
     if constexpr (std::is_same<T, half_t>::value) {

@@ -30,14 +30,6 @@ __device__ inline uint32_t perm32(uint32_t i) {
     return (i & ~12u) | ((i & 4u) << 1) | ((i & 8u) >> 1);
 }
 
-// f32: LDS row i = 8a + 4h + b of a 32-key tile holds key 8a + 2b + h (the
-// low three bits rotated), so that register r of a lane in half h holds key
-// 2r + h -- the B operand of the P V step over keys 2r and 2r + 1.
-// key_row32 is the row of key j.
-__device__ inline uint32_t key_row32(uint32_t j) {
-    return (j & ~7u) | ((j & 1u) << 2) | ((j >> 1) & 3u);
-}
-
 // Row stride (halves) of V in LDS for the transpose reads: the 32 lanes one
 // LDS cycle serves read 4 rows x 2 runs of 16 bytes; with 64 banks of 4
 // bytes those land on distinct banks when the stride in dwords is 16 or 48
@@ -65,6 +57,54 @@ __device__ inline h4 lds_read_transposed(const half_t* p) {
     const s16x4 r = __builtin_amdgcn_ds_read_tr16_b64_v4i16(
         (__attribute__((address_space(3))) s16x4*)(p));
     return __builtin_bit_cast(h4, r);
+}
+
+// f32 products on the bf16 matrix cores (v_mfma_f32_32x32x16_bf16, 16 times
+// the rate of the f32 ones).  An f32 value is the sum of three bf16 parts, each
+// the rounding of what the parts before it leave (8 + 8 + 8 bits, and their
+// signs: nothing is left of a normal value); of the nine products of two such
+// values the six of order 2^-18 and above are added, the three dropped are below
+// 2^-26 of the product.  Both operands of an instruction, and their layout,
+// are those of v_mfma_f32_32x32x16_f16.
+// An infinite or huge (>= 2^128 - 2^119) value's parts are not finite sums of
+// it (inf - inf): a result that is not finite has to be computed unsplit.
+typedef __bf16 b8 __attribute__((ext_vector_type(8)));
+typedef __bf16 b4 __attribute__((ext_vector_type(4)));
+typedef __bf16 b2 __attribute__((ext_vector_type(2)));
+typedef float f32x2 __attribute__((ext_vector_type(2)));
+typedef float f32x8 __attribute__((ext_vector_type(8)));
+
+struct Bf16x3 {
+    b8 part[3];  // high, middle, low
+};
+
+__device__ inline Bf16x3 split_bf16(f32x8 x) {
+    Bf16x3 r;
+#pragma unroll
+    for (int i = 0; i < 3; ++i)
+#pragma unroll
+        for (int e = 0; e < 8; e += 2) {
+            const b2 w = __builtin_convertvector((f32x2{x[e], x[e + 1]}), b2);
+            r.part[i][e] = w[0];
+            r.part[i][e + 1] = w[1];
+            x[e] -= float(w[0]);
+            x[e + 1] -= float(w[1]);
+        }
+    return r;
+}
+
+// acc += the five smaller products of a b, smallest first
+__device__ inline f32x16 mfma_bf16x3_low(const Bf16x3& a, const Bf16x3& b, f32x16 acc) {
+    acc = __builtin_amdgcn_mfma_f32_32x32x16_bf16(a.part[2], b.part[0], acc, 0, 0, 0);
+    acc = __builtin_amdgcn_mfma_f32_32x32x16_bf16(a.part[0], b.part[2], acc, 0, 0, 0);
+    acc = __builtin_amdgcn_mfma_f32_32x32x16_bf16(a.part[1], b.part[1], acc, 0, 0, 0);
+    acc = __builtin_amdgcn_mfma_f32_32x32x16_bf16(a.part[1], b.part[0], acc, 0, 0, 0);
+    return __builtin_amdgcn_mfma_f32_32x32x16_bf16(a.part[0], b.part[1], acc, 0, 0, 0);
+}
+// acc += a b
+__device__ inline f32x16 mfma_bf16x3(const Bf16x3& a, const Bf16x3& b, f32x16 acc) {
+    acc = mfma_bf16x3_low(a, b, acc);
+    return __builtin_amdgcn_mfma_f32_32x32x16_bf16(a.part[0], b.part[0], acc, 0, 0, 0);
 }
 
 }  // namespace

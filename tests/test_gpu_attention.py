@@ -467,3 +467,56 @@ TILE_ORDER_SHAPES = [
 @pytest.mark.parametrize("shape", TILE_ORDER_SHAPES)
 def test_attention_tile_order(ctx, dtype, shape):
     test_attention_within_float64_bound(ctx, dtype, shape)
+
+
+# ------------------------- f32 as bf16 parts: every workgroup shape, extremes
+
+F32_SHAPES = [
+    (1, 30, 10, 1250, 1250, 1280, 32, 0),   # 128-query tiles (150 pairs), ragged
+    (1, 50, 5, 700, 731, 736, 96, 31),
+    (1, 50, 5, 650, 650, 650, 128, 0),
+    (1, 3, 1, 129, 129, 160, 32, 0),        # 64-query tiles, four key shares
+    (2, 2, 2, 65, 200, 224, 64, 130),
+    (1, 4, 4, 63, 64, 64, 64, 1),           # at most 128 keys: two key shares
+    (1, 2, 1, 100, 128, 128, 32, 28),
+    (1, 4, 2, 90, 333, 352, 128, 200),
+    (1, 4, 2, 31, 31, 32, 96, 0),
+]
+
+
+@pytest.mark.parametrize("shape", F32_SHAPES)
+def test_attention_f32_shapes(ctx, shape):
+    test_attention_within_float64_bound(ctx, np.float32, shape)
+
+
+@pytest.mark.parametrize("hd,heads,ql", [(64, 4, 300), (96, 4, 130), (32, 150, 200)])
+def test_attention_f32_extremes(ctx, hd, heads, ql):
+    """Values whose low bf16 parts are subnormal, queries and keys at the ends
+    of the exponent range, and infinities: as in f32 products (the f32 bound;
+    its absolute term covers nothing here: it scales with the values)."""
+    q = synth.normal(51, (1, heads, ql, hd))
+    k = synth.normal(52, (1, heads // 2, ql, hd))
+    v = synth.normal(53, (1, heads // 2, ql, hd))
+    scale = 1.0 / np.sqrt(hd)
+    for qs, ks, vs in ((1, 1, 2.0 ** -118), (2.0 ** 90, 2.0 ** -90, 1), (2.0 ** -90, 2.0 ** 90, 1),
+                       (1, 1, 2.0 ** 120)):
+        x = [(a * np.float32(f)).astype(np.float32) for a, f in ((q, qs), (k, ks), (v, vs))]
+        got = run_attention(ctx, *x, scale, 0, ql).astype(np.float64) / vs
+        exact, bound = attention_bound(*[a.astype(np.float64) / f for a, f in
+                                         zip(x, (qs, ks, vs))], scale, 0, ql, "f32")
+        assert np.all(np.abs(got - exact) <= bound), (qs, ks, vs)
+    q, k, v = np.abs(q), k.copy(), v.copy()
+    k[0, :, 5] = -np.inf   # never contributes to queries >= 6
+    v[0, :, 20, 3] = np.inf
+    k[0, :, ql - 2] = np.nan
+    v[0, :, ql - 2] = np.nan
+    got = run_attention(ctx, q, k, v, scale, 0, ql).astype(np.float64)
+    assert np.isnan(got[:, :, ql - 2:]).all()
+    assert np.isposinf(got[:, :, 20:ql - 2, 3]).all()
+    v[0, :, 20, 3] = 0
+    keep = np.array([j for j in range(ql - 2) if j != 5])
+    exact, bound = attention_bound(q[:, :, 6:ql - 2], k[:, :, keep], v[:, :, keep], scale, 5,
+                                   ql - 3, "f32")
+    cols = [c for c in range(hd) if c != 3]
+    err = np.abs(got[:, :, 6:ql - 2] - exact)
+    assert np.all(err[..., cols] <= bound[..., cols])
