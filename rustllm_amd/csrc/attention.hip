@@ -88,19 +88,6 @@ __device__ inline float max3(float a, float b, float c) {
     return r;
 }
 
-// Chunk order of the unpadded LDS rows the DMA-fed kernel uses: 16-byte
-// chunk c of row r sits at chunk c ^ lds_swizzle(r) of that row.  The MFMA
-// operand reads of K (16 rows x one chunk per 16 lanes) and the transpose
-// reads of V (4 rows x 4 chunks per 32 lanes) then each fall on 64 distinct
-// banks (64 banks of 4 bytes; a row is D / 8 chunks).
-template <int NT>
-__device__ inline uint32_t lds_swizzle(uint32_t r) {
-    if constexpr (NT == 1) return (r >> 2) & 3u;
-    else if constexpr (NT == 2) return ((r & 2u) << 1) | ((r >> 2) & 3u);
-    else if constexpr (NT == 4 || NT == 8) return ((r & 3u) << 2) | ((r >> 2) & 3u);
-    else return 0u;
-}
-
 // Buffer resource (gfx9 descriptor: base, stride 0, size in bytes, 32-bit
 // data format) for raw loads from `base`: a load at or past `bytes` returns
 // zeros.

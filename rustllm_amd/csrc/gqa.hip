@@ -6,8 +6,8 @@
 // score rounded once.  gqa_pv_matmul (:72-110, metal :323-629):
 // out[b, h, i, d] = sum_j p[b, h, i, j] * v[b, h / g, j, d].
 //
-// In f16 both are bound by HBM (the [B, QH, Q, K] scores are written once
-// or read once; Q, K and V are small), in f32 by the f32 matrix cores.  A
+// Both are bound by HBM in f16 (the [B, QH, Q, K] scores are written once
+// or read once; Q, K and V are small), in f32 by the splitting too.  A
 // head size of 32..128 in steps of 32 takes the matrix cores
 // (v_mfma_f32_32x32x16_f16 for f16):
 //  * QK^T computes S^T = K Q^T per wave (32 queries x 128 keys; a
@@ -25,7 +25,7 @@
 //    Rows on the line grid are walked from a step that differs per
 //    workgroup (walk_step), so that the workgroups do not all read one
 //    column range at once.
-// f32 takes v_mfma_f32_32x32x2_f32 with the same workgroups (the f32
+// f32 takes the bf16 matrix cores, each operand as three bf16 parts (the f32
 // kernels below); other head sizes take row kernels on the vector ALUs.
 #include "common.hpp"
 #include "mfma_layout.hpp"
@@ -388,28 +388,48 @@ __global__ __launch_bounds__(256) void k_gqa_pv_mfma(const half_t* __restrict__ 
     }
 }
 
-// ----------------------------------------------------- f32, matrix cores
+// ------------------------------------ f32 on the bf16 matrix cores
 
-// QK^T in f32 (v_mfma_f32_32x32x2_f32, exact f32 products; bound by the
-// f32 matrix cores): workgroup = (head, 128 queries, run of k_per_block
-// 128-key tiles), wave = 32 queries.  The queries stay in registers for the
-// whole run; key tiles pass through registers into one of two LDS buffers
-// (tile t + 1 loads while tile t is multiplied), in key order at a stride of
-// 2 mod 64 floats (every operand read on its own bank).  Each lane stores
-// its result registers directly, four consecutive keys per 16-byte store: a
-// row receives 32-byte pieces that the L2 merges into whole lines.  VEC:
-// score rows on the 16-byte grid (kv_len % 4 == 0); otherwise the stores
-// are unaligned 16-byte stores, a row's last partial group element-wise.
-template <int NT, bool VEC>
-__global__ __launch_bounds__(256) void k_gqa_qk_mfma_f32(const float* __restrict__ q,
-                                                         const float* __restrict__ k,
-                                                         float* __restrict__ out, GqaParams p) {
+// Whether the parts of a value (Bf16x3) keep all its bits in any product
+// here: zero, or 2^-40 <= |x| < 2^60 (no part is subnormal, no sum of 2^16
+// products overflows).  `lo` and `hi` gather the least non-zero and the
+// largest magnitude; infinities and NaN are past any bound.
+struct Magnitudes {
+    uint32_t lo = 0xffffffffu, hi = 0u;
+    __device__ inline void add(float x) {
+        const uint32_t b = __float_as_uint(x);
+        lo = min(lo, (b << 1) - 1u);  // zero wraps to the largest
+        hi = max(hi, b & 0x7fffffffu);
+    }
+    __device__ inline bool in_range() const {
+        return lo >= (0x2b800000u << 1) - 1u && hi < 0x5d800000u;  // 2^-40, 2^60
+    }
+};
+
+// QK^T in f32: S = Q K^T per wave (32 queries, 32 keys at a time) with every
+// f32 product made of bf16 parts (v_mfma_f32_32x32x16_bf16).  Workgroup =
+// (head, 128 queries, run of k_per_block tiles of BN keys): the queries are
+// split once into registers; a key tile passes through registers and is split
+// into LDS for the four waves (three planes, rows in the chunk order of
+// lds_swizzle) while the next one loads.  With lane = key, register =
+// query a store writes two whole 128-byte row segments, at any row alignment.
+// Bound by the writes of the scores.  A tile with elements outside
+// Magnitudes::in_range is computed by plain dot products.  One MI355X, 9 heads
+// of 64 x [2048, 2048] (151 MB): 70.6 us on v_mfma_f32_32x32x2_f32
+// (whose rate bound it; 16-byte stores of 32 rows at a time), 51.3 us.
+template <int NT, int BN>
+__global__ __launch_bounds__(256) void k_gqa_qk_bf16x3(const float* __restrict__ q,
+                                                       const float* __restrict__ k,
+                                                       float* __restrict__ out, GqaParams p) {
     constexpr int D = 32 * NT;
-    constexpr int DS = D / 2;  // MFMA steps over the head
-    constexpr int KS = f32_stride(D, 2);
-    constexpr int ROW_CHUNKS = D / 4;
-    constexpr int LOADS = 128 * ROW_CHUNKS / 256;  // 16-byte pieces of a key tile per thread
-    __shared__ __align__(16) float ks[2][128 * KS];
+    constexpr int DC = D / 16;             // 16-wide slices of a head
+    constexpr int RD = NT == 3 ? 128 : D;  // elements of an LDS row
+    constexpr int SW = RD / 32;            // its chunk order
+    constexpr int ROW_CHUNKS = RD / 8;
+    constexpr int LOADS = BN * ROW_CHUNKS / 256;
+    constexpr int PLANE = BN * RD;
+    __shared__ __align__(16) __bf16 ks[3 * PLANE];
+    __shared__ uint32_t odd_tile;  // the last tile with a key out of range, + 1
     const uint32_t wave = threadIdx.x / 64;
     const uint32_t lane = threadIdx.x % 64;
     const uint32_t col = lane % 32;
@@ -424,113 +444,166 @@ __global__ __launch_bounds__(256) void k_gqa_qk_mfma_f32(const float* __restrict
     const uint32_t t_end = min(p.k_tiles, t_first + p.k_per_block);
 
     // keys past kv_len read row kv_len - 1 (their scores are not stored)
-    float4 kreg[LOADS];
+    f32x8 kreg[LOADS];
     auto load_tile = [&](uint32_t t) {
 #pragma unroll
         for (int li = 0; li < LOADS; ++li) {
             const uint32_t chunk = threadIdx.x + 256 * li;
-            const uint32_t key = min(t * 128 + chunk / ROW_CHUNKS, p.kv_len - 1);
-            kreg[li] = *reinterpret_cast<const float4*>(kh + uint64_t(key) * D +
-                                                        (chunk % ROW_CHUNKS) * 4);
+            const uint32_t ch = chunk % ROW_CHUNKS;
+            if (RD > D && ch >= D / 8) continue;  // head size 96: 12 of 16 chunks
+            const uint32_t key = min(t * BN + chunk / ROW_CHUNKS, p.kv_len - 1);
+            const float* src = kh + uint64_t(key) * D + ch * 8;
+            const f32x4 x0 = *reinterpret_cast<const f32x4*>(src);
+            const f32x4 x1 = *reinterpret_cast<const f32x4*>(src + 4);
+            kreg[li] = __builtin_shufflevector(x0, x1, 0, 1, 2, 3, 4, 5, 6, 7);
         }
     };
-    auto store_tile = [&](float* dst) {
+    auto store_tile = [&](uint32_t t) {
+        Magnitudes mag;
 #pragma unroll
         for (int li = 0; li < LOADS; ++li) {
             const uint32_t chunk = threadIdx.x + 256 * li;
-            float* row = dst + (chunk / ROW_CHUNKS) * KS + (chunk % ROW_CHUNKS) * 4;  // 8-byte aligned
-            *reinterpret_cast<float2*>(row) = float2{kreg[li].x, kreg[li].y};
-            *reinterpret_cast<float2*>(row + 2) = float2{kreg[li].z, kreg[li].w};
-        }
-    };
-    load_tile(t_first);
-    // B operand: lane (col, hs) holds elements 2j + hs of its query
-    const uint32_t qi = q0 + col;
-    const bool q_valid = qi < p.q_len;
-    const float* qrow = q + (uint64_t(bh) * p.q_len + (q_valid ? qi : 0)) * D + hs;
-    float qf[DS];
+            const uint32_t r = chunk / ROW_CHUNKS, ch = chunk % ROW_CHUNKS;
+            if (RD > D && ch >= D / 8) continue;
 #pragma unroll
-    for (int j = 0; j < DS; ++j) qf[j] = q_valid ? qrow[2 * j] : 0.0f;
-    store_tile(ks[0]);
+            for (int e = 0; e < 8; ++e) mag.add(kreg[li][e]);
+            const Bf16x3 x = split_bf16(kreg[li]);
+#pragma unroll
+            for (int i = 0; i < 3; ++i)
+                *reinterpret_cast<b8*>(ks + i * PLANE + r * RD + 8 * (ch ^ lds_swizzle<SW>(r))) =
+                    x.part[i];
+        }
+        if (!mag.in_range()) odd_tile = t + 1;
+    };
+    if (threadIdx.x == 0) odd_tile = 0;
+    load_tile(t_first);
+    // A operand: lane (row col, hs) holds elements 16c + 8hs .. + 7 of its query
+    const uint32_t qi = q0 + col;
+    const float* qrow = q + (uint64_t(bh) * p.q_len + (qi < p.q_len ? qi : 0)) * D + 8 * hs;
+    Magnitudes qmag;
+    Bf16x3 qf[DC];
+#pragma unroll
+    for (int c = 0; c < DC; ++c) {
+        const f32x4 x0 = *reinterpret_cast<const f32x4*>(qrow + 16 * c);
+        const f32x4 x1 = *reinterpret_cast<const f32x4*>(qrow + 16 * c + 4);
+        const f32x8 x = __builtin_shufflevector(x0, x1, 0, 1, 2, 3, 4, 5, 6, 7);
+#pragma unroll
+        for (int e = 0; e < 8; ++e) qmag.add(x[e]);
+        qf[c] = split_bf16(x);
+    }
+    const bool odd_queries = __any(!qmag.in_range());
+    uint32_t koff[DC];
+#pragma unroll
+    for (int c = 0; c < DC; ++c) koff[c] = col * RD + 8 * ((2 * c + hs) ^ lds_swizzle<SW>(col));
+    __syncthreads();  // odd_tile is set up
+    store_tile(t_first);
     __syncthreads();
 
-    float* orow = out + (uint64_t(bh) * p.q_len + (q_valid ? qi : 0)) * p.kv_len;
+    float* tile_out = out + (uint64_t(bh) * p.q_len + q0 + 4 * hs) * p.kv_len;
+    const uint32_t rows = q0 < p.q_len ? min(32u, p.q_len - q0) : 0u;
     for (uint32_t t = t_first; t < t_end; ++t) {
-        const uint32_t buf = (t - t_first) % 2;
         if (t + 1 < t_end) load_tile(t + 1);
-        if (q0 < p.q_len) {
+        if (rows > 0) {
+            const bool plain = odd_queries || odd_tile == t + 1;
 #pragma unroll
-            for (int st = 0; st < 4; ++st) {  // four 32-key sub-tiles
-                const uint32_t k0 = t * 128 + st * 32;
-                const float* krow = ks[buf] + (st * 32 + col) * KS + hs;
+            for (int st = 0; st < BN / 32; ++st) {
+                const uint32_t key = t * BN + st * 32 + col;
                 f32x16 s;
 #pragma unroll
                 for (int r = 0; r < 16; ++r) s[r] = 0.0f;
+                if (!plain) {
 #pragma unroll
-                for (int j = 0; j < DS; ++j)
-                    s = __builtin_amdgcn_mfma_f32_32x32x2f32(krow[2 * j], qf[j], s, 0, 0, 0);
-                if (!q_valid) continue;
-                // register 4g + e holds key k0 + 8g + 4hs + e; rows of
-                // kv_len % 4 != 0 scores start off the 16-byte grid and take
-                // unaligned 16-byte stores
+                    for (int c = 0; c < DC; ++c) {
+                        Bf16x3 kb;
 #pragma unroll
-                for (int g = 0; g < 4; ++g) {
-                    const uint32_t key = k0 + 8 * g + 4 * hs;
-                    const f32x4 w = {s[4 * g], s[4 * g + 1], s[4 * g + 2], s[4 * g + 3]};
-                    if constexpr (VEC) {  // kv_len % 4 == 0: a group is whole or past the end
-                        if (key < p.kv_len) *reinterpret_cast<f32x4*>(orow + key) = w;
-                    } else if (key + 4 <= p.kv_len) {
-                        *reinterpret_cast<f32x4u*>(orow + key) = w;
-                    } else {
+                        for (int i = 0; i < 3; ++i)
+                            kb.part[i] = *reinterpret_cast<const b8*>(ks + i * PLANE +
+                                                                      st * 32 * RD + koff[c]);
+                        s = mfma_bf16x3(qf[c], kb, s);
+                    }
+                } else {
+                    const float* krow = kh + uint64_t(min(key, p.kv_len - 1)) * D;
+                    for (int d = 0; d < D; ++d) {
+                        const float kd = krow[d];
 #pragma unroll
-                        for (int e = 0; e < 4; ++e)
-                            if (key + e < p.kv_len) orow[key + e] = s[4 * g + e];
+                        for (int r = 0; r < 16; ++r) {
+                            const uint32_t row = min(8u * (r / 4) + 4 * hs + r % 4, rows - 1);
+                            s[r] = __builtin_fmaf(
+                                q[(uint64_t(bh) * p.q_len + q0 + row) * D + d], kd, s[r]);
+                        }
+                    }
+                }
+                // register r: query row 8 (r / 4) + 4 hs + r % 4 of the tile
+                if (key < p.kv_len) {
+#pragma unroll
+                    for (int r = 0; r < 16; ++r) {
+                        const uint32_t row = 8 * (r / 4) + r % 4;
+                        if (rows == 32 || row + 4 * hs < rows)
+                            tile_out[uint64_t(row) * p.kv_len + key] = s[r];
                     }
                 }
             }
         }
-        if (t + 1 < t_end) store_tile(ks[buf ^ 1]);  // read during step t - 1, before its barrier
+        __syncthreads();
+        if (t + 1 < t_end) store_tile(t + 1);
         __syncthreads();
     }
 }
 
-// P V in f32: workgroup = (head, 128 queries), keys in steps of 64.  Each
-// wave stages its 32 x 64 probabilities in LDS (whole 256-byte row segments
-// per 16 lanes) at a row stride of 2 mod 64, so that lane (col, hs) reads the
-// probability of key 2s + hs of its query -- the B operand of the step over
-// keys 2s, 2s + 1 -- on its own bank; V rows at 32 mod 64 floats.  The next
-// step's operands are in flight during this step's products.  VEC:
-// probability rows on the 16-byte grid (streamed loads); otherwise plain
-// unaligned 16-byte loads, a row's last partial group element-wise.
-template <int NT, bool VEC>
-__global__ __launch_bounds__(256) void k_gqa_pv_mfma_f32(const float* __restrict__ probs,
-                                                         const float* __restrict__ v,
-                                                         float* __restrict__ out, GqaParams p) {
+// P V in f32: O^T = V^T P^T per wave (32 queries), products of bf16 parts.
+// Workgroup = (head, 32 QW queries), KS shares of the key steps (BN keys each,
+// share g takes steps g, g + KS, ..) merged through LDS at the end.  Each wave
+// stages its 32 x BN probabilities in LDS (whole row segments per load) and
+// splits its lane's 8 consecutive keys; V blocks are split into LDS as three
+// planes for the QW waves of a share.  The next step's operands are in flight
+// during this step's products.  Bound by the reads of the probabilities.
+// Outputs that are not finite or below 2^-36, and all of a wave's that met a
+// probability or value of 2^60 or more, are computed by plain dot products.
+// VEC: probability rows on the 16-byte grid (streamed loads); otherwise
+// plain unaligned 16-byte loads, a row's last partial group element-wise.
+// One MI355X, 9 heads of 64 x [2048, 2048]: 95.2 us on the f32 matrix
+// cores, 128 queries a workgroup, 66.8 us.
+template <int NT, int QW, int KS, int BN, bool VEC>
+__global__ __launch_bounds__(64 * QW * KS) void k_gqa_pv_bf16x3(const float* __restrict__ probs,
+                                                                const float* __restrict__ v,
+                                                                float* __restrict__ out,
+                                                                GqaParams p) {
     constexpr int D = 32 * NT;
-    constexpr int BN = 64;                      // keys per step
-    constexpr int VS = f32_stride(D, 32);       // LDS row stride of V
-    constexpr int PS = f32_stride(BN, 2);       // LDS row stride of a wave's probabilities
-    constexpr int ROW_CHUNKS = D / 4;
-    constexpr int LOADS = BN * ROW_CHUNKS / 256;
-    __shared__ __align__(16) float vs[BN * VS];
-    __shared__ __align__(16) float pt[4][32 * PS];
+    constexpr int RD = NT == 3 ? 128 : D;
+    constexpr int SW = RD / 32;
+    constexpr int ROW_CHUNKS = RD / 8;
+    constexpr int THREADS = 64 * QW * KS;
+    constexpr int BLOCK_CHUNKS = BN * ROW_CHUNKS;
+    constexpr int LOADS = BLOCK_CHUNKS * KS / THREADS;
+    constexpr int PLANE = BN * RD;
+    constexpr int PS = BN + 4;              // LDS row stride of a wave's probabilities
+    constexpr int P_LOADS = 32 * BN / 256;  // 16-byte pieces per lane
+    constexpr int P_ROWS = 256 / BN;        // rows per load instruction
+    constexpr int V_BYTES = KS * 3 * PLANE * 2;
+    constexpr int P_BYTES = QW * KS * 32 * PS * 4;
+    constexpr int MERGE_BYTES = (KS - 1) * QW * 64 * NT * 16 * 4;
+    constexpr int LDS_BYTES = V_BYTES + P_BYTES > MERGE_BYTES ? V_BYTES + P_BYTES : MERGE_BYTES;
+    static_assert((BLOCK_CHUNKS * KS) % THREADS == 0, "blocks must split evenly");
+    __shared__ __align__(16) unsigned char lds[LDS_BYTES];
+    __bf16* const vs = reinterpret_cast<__bf16*>(lds);
     const uint32_t wave = threadIdx.x / 64;
+    const uint32_t qw = wave % QW, sub = wave / QW;
     const uint32_t lane = threadIdx.x % 64;
     const uint32_t col = lane % 32;
     const uint32_t hs = lane / 32;
+    float* const my = reinterpret_cast<float*>(lds + V_BYTES) + wave * 32 * PS;
     const uint32_t qt = blockIdx.x % p.q_tiles;
     const uint32_t bh = blockIdx.x / p.q_tiles;
-    const uint32_t q0 = qt * 128 + wave * 32;
+    const uint32_t q0 = (qt * QW + qw) * 32;
     const float* vh = v + uint64_t(kv_head_of(bh, p)) * p.kv_head_stride;
     const float* pbase = probs + uint64_t(bh) * p.q_len * p.kv_len;
-    float* my = pt[wave];
 
     // rows past q_len and keys past kv_len as zeros
-    auto load_p = [&](uint32_t blk, f32x4 (&pr)[8]) {
+    auto load_p = [&](uint32_t blk, f32x4 (&pr)[P_LOADS]) {
 #pragma unroll
-        for (int i = 0; i < 8; ++i) {
-            const uint32_t r = i * 4 + lane / 16;
-            const uint32_t kb = blk * BN + (lane % 16) * 4;
+        for (int i = 0; i < P_LOADS; ++i) {
+            const uint32_t r = i * P_ROWS + lane / (BN / 4);
+            const uint32_t kb = blk * BN + (lane % (BN / 4)) * 4;
             const float* src = pbase + uint64_t(q0 + r) * p.kv_len + kb;
             if constexpr (VEC) {  // kv_len % 4 == 0: a group is whole or past the end
                 if (q0 + r < p.q_len && kb < p.kv_len)
@@ -548,33 +621,57 @@ __global__ __launch_bounds__(256) void k_gqa_pv_mfma_f32(const float* __restrict
             }
         }
     };
-    auto store_p = [&](const f32x4 (&pr)[8]) {
+    auto store_p = [&](const f32x4 (&pr)[P_LOADS]) {
 #pragma unroll
-        for (int i = 0; i < 8; ++i) {
-            float* dst = my + (i * 4 + lane / 16) * PS + (lane % 16) * 4;  // 8-byte aligned
-            *reinterpret_cast<float2*>(dst) = float2{pr[i][0], pr[i][1]};
-            *reinterpret_cast<float2*>(dst + 2) = float2{pr[i][2], pr[i][3]};
-        }
+        for (int i = 0; i < P_LOADS; ++i)
+            *reinterpret_cast<f32x4*>(my + (i * P_ROWS + lane / (BN / 4)) * PS +
+                                      (lane % (BN / 4)) * 4) = pr[i];
     };
-    auto load_v = [&](uint32_t blk, float4 (&vr)[LOADS]) {
+    auto load_v = [&](uint32_t step, f32x8 (&vr)[LOADS]) {
 #pragma unroll
         for (int li = 0; li < LOADS; ++li) {
-            const uint32_t chunk = threadIdx.x + 256 * li;
-            const uint32_t gk = blk * BN + chunk / ROW_CHUNKS;
-            const uint32_t d0 = (chunk % ROW_CHUNKS) * 4;
-            vr[li] = gk < p.kv_len
-                         ? *reinterpret_cast<const float4*>(vh + uint64_t(gk) * D + d0)
-                         : float4{0.0f, 0.0f, 0.0f, 0.0f};
+            const uint32_t chunk = threadIdx.x + THREADS * li;
+            const uint32_t c = chunk % BLOCK_CHUNKS;
+            const uint32_t gk = (step * KS + chunk / BLOCK_CHUNKS) * BN + c / ROW_CHUNKS;
+            const uint32_t ch = c % ROW_CHUNKS;
+            if (RD > D && ch >= D / 8) continue;
+            f32x4 x0 = {0.0f, 0.0f, 0.0f, 0.0f}, x1 = x0;
+            if (gk < p.kv_len) {
+                const float* src = vh + uint64_t(gk) * D + ch * 8;
+                x0 = *reinterpret_cast<const f32x4*>(src);
+                x1 = *reinterpret_cast<const f32x4*>(src + 4);
+            }
+            vr[li] = __builtin_shufflevector(x0, x1, 0, 1, 2, 3, 4, 5, 6, 7);
         }
     };
-    auto store_v = [&](const float4 (&vr)[LOADS]) {
+    float vmax = 0.0f, pmax = 0.0f;  // the largest magnitudes this thread split
+    auto store_v = [&](const f32x8 (&vr)[LOADS]) {
 #pragma unroll
         for (int li = 0; li < LOADS; ++li) {
-            const uint32_t chunk = threadIdx.x + 256 * li;
-            *reinterpret_cast<float4*>(vs + (chunk / ROW_CHUNKS) * VS + (chunk % ROW_CHUNKS) * 4) =
-                vr[li];
+            const uint32_t chunk = threadIdx.x + THREADS * li;
+            const uint32_t c = chunk % BLOCK_CHUNKS;
+            const uint32_t r = c / ROW_CHUNKS, ch = c % ROW_CHUNKS;
+            if (RD > D && ch >= D / 8) continue;
+#pragma unroll
+            for (int e = 0; e < 8; ++e) vmax = fmaxf(vmax, fabsf(vr[li][e]));
+            const Bf16x3 x = split_bf16(vr[li]);
+            __bf16* dst = vs + (chunk / BLOCK_CHUNKS) * 3 * PLANE + r * RD +
+                          8 * (ch ^ lds_swizzle<SW>(r));
+#pragma unroll
+            for (int i = 0; i < 3; ++i) *reinterpret_cast<b8*>(dst + i * PLANE) = x.part[i];
         }
     };
+    // transpose reads of V for the A operand, as in k_flash_attention
+    uint32_t voff[2][NT];
+#pragma unroll
+    for (int e2 = 0; e2 < 2; ++e2) {
+        const uint32_t row = 8 * (lane / 32) + (lane % 16) / 4 + 4 * e2;
+#pragma unroll
+        for (int t = 0; t < NT; ++t) {
+            const uint32_t ch = 2 * ((lane / 16) % 2) + (lane % 4) / 2 + 4 * t;
+            voff[e2][t] = row * RD + 8 * (ch ^ lds_swizzle<SW>(row)) + 4 * (lane % 2);
+        }
+    }
 
     f32x16 o[NT];
 #pragma unroll
@@ -583,46 +680,103 @@ __global__ __launch_bounds__(256) void k_gqa_pv_mfma_f32(const float* __restrict
         for (int r = 0; r < 16; ++r) o[t][r] = 0.0f;
 
     const uint32_t blocks = (p.kv_len + BN - 1) / BN;
-    f32x4 pnext[8];
-    float4 vnext[LOADS];
-    load_p(0, pnext);
+    const uint32_t steps = (blocks + KS - 1) / KS;
+    f32x4 pnext[P_LOADS];
+    f32x8 vnext[LOADS];
+    load_p(sub, pnext);
     load_v(0, vnext);
     store_p(pnext);
     store_v(vnext);
     __syncthreads();
-    for (uint32_t blk = 0; blk < blocks; ++blk) {
-        const bool more = blk + 1 < blocks;
+    for (uint32_t step = 0; step < steps; ++step) {
+        const bool more = step + 1 < steps;
         if (more) {
-            load_p(blk + 1, pnext);
-            load_v(blk + 1, vnext);
+            load_p((step + 1) * KS + sub, pnext);
+            load_v(step + 1, vnext);
         }
-        const float* prow = my + col * PS + hs;
-        const float* vcol = vs + hs * VS + col;
+        const __bf16* vsub = vs + sub * 3 * PLANE;
 #pragma unroll
-        for (int s = 0; s < BN / 2; ++s) {
-            const float pb = prow[2 * s];  // P of key 2s + hs
+        for (int c = 0; c < BN / 16; ++c) {
+            // P^T operand: keys 16 c + 8 hs + 0..7 of query row col
+            const float* prow = my + col * PS + 16 * c + 8 * hs;
+            const f32x4 x0 = *reinterpret_cast<const f32x4*>(prow);
+            const f32x4 x1 = *reinterpret_cast<const f32x4*>(prow + 4);
+            const f32x8 x = __builtin_shufflevector(x0, x1, 0, 1, 2, 3, 4, 5, 6, 7);
 #pragma unroll
-            for (int t = 0; t < NT; ++t)
-                o[t] = __builtin_amdgcn_mfma_f32_32x32x2f32(vcol[2 * s * VS + 32 * t], pb, o[t],
-                                                             0, 0, 0);
+            for (int e = 0; e < 8; ++e) pmax = fmaxf(pmax, fabsf(x[e]));
+            const Bf16x3 pb = split_bf16(x);
+#pragma unroll
+            for (int t = 0; t < NT; ++t) {
+                Bf16x3 va;
+#pragma unroll
+                for (int i = 0; i < 3; ++i) {
+                    const half_t* plane =
+                        reinterpret_cast<const half_t*>(vsub + i * PLANE + 16 * c * RD);
+                    const h4 lo = lds_read_transposed(plane + voff[0][t]);
+                    const h4 hi = lds_read_transposed(plane + voff[1][t]);
+                    const h8 w = {lo[0], lo[1], lo[2], lo[3], hi[0], hi[1], hi[2], hi[3]};
+                    va.part[i] = __builtin_bit_cast(b8, w);
+                }
+                o[t] = mfma_bf16x3(va, pb, o[t]);
+            }
         }
+        __syncthreads();
         if (more) {
-            __syncthreads();
             store_p(pnext);
             store_v(vnext);
-            __syncthreads();
+        }
+        __syncthreads();
+    }
+    // any value or probability past 2^60 anywhere in the workgroup
+    const bool huge = __syncthreads_or(!(vmax < 0x1p60f) || !(pmax < 0x1p60f));
+    if constexpr (KS > 1) {
+        float* mg = reinterpret_cast<float*>(lds);
+        if (sub > 0) {
+            float* dst = mg + ((sub - 1) * QW + qw) * 64 * NT * 16 + lane;
+#pragma unroll
+            for (int t = 0; t < NT; ++t)
+#pragma unroll
+                for (int r = 0; r < 16; ++r) dst[(16 * t + r) * 64] = o[t][r];
+        }
+        __syncthreads();
+        if (sub > 0) return;
+#pragma unroll
+        for (int h = 1; h < KS; ++h) {
+            const float* src = mg + ((h - 1) * QW + qw) * 64 * NT * 16 + lane;
+#pragma unroll
+            for (int t = 0; t < NT; ++t)
+#pragma unroll
+                for (int r = 0; r < 16; ++r) o[t][r] += src[(16 * t + r) * 64];
         }
     }
     const uint32_t qi = q0 + col;
     if (qi < p.q_len) {
         // register r of tile t: element 32t + 8(r / 4) + 4hs + r % 4
         float* orow = out + (uint64_t(bh) * p.q_len + qi) * D + 4 * hs;
+        bool odd = huge;
+#pragma unroll
+        for (int t = 0; t < NT; ++t)
+#pragma unroll
+            for (int r = 0; r < 16; ++r) {
+                const float a = fabsf(o[t][r]);
+                odd |= a != 0.0f && !(a > 0x1p-36f && a < INFINITY);
+            }
 #pragma unroll
         for (int t = 0; t < NT; ++t)
 #pragma unroll
             for (int g = 0; g < 4; ++g)
-                *reinterpret_cast<float4*>(orow + 32 * t + 8 * g) =
-                    float4{o[t][4 * g], o[t][4 * g + 1], o[t][4 * g + 2], o[t][4 * g + 3]};
+                *reinterpret_cast<f32x4*>(orow + 32 * t + 8 * g) =
+                    f32x4{o[t][4 * g], o[t][4 * g + 1], o[t][4 * g + 2], o[t][4 * g + 3]};
+        if (odd) {
+            const float* prow = pbase + uint64_t(qi) * p.kv_len;
+            for (uint32_t i = 0; i < D / 2; ++i) {
+                const uint32_t d = 8 * (i / 4) + i % 4;  // + 4 hs: this lane's elements
+                float sum = 0.0f;
+                for (uint32_t key = 0; key < p.kv_len; ++key)
+                    sum = __builtin_fmaf(prow[key], vh[uint64_t(key) * D + 4 * hs + d], sum);
+                orow[d] = sum;
+            }
+        }
     }
 }
 
@@ -750,6 +904,10 @@ bool use_mfma(const GqaShape& s, const void* a, const void* b, const void* o) {
            aligned_to(o, 16);
 }
 
+// f32 QK^T workgroups in one round: two a CU (9 heads of 64 x [2048, 2048]: 51.3
+// us; runs of tiles for 768 workgroups 53.3, 300 60.0).
+constexpr uint64_t kQkResident = 512;
+
 template <typename T>
 rl_status qk_entry(rl_context* ctx, const char* name, const rl_buffer* q, const rl_buffer* k,
                    const GqaShape& s, const rl_buffer* out) {
@@ -798,36 +956,27 @@ rl_status qk_entry(rl_context* ctx, const char* name, const rl_buffer* q, const 
         }
     } else {
         if (use_mfma<T>(s, qd, kd, od)) {
+            // key tiles of 128, or 64 for head sizes 96 and 128 (48 KB of LDS)
+            const uint64_t bn = s.head_dim <= 64 ? 128 : 64;
             p.q_tiles = uint32_t(ceil_div(s.q_len, 128));
-            p.k_tiles = uint32_t(ceil_div(s.kv_len, 128));
+            p.k_tiles = uint32_t(ceil_div(s.kv_len, bn));
             // Workgroups walk runs of key tiles; a query tile's keys split
             // over several only when the query tiles alone do not fill the
-            // resident workgroups (two per CU up to head size 64, one above).
+            // resident workgroups.
             const uint64_t base = heads * p.q_tiles;
-            const uint64_t resident = s.head_dim <= 64 ? 512 : 256;
             const uint64_t groups =
-                std::min<uint64_t>(p.k_tiles, std::max<uint64_t>(1, resident / base));
+                std::min<uint64_t>(p.k_tiles, std::max<uint64_t>(1, kQkResident / base));
             p.k_per_block = uint32_t(ceil_div(p.k_tiles, groups));
             p.k_groups = uint32_t(ceil_div(p.k_tiles, p.k_per_block));
             const uint64_t grid = base * p.k_groups;
             if (grid > UINT32_MAX) return fail(RL_ERR_INVALID_SHAPE, "GQA QK grid exceeds u32");
             const dim3 g(static_cast<unsigned>(grid)), b(256);
-            // score rows on the 16-byte grid (kv_len % 4 == 0) or off it
-            const bool vec = s.kv_len % 4 == 0;
-#define RL_QK32(NT)                                                                    \
-    do {                                                                               \
-        if (vec)                                                                       \
-            RL_LAUNCH(ctx, (k_gqa_qk_mfma_f32<NT, true>), g, b, qd, kd, od, p);        \
-        else                                                                           \
-            RL_LAUNCH(ctx, (k_gqa_qk_mfma_f32<NT, false>), g, b, qd, kd, od, p);       \
-    } while (0)
             switch (s.head_dim / 32) {
-                case 1: RL_QK32(1); break;
-                case 2: RL_QK32(2); break;
-                case 3: RL_QK32(3); break;
-                default: RL_QK32(4); break;
+                case 1: RL_LAUNCH(ctx, (k_gqa_qk_bf16x3<1, 128>), g, b, qd, kd, od, p); break;
+                case 2: RL_LAUNCH(ctx, (k_gqa_qk_bf16x3<2, 128>), g, b, qd, kd, od, p); break;
+                case 3: RL_LAUNCH(ctx, (k_gqa_qk_bf16x3<3, 64>), g, b, qd, kd, od, p); break;
+                default: RL_LAUNCH(ctx, (k_gqa_qk_bf16x3<4, 64>), g, b, qd, kd, od, p); break;
             }
-#undef RL_QK32
             return after_launch(ctx, name);
         }
     }
@@ -906,18 +1055,22 @@ rl_status pv_entry(rl_context* ctx, const char* name, const rl_buffer* probs, co
         }
     } else {
         if (use_mfma<T>(s, pd, vd, od)) {
-            p.q_tiles = uint32_t(ceil_div(s.q_len, 128));
+            // 64-query workgroups of two key shares, three a CU (9 heads of 64
+            // x [2048, 2048]: 66.8 us; four shares, one a CU, 80.7; 128 queries
+            // 64.3, but 92.4 against 77.8 at 2047 keys and 82.1 against 63.7 for
+            // 8 heads of 128 x [1500, 1500]; 32 queries 77.9)
+            p.q_tiles = uint32_t(ceil_div(s.q_len, 64));
             const uint64_t grid = heads * p.q_tiles;
             if (grid > UINT32_MAX) return fail(RL_ERR_INVALID_SHAPE, "GQA PV grid exceeds u32");
-            const dim3 g(static_cast<unsigned>(grid)), b(256);
+            const dim3 g(static_cast<unsigned>(grid));
             // probability rows on the 16-byte grid (kv_len % 4 == 0) or off it
             const bool vec = s.kv_len % 4 == 0;
-#define RL_PV32(NT)                                                                    \
-    do {                                                                               \
-        if (vec)                                                                       \
-            RL_LAUNCH(ctx, (k_gqa_pv_mfma_f32<NT, true>), g, b, pd, vd, od, p);        \
-        else                                                                           \
-            RL_LAUNCH(ctx, (k_gqa_pv_mfma_f32<NT, false>), g, b, pd, vd, od, p);       \
+#define RL_PV32(NT)                                                                           \
+    do {                                                                                      \
+        if (vec)                                                                              \
+            RL_LAUNCH(ctx, (k_gqa_pv_bf16x3<NT, 2, 2, 32, true>), g, dim3(256), pd, vd, od, p);  \
+        else                                                                                  \
+            RL_LAUNCH(ctx, (k_gqa_pv_bf16x3<NT, 2, 2, 32, false>), g, dim3(256), pd, vd, od, p); \
     } while (0)
             switch (s.head_dim / 32) {
                 case 1: RL_PV32(1); break;

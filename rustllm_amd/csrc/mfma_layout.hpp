@@ -1,7 +1,7 @@
 // mfma_layout.hpp -- operand layouts shared by the matrix-core kernels of
 // attention.hip and gqa.hip (gfx950, wave64).
 //
-// v_mfma_f32_32x32x16_f16 and v_mfma_f32_32x32x2_f32 take A / B operands
+// v_mfma_f32_32x32x16_f16 and _bf16 take A / B operands
 // with lane l holding row (A) or column (B) l % 32 and the inner-dimension
 // slice l / 32; the 32 x 32 result leaves lane l with column l % 32 and, in
 // register r, row 8 (r / 4) + 4 (l / 32) + r % 4.  The key orders below
@@ -40,14 +40,17 @@ __host__ __device__ constexpr int v_stride_tr(int d) {
     return s;
 }
 
-// Row strides (floats) of f32 tiles in LDS.  An operand read that takes one
-// element of 32 rows (lanes 0-31) and the next element of the same rows
-// (lanes 32-63) hits 64 banks at a stride of 2 mod 64; one that takes 32
-// consecutive elements of two adjacent rows does at 32 mod 64.
-__host__ __device__ constexpr int f32_stride(int d, int residue) {
-    int s = d;
-    while (s % 64 != residue) ++s;
-    return s;
+// Chunk order of the unpadded LDS rows the attention and f32 kernels use: 16-byte
+// chunk c of row r sits at chunk c ^ lds_swizzle(r) of that row.  The MFMA
+// operand reads of K (16 rows x one chunk per 16 lanes) and the transpose
+// reads of V (4 rows x 4 chunks per 32 lanes) then each fall on 64 distinct
+// banks (64 banks of 4 bytes; a row is D / 8 chunks).
+template <int NT>
+__device__ inline uint32_t lds_swizzle(uint32_t r) {
+    if constexpr (NT == 1) return (r >> 2) & 3u;
+    else if constexpr (NT == 2) return ((r & 2u) << 1) | ((r >> 2) & 3u);
+    else if constexpr (NT == 4 || NT == 8) return ((r & 3u) << 2) | ((r >> 2) & 3u);
+    else return 0u;
 }
 
 // ds_read_b64_tr_b16: in each group of 16 lanes, lanes 4j .. 4j + 3 read 8

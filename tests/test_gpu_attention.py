@@ -520,3 +520,42 @@ def test_attention_f32_extremes(ctx, hd, heads, ql):
     cols = [c for c in range(hd) if c != 3]
     err = np.abs(got[:, :, 6:ql - 2] - exact)
     assert np.all(err[..., cols] <= bound[..., cols])
+
+
+@pytest.mark.parametrize("hd,ql,kl", [(64, 130, 131), (128, 70, 200), (96, 33, 65), (32, 129, 260)])
+def test_gqa_f32_extremes(ctx, hd, ql, kl):
+    """f32 operands as bf16 parts: magnitudes whose parts would be subnormal or
+    overflow, exact zeros, infinities and NaN come out as f32 products do."""
+    q = synth.normal(61, (1, 4, ql, hd))
+    k = synth.normal(62, (1, 2, kl, hd))
+    p = np.abs(synth.normal(63, (1, 4, ql, kl)))
+    v = synth.normal(64, (1, 2, kl, hd))
+    q[:, :, 3], k[:, :, 5], p[:, :, 4], v[:, :, 6] = 0, 0, 0, 0
+    for a, b in ((2.0 ** -118, 2.0 ** 90), (2.0 ** 100, 2.0 ** -100), (2.0 ** -50, 2.0 ** -50)):
+        x = [(m * np.float32(f)).astype(np.float32) for m, f in ((q, a), (k, b), (p, a), (v, b))]
+        ctx.begin()
+        s = ctx.gqa_qk(ctx.upload(x[0]), ctx.upload(x[1]))
+        o_ = ctx.gqa_pv(ctx.upload(x[2]), ctx.upload(x[3]))
+        ctx.finish()
+        exact, mag = gqa_exact(x[0].astype(np.float64) / a, x[1].astype(np.float64) / b, kl)
+        assert np.all(np.abs(s.numpy().astype(np.float64) / a / b - exact) <= (hd + 2) * U32 * mag)
+        ve = np.repeat(x[3].astype(np.float64) / b, 2, 1)
+        pe = x[2].astype(np.float64) / a
+        err = np.abs(o_.numpy().astype(np.float64) / a / b - pe @ ve)
+        assert np.all(err <= (kl + 2) * U32 * (pe @ np.abs(ve)))
+    k[0, 0, 7, 1], k[0, 1, 9, 0] = np.inf, np.nan
+    v[0, 0, 2, 1], v[0, 1, 9, 0] = np.inf, np.nan
+    p[:, :, :, 2] += 0.5
+    ctx.begin()
+    s = ctx.gqa_qk(ctx.upload(q), ctx.upload(k)).numpy()
+    o_ = ctx.gqa_pv(ctx.upload(p), ctx.upload(v)).numpy()
+    ctx.finish()
+    with np.errstate(invalid="ignore"):
+        s_ref = np.matmul(q.astype(np.float64), np.swapaxes(np.repeat(k, 2, 1), -1, -2))
+        o_ref = np.matmul(p.astype(np.float64), np.repeat(v, 2, 1).astype(np.float64))
+    for got, ref in ((s, s_ref), (o_, o_ref)):
+        assert np.array_equal(np.isnan(got), np.isnan(ref))
+        inf = np.isinf(ref)
+        assert np.array_equal(got[inf], ref[inf].astype(np.float32))
+        ok = np.isfinite(ref)
+        assert np.allclose(got[ok], ref[ok], rtol=0, atol=1e-3)
