@@ -56,6 +56,7 @@ struct BufferPool {
 struct FusedOp {
     uint32_t kind = 0;
     uint32_t blocks = 0;
+    uint32_t block_elements = 0;  // maps, bias adds: elements of one block
     const void* a = nullptr;
     const void* b = nullptr;
     void* out = nullptr;

@@ -14,6 +14,7 @@
 #include "common.hpp"
 #include "movement_bodies.hpp"
 
+#include <algorithm>
 #include <type_traits>
 
 namespace rl {
@@ -184,8 +185,16 @@ constexpr int map_pack() {
 // out[i] = op(a[i], b[i]) for ARITY 2, op(a[i]) for ARITY 1.  Block blk covers
 // packs [blk * 256 * UNROLL, (blk + 1) * 256 * UNROLL): the grid spans the
 // whole array (at most 2^32 elements, so at most 2^22 blocks), with no loop.
+template <bool STREAM, typename V>
+__device__ inline V load_in(const V* p) {
+    if constexpr (STREAM)
+        return load_stream(p);
+    else
+        return *p;
+}
+
 template <typename TIn, typename TOut, int N, int UNROLL, int ARITY, bool NTS, bool PHASED,
-          typename Op>
+          typename Op, bool STREAM = true>
 __device__ inline void map_body(const TIn* __restrict__ a, const TIn* __restrict__ b,
                                 TOut* __restrict__ out, uint64_t n_packs, uint32_t tail, Op op,
                                 uint32_t blk) {
@@ -210,8 +219,8 @@ __device__ inline void map_body(const TIn* __restrict__ a, const TIn* __restrict
             for (int u = 0; u < UNROLL; ++u) {
                 const uint64_t i = base + uint64_t(u) * kThreads;
                 const uint64_t ic = i < n_packs ? i : n_packs - 1;
-                ra[u] = load_stream(va + ic);
-                if constexpr (ARITY == 2) rb[u] = load_stream(vb + ic);
+                ra[u] = load_in<STREAM>(va + ic);
+                if constexpr (ARITY == 2) rb[u] = load_in<STREAM>(vb + ic);
             }
 #pragma unroll
             for (int u = 0; u < UNROLL; ++u) {
@@ -239,8 +248,8 @@ __device__ inline void map_body(const TIn* __restrict__ a, const TIn* __restrict
         for (int u = 0; u < UNROLL; ++u) {
             const uint64_t i = base + uint64_t(u) * kThreads;
             if (i < n_packs) {
-                ra[u] = load_stream(va + i);
-                if constexpr (ARITY == 2) rb[u] = load_stream(vb + i);
+                ra[u] = load_in<STREAM>(va + i);
+                if constexpr (ARITY == 2) rb[u] = load_in<STREAM>(vb + i);
             }
         }
 #pragma unroll
@@ -282,7 +291,7 @@ __global__ __launch_bounds__(kThreads) void k_map(const TIn* __restrict__ a,
 
 // out[r, c] = x[r, c] + bias[c] on packs; col_packs = cols / N.  Block blk
 // of nblk strides over the packs.
-template <typename T, int N, int UNROLL>
+template <typename T, int N, int UNROLL, bool STREAM = true>
 __device__ inline void broadcast_body(const T* __restrict__ x, const T* __restrict__ bias,
                                       T* __restrict__ out, uint64_t n_packs, FastDiv col_packs,
                                       uint32_t blk, uint32_t nblk) {
@@ -300,7 +309,7 @@ __device__ inline void broadcast_body(const T* __restrict__ x, const T* __restri
             if (i < n_packs) {
                 uint32_t row, col;
                 col_packs.divmod(uint32_t(i), row, col);
-                rx[u] = load_stream(vx + i);
+                rx[u] = load_in<STREAM>(vx + i);
                 rb[u] = vbias[col];  // a few KiB, stays in L2
             }
         }
@@ -406,11 +415,39 @@ struct FusedSeg {
     uint32_t small_index;
     FusedDims outer;      // row gather / scatter
 };
+
+// Ops that read the same input walk it together: a group's grid is cut into
+// slots (slot_elements), and the blocks of all its ops for one slot are
+// neighbours on one XCD (hardware block b runs on XCD b mod 8), op by op, so
+// that the input is fetched once and found in that XCD's L2 by the others
+// (plain loads: streamed ones do not stay there).  The [4096, 1536] f16 batch
+// add, mul, SiLU, SwiGLU, bias add, cast, which reads one array six times and
+// another three times, one MI355X, as a replayed graph: 35.0 us with each op's
+// blocks in a run of their own and streamed loads (201 MB in and out of the
+// L2s), 28.2 with plain loads, 28.6 in groups; [4096, 2560] 54.5, 52.5, 49.8; f32
+// [4096, 1536] 58.6, 59.6, 46.9; f32 [2000, 960] 25.3, 22.4, 18.1.
 struct FusedTable {
-    uint32_t first[kMaxFused];  // each op's first block in the fused grid (ascending)
+    // each group's first block in the fused grid (ascending) at its first op's
+    // index, kNoBlock at its other ops
+    uint32_t first[kMaxFused];
     uint32_t count;
+    uint32_t members[kMaxFused];  // ops of the group, at its first op
+    uint32_t weight[kMaxFused];   // blocks of a slot each op takes (groups of several)
+    uint32_t weights[kMaxFused];  // their sum over the group, at its first op
     FusedSeg seg[kMaxFused];
 };
+constexpr uint32_t kNoBlock = 0xffffffffu;
+
+// Elements of a slot: a power of two of at least the largest block (4096) and
+// at most an eighth of an XCD's share (so that the XCDs come out even), up to
+// kMaxSlot (f16 [4096, 2560]: slots of 4096 53.1 us, 16384 52.5, 65536 49.8,
+// 2^18 50.1).
+constexpr uint32_t kMinSlot = 4096, kMaxSlot = 65536;
+inline uint32_t slot_elements(uint64_t n) {
+    uint32_t s = kMinSlot;
+    while (s < kMaxSlot && n >= uint64_t(s) * 2 * 64) s *= 2;
+    return s;
+}
 
 constexpr int kBroadcastUnroll = 4;  // packs per thread of the bias add
 constexpr int kFusedBiasUnroll = 1;  // the same inside the fused launch (FusedShape)
@@ -436,14 +473,14 @@ constexpr uint32_t fused_kind() {
 template <typename TIn, typename TOut, int ARITY, typename Op>
 __device__ inline void fused_map(const FusedSeg& s, uint32_t blk) {
     typedef FusedShape<Op, TIn, TOut> M;
-    map_body<TIn, TOut, map_pack<TIn, TOut>(), M::unroll, ARITY, M::nt_store, M::phased, Op>(
+    map_body<TIn, TOut, map_pack<TIn, TOut>(), M::unroll, ARITY, M::nt_store, M::phased, Op, false>(
         static_cast<const TIn*>(s.a), static_cast<const TIn*>(s.b), static_cast<TOut*>(s.out),
         s.n_packs, s.tail, Op{}, blk);
 }
 
 template <typename T>
 __device__ inline void fused_bias(const FusedSeg& s, uint32_t blk, uint32_t nblk) {
-    broadcast_body<T, 16 / sizeof(T), kFusedBiasUnroll>(
+    broadcast_body<T, 16 / sizeof(T), kFusedBiasUnroll, false>(
         static_cast<const T*>(s.a), static_cast<const T*>(s.b), static_cast<T*>(s.out),
         s.n_packs, s.div, blk, nblk);
 }
@@ -472,15 +509,26 @@ __device__ inline void fused_repeat(const FusedSeg& s, uint32_t blk, uint32_t nb
 }
 
 __global__ __launch_bounds__(kThreads) void k_fused(FusedTable t) {
-    // the op of this block: the last whose first block is not past it (the
+    // the group of this block: the last whose first block is not past it (the
     // firsts are read at once and compared, no dependent loads)
-    uint32_t i = 0;
+    uint32_t i = 0, end = gridDim.x;
 #pragma unroll
-    for (uint32_t j = 1; j < kMaxFused; ++j) i += (j < t.count && blockIdx.x >= t.first[j]) ? 1u : 0u;
+    for (uint32_t j = 1; j < kMaxFused; ++j)
+        if (j < t.count && blockIdx.x >= t.first[j]) i = j;
+#pragma unroll
+    for (uint32_t j = kMaxFused - 1; j >= 1; --j)
+        if (j < t.count && j > i && t.first[j] != kNoBlock) end = t.first[j];
+    uint32_t blk = blockIdx.x - t.first[i];
+    const uint32_t nblk = end - t.first[i];  // (groups of one op)
+    if (t.members[i] > 1) {
+        // block 8 (w s + j) + x: share j of slot 8 s + x, w shares a slot
+        const uint32_t w = t.weights[i];
+        const uint32_t k = blk / 8, s8 = k / w;
+        uint32_t j = k - s8 * w;
+        while (j >= t.weight[i]) j -= t.weight[i++];  // the op of share j
+        blk = (s8 * 8 + blk % 8) * t.weight[i] + j;
+    }
     const FusedSeg& s = t.seg[i];  // read in place from the kernel arguments
-    const uint32_t first = t.first[i];
-    const uint32_t blk = blockIdx.x - first;
-    const uint32_t nblk = (i + 1 < t.count ? t.first[i + 1] : gridDim.x) - first;
     switch (s.kind) {
         case kFusedAddF32: fused_map<float, float, 2, AddOp>(s, blk); break;
         case kFusedMulF32: fused_map<float, float, 2, MulOp>(s, blk); break;
@@ -492,7 +540,7 @@ __global__ __launch_bounds__(kThreads) void k_fused(FusedTable t) {
         case kFusedSwigluF16: fused_map<half_t, half_t, 2, SwigluF16Op>(s, blk); break;
         case kFusedCastF32F16: fused_map<float, half_t, 1, CopyOp>(s, blk); break;
         case kFusedCastF16F32: fused_map<half_t, float, 1, CopyOp>(s, blk); break;
-        case kFusedBiasF32: fused_bias<float>(s, blk, nblk); break;
+        case kFusedBiasF32: fused_bias<float>(s, blk, nblk); break;  // one tile a block
         case kFusedBiasF16: fused_bias<half_t>(s, blk, nblk); break;
         case kFusedGatherF32: fused_gather<float>(s, blk, nblk); break;
         case kFusedGatherF16: fused_gather<half_t>(s, blk, nblk); break;
@@ -535,7 +583,9 @@ rl_status launch_map(rl_context* ctx, const char* name, const void* a, const voi
         if (kind != 0 && fusing(ctx)) {
             FusedOp f;
             f.kind = kind;
-            f.blocks = grid_for(n_packs, uint64_t(kThreads) * FusedShape<Op, TIn, TOut>::unroll);
+            constexpr uint32_t per_block = kThreads * FusedShape<Op, TIn, TOut>::unroll;
+            f.blocks = grid_for(n_packs, per_block);
+            f.block_elements = per_block * N;
             f.a = pa;
             f.b = pb;
             f.out = po;
@@ -588,6 +638,7 @@ rl_status launch_add_broadcast(rl_context* ctx, const char* name, const rl_buffe
         FusedOp f;
         f.kind = sizeof(T) == 4 ? kFusedBiasF32 : kFusedBiasF16;
         f.blocks = grid_for(n_packs, uint64_t(kThreads) * kFusedBiasUnroll);
+        f.block_elements = kThreads * kFusedBiasUnroll * N;
         f.a = px;
         f.b = pbias;
         f.out = po;
@@ -654,11 +705,45 @@ rl_status defer_fused(rl_context* ctx, const FusedOp& f) {
 
 rl_status flush_fused(rl_context* ctx) {
     if (ctx->fused_count == 0) return RL_OK;
+    // ops in their recorded order, those of a group right after its first
+    // (they are independent, so the order is free)
+    uint32_t order[kMaxFused], n = 0;
+    bool taken[kMaxFused] = {};
     FusedTable t{};
     uint32_t first = 0;
     for (uint32_t i = 0; i < ctx->fused_count; ++i) {
-        const FusedOp& f = ctx->fused[i];
-        t.first[i] = first;
+        if (taken[i]) continue;
+        const FusedOp& lead = ctx->fused[i];
+        const uint32_t start = n;
+        order[n++] = i;
+        for (uint32_t j = i + 1; j < ctx->fused_count && lead.block_elements != 0; ++j) {
+            const FusedOp& f = ctx->fused[j];
+            if (taken[j] || f.block_elements == 0 || f.read[0][0] != lead.read[0][0] ||
+                f.read[0][1] != lead.read[0][1])
+                continue;
+            taken[j] = true;
+            order[n++] = j;
+        }
+        uint32_t blocks = lead.blocks;
+        if (n - start > 1) {
+            const uint32_t slot =
+                slot_elements(uint64_t(lead.blocks) * lead.block_elements);
+            uint32_t w = 0, slots = 0;
+            for (uint32_t k = start; k < n; ++k) {
+                const FusedOp& f = ctx->fused[order[k]];
+                t.weight[k] = slot / f.block_elements;
+                w += t.weight[k];
+                slots = std::max(slots, uint32_t(ceil_div(f.blocks, t.weight[k])));
+            }
+            t.weights[start] = w;
+            blocks = uint32_t(ceil_div(slots, 8)) * 8 * w;  // blocks past an op's last do nothing
+        }
+        t.members[start] = n - start;
+        for (uint32_t k = start; k < n; ++k) t.first[k] = k == start ? first : kNoBlock;
+        first += blocks;
+    }
+    for (uint32_t i = 0; i < n; ++i) {
+        const FusedOp& f = ctx->fused[order[i]];
         FusedSeg& g = t.seg[i];
         g.kind = f.kind;
         g.tail = f.tail;
@@ -675,7 +760,6 @@ rl_status flush_fused(rl_context* ctx) {
             g.outer.dim[d] = FastDiv(f.outer_dim[d] ? f.outer_dim[d] : 1u);
             g.outer.stride[d] = f.outer_stride[d];
         }
-        first += f.blocks;
     }
     t.count = ctx->fused_count;
     ctx->fused_count = 0;

@@ -220,3 +220,32 @@ def test_other_kernels_between_fused_ops(ctx):
     eager = replay_and_compare(ctx, record, [s, y, z])
     assert_bitexact(eager[0], o.add(a, b), "add")
     assert_bitexact(eager[2], o.mul(eager[1], a), "mul of the RMSNorm output")
+
+
+@pytest.mark.parametrize("dtype", [F16, F32])
+@pytest.mark.parametrize("n", [7, 4096, 4097, 300 * 1536 + 5, 4096 * 64 * 8 + 8])
+def test_ops_over_one_input_share_its_slots(ctx, dtype, n):
+    """Ops that read one array go out slot by slot over all of them (several
+    blocks an op where packs are smaller): one block, whole and ragged slots,
+    several slots a round of the XCDs, a second group and an op of its own."""
+    shape = (1, n)
+    a, b = (ctx.upload(norm(f"slot-{t}", shape, dtype)) for t in "ab")
+    other = F32 if dtype == F16 else F16
+    x = ctx.upload(norm("slot-x", (3, 1536), F32))
+    bias = ctx.upload(norm("slot-bias", (1536,), F32))
+    outs = [ctx.empty(shape, dtype) for _ in range(5)] + [ctx.empty(shape, other)]
+    outs += [ctx.empty((3, 1536), F32) for _ in range(3)]
+
+    def record():
+        ctx.add(a, b, outs[0])
+        ctx.add_broadcast(x, bias, outs[6])
+        ctx.mul(b, a, outs[1])
+        ctx.silu(a, outs[2])
+        ctx.swiglu(a, b, outs[3])
+        ctx.silu(b, outs[4])
+        ctx.cast(a, other, outs[5])
+        ctx.silu(x, outs[7])
+        ctx.mul(bias_rows, bias_rows, outs[8])
+
+    bias_rows = ctx.upload(norm("slot-rows", (3, 1536), F32))
+    replay_and_compare(ctx, record, outs)
