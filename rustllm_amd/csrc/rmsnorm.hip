@@ -34,11 +34,27 @@ __device__ inline uint32_t clamp_pack(uint32_t p, uint32_t h_packs) {
 // Rows per launch chunk: keeps blocks x threads far below 2^32.
 constexpr uint32_t kRowChunk = 1u << 22;
 
+// Rows are read with plain loads while a launch reads at most
+// kStreamReadBytes (CACHED): what the MALL still holds of them, from the
+// kernel or launch before, is then found there.  One MI355X, three rotated
+// buffer sets, streamed against plain: RMSNorm then add + RMSNorm over the
+// same x, f32 [16384, 960] 63.7 / 60.3 us, [8192, 960] 33.3 / 28.4, [16384, 576]
+// 38.0 / 33.6, f16 [16384, 960] 31.7 / 29.4, [4096, 960] 10.5 / 9.3; one op
+// alone, f32 [16384, 960] 21.6 / 18.8, with the add 42.2 / 42.6.  Over more sets
+// than the MALL holds plain loads cost a little: 22.1 / 22.3 and 42.7 / 44.1.
+template <bool CACHED, typename V>
+__device__ inline V load_row(const V* p) {
+    if constexpr (CACHED)
+        return *p;
+    else
+        return load_stream(p);
+}
+
 // Rows [row_base, row_base + rows) of the launch chunk; TPR lanes per row,
 // kThreads / TPR rows per block.  Lanes of a group stride over the row's
 // packs (pack p = lane + k * TPR), so each load instruction covers TPR
 // consecutive packs of every row in the wave.
-template <typename T, int N, int NV, int TPR, bool ADD, bool WLATE>
+template <typename T, int N, int NV, int TPR, bool ADD, bool WLATE, bool CACHED>
 __global__ __launch_bounds__(kThreads) void k_rmsnorm_rows(
     const T* __restrict__ x, const T* __restrict__ residual, const T* __restrict__ weight,
     T* __restrict__ sum_out, T* __restrict__ y, uint32_t row_base, uint32_t rows,
@@ -57,13 +73,13 @@ __global__ __launch_bounds__(kThreads) void k_rmsnorm_rows(
     // row are reloads of its last pack, never used): a load under a per-pack
     // branch made the compiler wait for each f16 load before issuing the next.
 #pragma unroll
-    for (int k = 0; k < NV; ++k) v[k] = load_stream(xr + clamp_pack(lane + k * TPR, h_packs));
+    for (int k = 0; k < NV; ++k) v[k] = load_row<CACHED>(xr + clamp_pack(lane + k * TPR, h_packs));
     if constexpr (ADD) {
         const V* rr = reinterpret_cast<const V*>(residual) + row_off;
         V* sr = reinterpret_cast<V*>(sum_out) + row_off;
         V r[NV];
 #pragma unroll
-        for (int k = 0; k < NV; ++k) r[k] = load_stream(rr + clamp_pack(lane + k * TPR, h_packs));
+        for (int k = 0; k < NV; ++k) r[k] = load_row<CACHED>(rr + clamp_pack(lane + k * TPR, h_packs));
 #pragma unroll
         for (int k = 0; k < NV; ++k) {
             const uint32_t p = lane + k * TPR;
@@ -221,11 +237,17 @@ void launch_rows(rl_context* ctx, const T* x, const T* residual, const T* weight
                  T* y, uint32_t rows, uint32_t h_packs, float hidden, float eps) {
     constexpr uint32_t kRowsPerBlock = kThreads / TPR;
     static_assert(kRowChunk % kRowsPerBlock == 0, "chunks must hold whole blocks");
+    const bool cached =
+        uint64_t(rows) * h_packs * 16 * (ADD ? 2 : 1) <= kStreamReadBytes;
     for (uint32_t base = 0; base < rows; base += kRowChunk) {
         const uint32_t n = rows - base < kRowChunk ? rows - base : kRowChunk;
         const dim3 grid(unsigned(ceil_div(n, kRowsPerBlock))), block(kThreads);
-        RL_LAUNCH(ctx, (k_rmsnorm_rows<T, N, NV, TPR, ADD, (NV >= 3)>), grid, block, x,
-                  residual, weight, sum_out, y, base, rows, h_packs, hidden, eps);
+        if (cached)
+            RL_LAUNCH(ctx, (k_rmsnorm_rows<T, N, NV, TPR, ADD, (NV >= 3), true>), grid, block, x,
+                      residual, weight, sum_out, y, base, rows, h_packs, hidden, eps);
+        else
+            RL_LAUNCH(ctx, (k_rmsnorm_rows<T, N, NV, TPR, ADD, (NV >= 3), false>), grid, block, x,
+                      residual, weight, sum_out, y, base, rows, h_packs, hidden, eps);
         if (rows - base <= kRowChunk) break;
     }
 }

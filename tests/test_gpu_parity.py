@@ -1056,3 +1056,27 @@ def test_rope_and_add_rmsnorm_over_inputs(ctx, dtype, shape):
     run(ctx, lambda: ctx.add_rmsnorm(da, dr, wt, 1e-5, sum_out=da, norm_out=dr))
     assert_bitexact(da.numpy(), s_ref, f"add + rmsnorm sum over x {shape}")
     assert_bitexact(dr.numpy(), y_ref, f"add + rmsnorm rows over the residual {shape}")
+
+
+@pytest.mark.parametrize("dtype", [np.float32, np.float16])
+def test_add_rmsnorm_rows_past_the_streaming_size(ctx, dtype):
+    """A launch that reads more than 160 MB streams its rows, one below reads
+    them plainly: both sides of the rule, sampled rows against the oracle (the
+    rows are independent) and the same rows in a small launch bit for bit."""
+    h = 960
+    edge = (160 << 20) // (2 * h * np.dtype(dtype).itemsize)  # rows at the rule, with the add
+    w = synth.uniform_range(71, (h,), 0.5, 1.5, dtype)
+    base = synth.normal(72, (1024, h), 0.0, 2.0, dtype)
+    for rows in (edge, edge + 1):
+        x = np.resize(base, (rows, h))
+        ctx.begin()
+        s, y = ctx.add_rmsnorm(ctx.upload(x), ctx.upload(x[::-1]), ctx.upload(w), 1e-5)
+        ctx.finish()
+        s, y = s.numpy(), y.numpy()
+        pick = np.array([0, 1, rows // 2, rows - 2, rows - 1])
+        ctx.begin()
+        s2, y2 = ctx.add_rmsnorm(ctx.upload(x[pick]), ctx.upload(x[::-1][pick]), ctx.upload(w),
+                                 1e-5)
+        ctx.finish()
+        assert np.array_equal(s[pick], s2.numpy()) and np.array_equal(y[pick], y2.numpy())
+        assert np.array_equal(s, x + x[::-1])
