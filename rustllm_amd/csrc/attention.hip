@@ -1753,16 +1753,30 @@ uint32_t flash_pairs(const rl_context* ctx, uint64_t heads, uint32_t tiles) {
 // Causal squares with fewer pairs stay on the 32-query tiles (8 heads of 128
 // x [2048, 2048]: 31.8 us against 34.0 in 4 chunks; 15 x [1024, 1024]: 14.0
 // against 20.1): each chunk writes and merges another f32 copy of the output.
-uint32_t flash_key_chunks(uint64_t heads, uint64_t q_len, uint64_t kv_len, uint64_t start,
-                          uint64_t head_dim) {
+// Far behind the cache (start >= 4 q_len) all tiles are about equally long, and
+// one tile a workgroup in half the chunks is the same share of the work with
+// half the partials: taken where the halved count does not leave the shares
+// larger (32 heads of 128 x 512 queries after 3000 keys: 2 chunks a tile 45.0
+// us, 4 a pair 56.8; 15 of 64 x 512 after 3584 22.8, 26.6; 8 of 128 x 200 after
+// 2000 18.5, 27.1).
+struct FlashChunks {
+    uint32_t chunks;  // per tile
+    bool by_tile;     // workgroups of one tile, not of a pair
+};
+FlashChunks flash_key_chunks(uint64_t heads, uint64_t q_len, uint64_t kv_len, uint64_t start,
+                             uint64_t head_dim) {
     const uint64_t wide = heads * ((ceil_div(q_len, 128) + 1) / 2);
     const uint64_t bn = head_dim <= 64 ? 128 : 64;
     const uint64_t keys = std::min<uint64_t>(kv_len, start + q_len);  // the longest tile's
     const uint64_t steps = ceil_div(ceil_div(keys, bn), 2);
-    if (wide >= kFlashFillBlocks) return wide <= 128 && steps >= 16 ? 2 : 1;
-    if (start == 0 || steps < 16) return 1;
-    const uint64_t chunks = std::min<uint64_t>({256 / wide, 8, steps / 2});
-    return uint32_t(std::max<uint64_t>(chunks, 1));
+    if (wide >= kFlashFillBlocks) return {wide <= 128 && steps >= 16 ? 2u : 1u, false};
+    if (start == 0 || steps < 16) return {1, false};
+    const uint64_t chunks = std::max<uint64_t>(std::min<uint64_t>({256 / wide, 8, steps / 2}), 1);
+    const uint64_t halved =
+        std::min<uint64_t>({256 / (heads * ceil_div(q_len, 128)), 8, steps / 2});
+    if (start >= 4 * q_len && halved >= 2 && 2 * halved >= chunks)
+        return {uint32_t(halved), true};
+    return {uint32_t(chunks), false};
 }
 
 // The matrix-core kernels by head size: f16 in key blocks of 128 (head
@@ -2104,10 +2118,11 @@ rl_status attention_entry(rl_context* ctx, const char* name, const rl_buffer* q,
             // (chunked prefill, short or few-head prefills), the pool holding
             // the partials (not while a graph records, nor for the
             // allocation-free entry).
-            const uint32_t chunks = flash_key_chunks(heads, s.q_len, s.kv_len, start, s.head_dim);
+            const auto [chunks, by_tile] =
+                flash_key_chunks(heads, s.q_len, s.kv_len, start, s.head_dim);
             if (chunks > 1 && mode == DecodeScratch::kPool && !ctx->capturing) {
                 p.tiles = uint32_t(ceil_div(s.q_len, 128));
-                p.pairs = (p.tiles + 1) / 2;
+                p.pairs = by_tile ? p.tiles : (p.tiles + 1) / 2;
                 p.kchunks = chunks;
                 const uint64_t units = heads * p.tiles * chunks * 128;
                 void* part = nullptr;

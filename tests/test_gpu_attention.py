@@ -559,3 +559,13 @@ def test_gqa_f32_extremes(ctx, hd, ql, kl):
         assert np.array_equal(got[inf], ref[inf].astype(np.float32))
         ok = np.isfinite(ref)
         assert np.allclose(got[ok], ref[ok], rtol=0, atol=1e-3)
+
+
+@pytest.mark.parametrize("shape", [
+    (1, 32, 8, 500, 3000, 3008, 128, 2500),   # 128 tiles: 2 key chunks of one tile each
+    (1, 15, 5, 300, 4500, 4544, 64, 4200),    # 45 tiles, odd per head: 5 chunks of one tile
+    (1, 25, 5, 512, 3072, 3072, 128, 2560),   # 100 tiles: 5 chunks of a pair
+    (2, 5, 5, 130, 4100, 4128, 96, 3970),     # 20 tiles, batch 2: 8 chunks of one tile
+])
+def test_attention_key_chunks_by_tile(ctx, shape):
+    test_attention_within_float64_bound(ctx, np.float16, shape)
