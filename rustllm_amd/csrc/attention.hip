@@ -1758,7 +1758,10 @@ uint32_t flash_pairs(const rl_context* ctx, uint64_t heads, uint32_t tiles) {
 // half the partials: taken where the halved count does not leave the shares
 // larger (32 heads of 128 x 512 queries after 3000 keys: 2 chunks a tile 45.0
 // us, 4 a pair 56.8; 15 of 64 x 512 after 3584 22.8, 26.6; 8 of 128 x 200 after
-// 2000 18.5, 27.1).
+// 2000 18.5, 27.1).  Where the tiles alone fill the CUs, from 96 pairs on, they
+// are not split at all (32 heads of 128 x 900 after 4000 keys: 83.5 us, 2
+// chunks a pair 104.2; 48 x 500 after 2500 48.4, 65.0; 15 of 64 x 2048 after 9000
+// 107.5, 111.4).
 struct FlashChunks {
     uint32_t chunks;  // per tile
     bool by_tile;     // workgroups of one tile, not of a pair
@@ -1769,7 +1772,10 @@ FlashChunks flash_key_chunks(uint64_t heads, uint64_t q_len, uint64_t kv_len, ui
     const uint64_t bn = head_dim <= 64 ? 128 : 64;
     const uint64_t keys = std::min<uint64_t>(kv_len, start + q_len);  // the longest tile's
     const uint64_t steps = ceil_div(ceil_div(keys, bn), 2);
-    if (wide >= kFlashFillBlocks) return {wide <= 128 && steps >= 16 ? 2u : 1u, false};
+    if (wide >= kFlashFillBlocks) {
+        const bool tiles_fit = start >= 4 * q_len && heads * ceil_div(q_len, 128) <= 256;
+        return {wide <= 128 && steps >= 16 && !tiles_fit ? 2u : 1u, false};
+    }
     if (start == 0 || steps < 16) return {1, false};
     const uint64_t chunks = std::max<uint64_t>(std::min<uint64_t>({256 / wide, 8, steps / 2}), 1);
     const uint64_t halved =

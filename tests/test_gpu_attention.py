@@ -566,6 +566,7 @@ def test_gqa_f32_extremes(ctx, hd, ql, kl):
     (1, 15, 5, 300, 4500, 4544, 64, 4200),    # 45 tiles, odd per head: 5 chunks of one tile
     (1, 25, 5, 512, 3072, 3072, 128, 2560),   # 100 tiles: 5 chunks of a pair
     (2, 5, 5, 130, 4100, 4128, 96, 3970),     # 20 tiles, batch 2: 8 chunks of one tile
+    (1, 48, 8, 300, 2100, 2112, 128, 1800),   # 144 tiles, 96 pairs: one tile, not split
 ])
 def test_attention_key_chunks_by_tile(ctx, shape):
     test_attention_within_float64_bound(ctx, np.float16, shape)
