@@ -65,6 +65,7 @@ struct AttnParams {
     uint64_t kv_head_stride;  // elements between KV heads (kv_capacity * head_dim)
     float scale;           // attention scale
     float scale_log2;      // scale * log2(e)
+    float slack;           // rescaling threshold (f16 MFMA kernel): kRescaleSlack or kFarSlack
     uint32_t kchunks;      // key chunks per query tile (f16 MFMA kernel, PARTIAL)
     float* part;           // PARTIAL: unnormalised outputs, [tile unit][query][head_dim]
     float* part_ml;        // PARTIAL: (max in log2 units, sum) per [tile unit][query]
@@ -122,6 +123,15 @@ __device__ inline void dma_to_lds(i32x4 rsrc, uint32_t lds_addr, uint32_t voffse
 // rescale of the running sum and output; probabilities exp2(t - m) then stay
 // below 2^3, well inside f16 and f32 range.
 constexpr float kRescaleSlack = 3.0f;
+// The threshold where flash_key_chunks takes few or no chunks far behind the
+// cache.  f16 probabilities round finest just below the maximum they are
+// scaled by, and every chunk follows its own, so fewer chunks need to follow
+// it more closely to be as accurate.  Relative error against 64 bits of 15
+// heads of 64 x 512 queries after 3584 keys: 2.77e-4 in 8 chunks a tile pair,
+// in 5 a tile 2.83e-4 at a threshold of 3, 2.79e-4 at 2, 2.74e-4 at 1 (32 heads
+// of 128 x 512 after 3000: 2.86e-4; 2.89, 2.85, 2.79).  One MI355X, 3 against
+// 1: 49.0 / 50.0 us for the latter, 32 of 128 x 900 after 4000 88.9 / 91.3.
+constexpr float kFarSlack = 1.0f;
 
 // One query row by one wave with plain f32 products, as k_attention_rows
 // computes it: for rows whose output the split products leave non-finite
@@ -416,7 +426,7 @@ __global__ __launch_bounds__(64 * QW * KSPLIT) void k_flash_attention(
                 mx = fmaxf(mx, my);
                 mx = max_halves(mx);
                 const float mx_log2 = mx * p.scale_log2;
-                if (__any(mx_log2 > m + kRescaleSlack)) {
+                if (__any(mx_log2 > m + (ANY ? kRescaleSlack : p.slack))) {
                     const float m_new = fmaxf(m, mx_log2);
                     const float alpha = m_new > m ? __builtin_amdgcn_exp2f(m - m_new) : 1.0f;
                     m = m_new;
@@ -1765,6 +1775,7 @@ uint32_t flash_pairs(const rl_context* ctx, uint64_t heads, uint32_t tiles) {
 struct FlashChunks {
     uint32_t chunks;  // per tile
     bool by_tile;     // workgroups of one tile, not of a pair
+    float slack;      // rescaling threshold
 };
 FlashChunks flash_key_chunks(uint64_t heads, uint64_t q_len, uint64_t kv_len, uint64_t start,
                              uint64_t head_dim) {
@@ -1774,15 +1785,17 @@ FlashChunks flash_key_chunks(uint64_t heads, uint64_t q_len, uint64_t kv_len, ui
     const uint64_t steps = ceil_div(ceil_div(keys, bn), 2);
     if (wide >= kFlashFillBlocks) {
         const bool tiles_fit = start >= 4 * q_len && heads * ceil_div(q_len, 128) <= 256;
-        return {wide <= 128 && steps >= 16 && !tiles_fit ? 2u : 1u, false};
+        if (wide > 128 || steps < 16) return {1, false, kRescaleSlack};
+        if (tiles_fit) return {1, false, kFarSlack};
+        return {2, false, kRescaleSlack};
     }
-    if (start == 0 || steps < 16) return {1, false};
+    if (start == 0 || steps < 16) return {1, false, kRescaleSlack};
     const uint64_t chunks = std::max<uint64_t>(std::min<uint64_t>({256 / wide, 8, steps / 2}), 1);
     const uint64_t halved =
         std::min<uint64_t>({256 / (heads * ceil_div(q_len, 128)), 8, steps / 2});
     if (start >= 4 * q_len && halved >= 2 && 2 * halved >= chunks)
-        return {uint32_t(halved), true};
-    return {uint32_t(chunks), false};
+        return {uint32_t(halved), true, kFarSlack};
+    return {uint32_t(chunks), false, kRescaleSlack};
 }
 
 // The matrix-core kernels by head size: f16 in key blocks of 128 (head
@@ -2124,9 +2137,11 @@ rl_status attention_entry(rl_context* ctx, const char* name, const rl_buffer* q,
             // (chunked prefill, short or few-head prefills), the pool holding
             // the partials (not while a graph records, nor for the
             // allocation-free entry).
-            const auto [chunks, by_tile] =
+            const auto [chunks, by_tile, slack] =
                 flash_key_chunks(heads, s.q_len, s.kv_len, start, s.head_dim);
-            if (chunks > 1 && mode == DecodeScratch::kPool && !ctx->capturing) {
+            const bool pooled = mode == DecodeScratch::kPool && !ctx->capturing;
+            p.slack = pooled ? slack : kRescaleSlack;
+            if (chunks > 1 && pooled) {
                 p.tiles = uint32_t(ceil_div(s.q_len, 128));
                 p.pairs = by_tile ? p.tiles : (p.tiles + 1) / 2;
                 p.kchunks = chunks;

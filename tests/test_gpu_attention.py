@@ -570,3 +570,23 @@ def test_gqa_f32_extremes(ctx, hd, ql, kl):
 ])
 def test_attention_key_chunks_by_tile(ctx, shape):
     test_attention_within_float64_bound(ctx, np.float16, shape)
+
+
+@pytest.mark.parametrize("shape,most", [
+    ((1, 15, 5, 512, 4096, 4096, 64, 3584), 2.78e-4),   # 5 chunks a tile
+    ((1, 32, 8, 512, 3512, 3520, 128, 3000), 2.875e-4),  # 2 chunks a tile
+    ((1, 48, 8, 300, 2800, 2816, 128, 2500), 2.888e-4),  # 144 tiles, 96 pairs: not split
+])
+def test_attention_far_behind_the_cache_rounds_no_coarser(ctx, shape, most):
+    """Relative 2-norm error of f16 calls that take fewer key chunks than their
+    tile pairs would: no more than the pairs' chunks leave (`most`, measured on
+    these inputs; the rounding of the output alone is 2.0e-4)."""
+    b, qh, kvh, ql, kl, cap, hd, start = shape
+    q = synth.normal(synth.seed_for("far-q", *shape), (b, qh, ql, hd)).astype(np.float16)
+    k = cache(synth.seed_for("far-k", *shape), b, kvh, cap, hd, kl, np.float16)
+    v = cache(synth.seed_for("far-v", *shape), b, kvh, cap, hd, kl, np.float16)
+    scale = 1.0 / np.sqrt(hd)
+    got = run_attention(ctx, q, k, v, scale, start, kl)
+    exact, _, _ = attention_exact(q, k, v, scale, start, kl)
+    err = np.linalg.norm(got.astype(np.float64) - exact) / np.linalg.norm(exact)
+    assert err <= most, f"{shape}: {err:.4g}"
