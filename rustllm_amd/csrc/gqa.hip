@@ -556,13 +556,19 @@ __global__ __launch_bounds__(256) void k_gqa_qk_bf16x3(const float* __restrict__
 // stages its 32 x BN probabilities in LDS (whole row segments per load) and
 // splits its lane's 8 consecutive keys; V blocks are split into LDS as three
 // planes for the QW waves of a share.  The next step's operands are in flight
-// during this step's products.  Bound by the reads of the probabilities.
-// Outputs that are not finite or below 2^-36, and all of a wave's that met a
-// probability or value of 2^60 or more, are computed by plain dot products.
+// during this step's products.  Bound by the splitting, two or three waves a
+// SIMD (151 MB of probabilities at 2.3 TB/s).
+// A lane's half row of its wave's share whose sums are not finite (infinities,
+// NaN, sums of 2^80 or more) is computed again by plain products; with an
+// infinite value row, so in every query of its heads, 9 heads of 64 x [1024,
+// 1024] take 161 us for 26.
 // VEC: probability rows on the 16-byte grid (streamed loads); otherwise
 // plain unaligned 16-byte loads, a row's last partial group element-wise.
+// The probabilities are scaled on their way into LDS, or where the loads are
+// unaligned as they are split ([15, 4093, 4093]: 322 us, on the way 327; aligned
+// [9, 2048, 2048] 65.7, split 68.9).
 // One MI355X, 9 heads of 64 x [2048, 2048]: 95.2 us on the f32 matrix
-// cores, 128 queries a workgroup, 66.8 us.
+// cores, 128 queries a workgroup, 66 us.
 template <int NT, int QW, int KS, int BN, bool VEC>
 __global__ __launch_bounds__(64 * QW * KS) void k_gqa_pv_bf16x3(const float* __restrict__ probs,
                                                                 const float* __restrict__ v,
@@ -625,7 +631,8 @@ __global__ __launch_bounds__(64 * QW * KS) void k_gqa_pv_bf16x3(const float* __r
 #pragma unroll
         for (int i = 0; i < P_LOADS; ++i)
             *reinterpret_cast<f32x4*>(my + (i * P_ROWS + lane / (BN / 4)) * PS +
-                                      (lane % (BN / 4)) * 4) = pr[i];
+                                      (lane % (BN / 4)) * 4) =
+                pr[i] * (VEC ? kPartScale : 1.0f);
     };
     auto load_v = [&](uint32_t step, f32x8 (&vr)[LOADS]) {
 #pragma unroll
@@ -644,7 +651,6 @@ __global__ __launch_bounds__(64 * QW * KS) void k_gqa_pv_bf16x3(const float* __r
             vr[li] = __builtin_shufflevector(x0, x1, 0, 1, 2, 3, 4, 5, 6, 7);
         }
     };
-    float vmax = 0.0f, pmax = 0.0f;  // the largest magnitudes this thread split
     auto store_v = [&](const f32x8 (&vr)[LOADS]) {
 #pragma unroll
         for (int li = 0; li < LOADS; ++li) {
@@ -652,9 +658,7 @@ __global__ __launch_bounds__(64 * QW * KS) void k_gqa_pv_bf16x3(const float* __r
             const uint32_t c = chunk % BLOCK_CHUNKS;
             const uint32_t r = c / ROW_CHUNKS, ch = c % ROW_CHUNKS;
             if (RD > D && ch >= D / 8) continue;
-#pragma unroll
-            for (int e = 0; e < 8; ++e) vmax = fmaxf(vmax, fabsf(vr[li][e]));
-            const Bf16x3 x = split_bf16(vr[li]);
+            const Bf16x3 x = split_bf16(vr[li] * kPartScale);
             __bf16* dst = vs + (chunk / BLOCK_CHUNKS) * 3 * PLANE + r * RD +
                           8 * (ch ^ lds_swizzle<SW>(r));
 #pragma unroll
@@ -702,9 +706,7 @@ __global__ __launch_bounds__(64 * QW * KS) void k_gqa_pv_bf16x3(const float* __r
             const f32x4 x0 = *reinterpret_cast<const f32x4*>(prow);
             const f32x4 x1 = *reinterpret_cast<const f32x4*>(prow + 4);
             const f32x8 x = __builtin_shufflevector(x0, x1, 0, 1, 2, 3, 4, 5, 6, 7);
-#pragma unroll
-            for (int e = 0; e < 8; ++e) pmax = fmaxf(pmax, fabsf(x[e]));
-            const Bf16x3 pb = split_bf16(x);
+            const Bf16x3 pb = split_bf16(x * (VEC ? 1.0f : kPartScale));
 #pragma unroll
             for (int t = 0; t < NT; ++t) {
                 Bf16x3 va;
@@ -727,8 +729,39 @@ __global__ __launch_bounds__(64 * QW * KS) void k_gqa_pv_bf16x3(const float* __r
         }
         __syncthreads();
     }
-    // any value or probability past 2^60 anywhere in the workgroup
-    const bool huge = __syncthreads_or(!(vmax < 0x1p60f) || !(pmax < 0x1p60f));
+    const uint32_t qi = q0 + col;
+    float finite = 0.0f;  // NaN if a sum is not finite
+#pragma unroll
+    for (int t = 0; t < NT; ++t)
+#pragma unroll
+        for (int r = 0; r < 16; ++r) {
+            finite = __builtin_fmaf(o[t][r], 0.0f, finite);
+            o[t][r] *= kProductUnscale;
+        }
+    if (finite != 0.0f) {  // this lane's half of a row, by plain products
+        const float* prow = pbase + uint64_t(min(qi, p.q_len - 1)) * p.kv_len;
+#pragma unroll
+        for (int t = 0; t < NT; ++t)
+#pragma unroll
+            for (int r = 0; r < 16; ++r) o[t][r] = 0.0f;
+        for (uint32_t blk = sub; blk < blocks; blk += KS) {
+            const uint32_t end = min(p.kv_len, (blk + 1) * BN);
+#pragma unroll 1
+            for (uint32_t key = blk * BN; key < end; ++key) {
+                const float pk = prow[key];
+                const float* vrow = vh + uint64_t(key) * D + 4 * hs;
+#pragma unroll
+                for (int t = 0; t < NT; ++t)
+#pragma unroll
+                    for (int g = 0; g < 4; ++g) {
+                        const f32x4 w = *reinterpret_cast<const f32x4*>(vrow + 32 * t + 8 * g);
+#pragma unroll
+                        for (int e = 0; e < 4; ++e)
+                            o[t][4 * g + e] = __builtin_fmaf(pk, w[e], o[t][4 * g + e]);
+                    }
+            }
+        }
+    }
     if constexpr (KS > 1) {
         float* mg = reinterpret_cast<float*>(lds);
         if (sub > 0) {
@@ -749,34 +782,15 @@ __global__ __launch_bounds__(64 * QW * KS) void k_gqa_pv_bf16x3(const float* __r
                 for (int r = 0; r < 16; ++r) o[t][r] += src[(16 * t + r) * 64];
         }
     }
-    const uint32_t qi = q0 + col;
     if (qi < p.q_len) {
         // register r of tile t: element 32t + 8(r / 4) + 4hs + r % 4
         float* orow = out + (uint64_t(bh) * p.q_len + qi) * D + 4 * hs;
-        bool odd = huge;
-#pragma unroll
-        for (int t = 0; t < NT; ++t)
-#pragma unroll
-            for (int r = 0; r < 16; ++r) {
-                const float a = fabsf(o[t][r]);
-                odd |= a != 0.0f && !(a > 0x1p-36f && a < INFINITY);
-            }
 #pragma unroll
         for (int t = 0; t < NT; ++t)
 #pragma unroll
             for (int g = 0; g < 4; ++g)
                 *reinterpret_cast<f32x4*>(orow + 32 * t + 8 * g) =
                     f32x4{o[t][4 * g], o[t][4 * g + 1], o[t][4 * g + 2], o[t][4 * g + 3]};
-        if (odd) {
-            const float* prow = pbase + uint64_t(qi) * p.kv_len;
-            for (uint32_t i = 0; i < D / 2; ++i) {
-                const uint32_t d = 8 * (i / 4) + i % 4;  // + 4 hs: this lane's elements
-                float sum = 0.0f;
-                for (uint32_t key = 0; key < p.kv_len; ++key)
-                    sum = __builtin_fmaf(prow[key], vh[uint64_t(key) * D + 4 * hs + d], sum);
-                orow[d] = sum;
-            }
-        }
     }
 }
 

@@ -69,8 +69,13 @@ __device__ inline h4 lds_read_transposed(const half_t* p) {
 // values the six of order 2^-18 and above are added, the three dropped are below
 // 2^-26 of the product.  Both operands of an instruction, and their layout,
 // are those of v_mfma_f32_32x32x16_f16.
-// An infinite or huge (>= 2^128 - 2^119) value's parts are not finite sums of
-// it (inf - inf): a result that is not finite has to be computed unsplit.
+// Values are scaled by kPartScale first: every f32 value, subnormals included,
+// is a multiple of 2^-149, so its parts are then multiples of 2^-125 and none
+// falls below bf16's normal range.  Values of 2^104 and above (infinities too)
+// have no such parts (inf - inf), and sums past the scaled range are infinite:
+// a result that is not finite has to be computed unsplit.
+constexpr float kPartScale = 0x1p24f;
+constexpr float kProductUnscale = 0x1p-48f;  // of a sum of products of two scaled values
 typedef __bf16 b8 __attribute__((ext_vector_type(8)));
 typedef __bf16 b4 __attribute__((ext_vector_type(4)));
 typedef __bf16 b2 __attribute__((ext_vector_type(2)));

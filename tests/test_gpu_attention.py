@@ -590,3 +590,73 @@ def test_attention_far_behind_the_cache_rounds_no_coarser(ctx, shape, most):
     exact, _, _ = attention_exact(q, k, v, scale, start, kl)
     err = np.linalg.norm(got.astype(np.float64) - exact) / np.linalg.norm(exact)
     assert err <= most, f"{shape}: {err:.4g}"
+
+
+def wide_range(seed, shape):
+    """Signed values spread evenly over all of f32's exponents up to 2^20,
+    subnormals included, whole mantissas, a tenth zeros."""
+    rng = np.random.default_rng(seed)
+    x = np.ldexp(rng.uniform(1, 2, shape), rng.integers(-148, 20, shape)).astype(np.float32)
+    return x * rng.choice(np.float32([-1, 0, 1]), shape, p=[0.45, 0.1, 0.45])
+
+
+def one_exponent_each(seed, shape, lo):
+    """Rows (the last axis) of one exponent each, from 2^lo to 2^19."""
+    rng = np.random.default_rng(seed)
+    e = rng.integers(lo, 20, shape[:-1] + (1,))
+    return np.ldexp(rng.uniform(1, 2, shape), e).astype(np.float32)
+
+
+def median_us(ctx, call):
+    """Of five calls back to back, the median of six runs, one call's share."""
+    a, b = ctx.event(), ctx.event()
+    times = []
+    for _ in range(6):
+        ctx.begin()
+        ctx.record(a)
+        for _ in range(5):
+            call()
+        ctx.record(b)
+        ctx.finish()
+        times.append(ctx.elapsed_ms(a, b) * 200)
+    ctx.destroy_event(a)
+    ctx.destroy_event(b)
+    return sorted(times)[2]
+
+
+# n products of whole f32 values: their sum's roundings, and 2^-150 each where
+# partial sums are subnormal.
+def product_bound(n, magnitude):
+    return (n + 2) * U32 * magnitude + n * 2.0 ** -150
+
+
+@pytest.mark.parametrize("hd,ql,kl", [(64, 130, 131), (128, 33, 200), (96, 64, 64), (32, 1, 37)])
+def test_gqa_pv_f32_keeps_every_exponent(ctx, hd, ql, kl):
+    """Probabilities and values of every exponent, in rows and columns of their
+    own and mixed: no part of a value is lost, subnormal results included."""
+    for p, v in ((wide_range(71, (1, 4, ql, kl)), wide_range(72, (1, 2, kl, hd))),
+                 (one_exponent_each(73, (1, 4, ql, kl), -148),
+                  np.swapaxes(one_exponent_each(74, (1, 2, hd, kl), -148), -1, -2)),
+                 (np.ones((1, 4, ql, kl), np.float32),
+                  np.full((1, 2, kl, hd), 3 * 2.0 ** -140, np.float32))):
+        ctx.begin()
+        got = ctx.gqa_pv(ctx.upload(p), ctx.upload(np.ascontiguousarray(v)))
+        ctx.finish()
+        pe, ve = p.astype(np.float64), np.repeat(v.astype(np.float64), 2, 1)
+        err = np.abs(got.numpy().astype(np.float64) - pe @ ve)
+        assert np.all(err <= product_bound(kl, np.abs(pe) @ np.abs(ve)))
+
+
+def test_gqa_pv_f32_time_does_not_depend_on_small_values(ctx):
+    """A value channel of 1e-12, and one of subnormals, at the time of ordinary
+    ones (equal as measured; the bound allows for a shared machine)."""
+    h, n, d = 9, 1024, 64
+    p = np.full((1, h, n, n), 1.0 / n, np.float32)
+    out = ctx.empty((1, h, n, d), np.float32)
+    dp, times = ctx.upload(p), []
+    for factor in (1, 1e-12, 1e-38):
+        v = synth.normal(75, (1, 3, n, d))
+        v[..., 5] *= np.float32(factor)
+        dv = ctx.upload(v)
+        times.append(median_us(ctx, lambda: ctx.gqa_pv(dp, dv, out)))
+    assert max(times[1:]) <= 2 * times[0], times
