@@ -390,22 +390,6 @@ __global__ __launch_bounds__(256) void k_gqa_pv_mfma(const half_t* __restrict__ 
 
 // ------------------------------------ f32 on the bf16 matrix cores
 
-// Whether the parts of a value (Bf16x3) keep all its bits in any product
-// here: zero, or 2^-40 <= |x| < 2^60 (no part is subnormal, no sum of 2^16
-// products overflows).  `lo` and `hi` gather the least non-zero and the
-// largest magnitude; infinities and NaN are past any bound.
-struct Magnitudes {
-    uint32_t lo = 0xffffffffu, hi = 0u;
-    __device__ inline void add(float x) {
-        const uint32_t b = __float_as_uint(x);
-        lo = min(lo, (b << 1) - 1u);  // zero wraps to the largest
-        hi = max(hi, b & 0x7fffffffu);
-    }
-    __device__ inline bool in_range() const {
-        return lo >= (0x2b800000u << 1) - 1u && hi < 0x5d800000u;  // 2^-40, 2^60
-    }
-};
-
 // QK^T in f32: S = Q K^T per wave (32 queries, 32 keys at a time) with every
 // f32 product made of bf16 parts (v_mfma_f32_32x32x16_bf16).  Workgroup =
 // (head, 128 queries, run of k_per_block tiles of BN keys): the queries are
@@ -413,10 +397,11 @@ struct Magnitudes {
 // into LDS for the four waves (three planes, rows in the chunk order of
 // lds_swizzle) while the next one loads.  With lane = key, register =
 // query a store writes two whole 128-byte row segments, at any row alignment.
-// Bound by the writes of the scores.  A tile with elements outside
-// Magnitudes::in_range is computed by plain dot products.  One MI355X, 9 heads
-// of 64 x [2048, 2048] (151 MB): 70.6 us on v_mfma_f32_32x32x2_f32
-// (whose rate bound it; 16-byte stores of 32 rows at a time), 51.3 us.
+// Where an element of 2^36 or more was met, scores that are not finite
+// (infinities, sums of 2^80 or more) are computed again by plain products.
+// One MI355X, 9 heads of 64 x [2048, 2048] (151 MB): 70.6 us on
+// v_mfma_f32_32x32x2_f32 (whose rate bound it; 16-byte stores of 32 rows at a
+// time), 50.3 us; with a key channel of 1e-12 50.4, with one infinite key 157.
 template <int NT, int BN>
 __global__ __launch_bounds__(256) void k_gqa_qk_bf16x3(const float* __restrict__ q,
                                                        const float* __restrict__ k,
@@ -429,7 +414,6 @@ __global__ __launch_bounds__(256) void k_gqa_qk_bf16x3(const float* __restrict__
     constexpr int LOADS = BN * ROW_CHUNKS / 256;
     constexpr int PLANE = BN * RD;
     __shared__ __align__(16) __bf16 ks[3 * PLANE];
-    __shared__ uint32_t odd_tile;  // the last tile with a key out of range, + 1
     const uint32_t wave = threadIdx.x / 64;
     const uint32_t lane = threadIdx.x % 64;
     const uint32_t col = lane % 32;
@@ -458,29 +442,26 @@ __global__ __launch_bounds__(256) void k_gqa_qk_bf16x3(const float* __restrict__
             kreg[li] = __builtin_shufflevector(x0, x1, 0, 1, 2, 3, 4, 5, 6, 7);
         }
     };
-    auto store_tile = [&](uint32_t t) {
-        Magnitudes mag;
+    float largest = 0.0f;  // magnitude this thread split (NaN aside: its scores are NaN)
+    auto store_tile = [&]() {
 #pragma unroll
         for (int li = 0; li < LOADS; ++li) {
             const uint32_t chunk = threadIdx.x + 256 * li;
             const uint32_t r = chunk / ROW_CHUNKS, ch = chunk % ROW_CHUNKS;
             if (RD > D && ch >= D / 8) continue;
 #pragma unroll
-            for (int e = 0; e < 8; ++e) mag.add(kreg[li][e]);
-            const Bf16x3 x = split_bf16(kreg[li]);
+            for (int e = 0; e < 8; ++e) largest = fmaxf(largest, fabsf(kreg[li][e]));
+            const Bf16x3 x = split_bf16(kreg[li] * kPartScale);
 #pragma unroll
             for (int i = 0; i < 3; ++i)
                 *reinterpret_cast<b8*>(ks + i * PLANE + r * RD + 8 * (ch ^ lds_swizzle<SW>(r))) =
                     x.part[i];
         }
-        if (!mag.in_range()) odd_tile = t + 1;
     };
-    if (threadIdx.x == 0) odd_tile = 0;
     load_tile(t_first);
     // A operand: lane (row col, hs) holds elements 16c + 8hs .. + 7 of its query
     const uint32_t qi = q0 + col;
     const float* qrow = q + (uint64_t(bh) * p.q_len + (qi < p.q_len ? qi : 0)) * D + 8 * hs;
-    Magnitudes qmag;
     Bf16x3 qf[DC];
 #pragma unroll
     for (int c = 0; c < DC; ++c) {
@@ -488,15 +469,13 @@ __global__ __launch_bounds__(256) void k_gqa_qk_bf16x3(const float* __restrict__
         const f32x4 x1 = *reinterpret_cast<const f32x4*>(qrow + 16 * c + 4);
         const f32x8 x = __builtin_shufflevector(x0, x1, 0, 1, 2, 3, 4, 5, 6, 7);
 #pragma unroll
-        for (int e = 0; e < 8; ++e) qmag.add(x[e]);
-        qf[c] = split_bf16(x);
+        for (int e = 0; e < 8; ++e) largest = fmaxf(largest, fabsf(x[e]));
+        qf[c] = split_bf16(x * kPartScale);
     }
-    const bool odd_queries = __any(!qmag.in_range());
     uint32_t koff[DC];
 #pragma unroll
     for (int c = 0; c < DC; ++c) koff[c] = col * RD + 8 * ((2 * c + hs) ^ lds_swizzle<SW>(col));
-    __syncthreads();  // odd_tile is set up
-    store_tile(t_first);
+    store_tile();
     __syncthreads();
 
     float* tile_out = out + (uint64_t(bh) * p.q_len + q0 + 4 * hs) * p.kv_len;
@@ -504,35 +483,23 @@ __global__ __launch_bounds__(256) void k_gqa_qk_bf16x3(const float* __restrict__
     for (uint32_t t = t_first; t < t_end; ++t) {
         if (t + 1 < t_end) load_tile(t + 1);
         if (rows > 0) {
-            const bool plain = odd_queries || odd_tile == t + 1;
 #pragma unroll
             for (int st = 0; st < BN / 32; ++st) {
                 const uint32_t key = t * BN + st * 32 + col;
                 f32x16 s;
 #pragma unroll
                 for (int r = 0; r < 16; ++r) s[r] = 0.0f;
-                if (!plain) {
 #pragma unroll
-                    for (int c = 0; c < DC; ++c) {
-                        Bf16x3 kb;
+                for (int c = 0; c < DC; ++c) {
+                    Bf16x3 kb;
 #pragma unroll
-                        for (int i = 0; i < 3; ++i)
-                            kb.part[i] = *reinterpret_cast<const b8*>(ks + i * PLANE +
-                                                                      st * 32 * RD + koff[c]);
-                        s = mfma_bf16x3(qf[c], kb, s);
-                    }
-                } else {
-                    const float* krow = kh + uint64_t(min(key, p.kv_len - 1)) * D;
-                    for (int d = 0; d < D; ++d) {
-                        const float kd = krow[d];
-#pragma unroll
-                        for (int r = 0; r < 16; ++r) {
-                            const uint32_t row = min(8u * (r / 4) + 4 * hs + r % 4, rows - 1);
-                            s[r] = __builtin_fmaf(
-                                q[(uint64_t(bh) * p.q_len + q0 + row) * D + d], kd, s[r]);
-                        }
-                    }
+                    for (int i = 0; i < 3; ++i)
+                        kb.part[i] =
+                            *reinterpret_cast<const b8*>(ks + i * PLANE + st * 32 * RD + koff[c]);
+                    s = mfma_bf16x3(qf[c], kb, s);
                 }
+#pragma unroll
+                for (int r = 0; r < 16; ++r) s[r] *= kProductUnscale;
                 // register r: query row 8 (r / 4) + 4 hs + r % 4 of the tile
                 if (key < p.kv_len) {
 #pragma unroll
@@ -545,8 +512,35 @@ __global__ __launch_bounds__(256) void k_gqa_qk_bf16x3(const float* __restrict__
             }
         }
         __syncthreads();
-        if (t + 1 < t_end) store_tile(t + 1);
+        if (t + 1 < t_end) store_tile();
         __syncthreads();
+    }
+    // D <= 128 products of elements below 2^36 keep within the scaled range
+    if (!__syncthreads_or(largest >= 0x1p36f)) return;
+    // the wave's scores that are not finite (each lane reads back its own)
+    for (uint32_t key0 = t_first * BN; key0 < min(t_end * BN, p.kv_len); key0 += 32) {
+        const uint32_t key = min(key0 + col, p.kv_len - 1);
+        uint32_t odd = 0;
+#pragma unroll
+        for (int r = 0; r < 16; ++r) {
+            const uint32_t row = 8 * (r / 4) + r % 4;
+            if (row + 4 * hs < rows && !(fabsf(tile_out[uint64_t(row) * p.kv_len + key]) < INFINITY))
+                odd |= 1u << r;
+        }
+        if (!__any(odd != 0)) continue;
+        float s[16] = {};
+#pragma unroll 1
+        for (int d = 0; d < D; ++d) {
+            const float kd = kh[uint64_t(key) * D + d];
+#pragma unroll
+            for (int r = 0; r < 16; ++r) {
+                const uint32_t row = min(8u * (r / 4) + 4 * hs + r % 4, rows - 1);
+                s[r] = __builtin_fmaf(q[(uint64_t(bh) * p.q_len + q0 + row) * D + d], kd, s[r]);
+            }
+        }
+#pragma unroll
+        for (int r = 0; r < 16; ++r)
+            if (odd >> r & 1) tile_out[uint64_t(8 * (r / 4) + r % 4) * p.kv_len + key] = s[r];
     }
 }
 

@@ -647,6 +647,37 @@ def test_gqa_pv_f32_keeps_every_exponent(ctx, hd, ql, kl):
         assert np.all(err <= product_bound(kl, np.abs(pe) @ np.abs(ve)))
 
 
+@pytest.mark.parametrize("hd,ql,kl", [(64, 130, 131), (128, 33, 200), (96, 64, 64), (32, 1, 37)])
+def test_gqa_qk_f32_keeps_every_exponent(ctx, hd, ql, kl):
+    """Queries and keys of every exponent, in rows of their own and mixed: no
+    part of a value is lost, subnormal scores included."""
+    for q, k in ((wide_range(81, (1, 4, ql, hd)), wide_range(82, (1, 2, kl, hd))),
+                 (one_exponent_each(83, (1, 4, ql, hd), -148),
+                  one_exponent_each(84, (1, 2, kl, hd), -148)),
+                 (np.ones((1, 4, ql, hd), np.float32),
+                  np.full((1, 2, kl, hd), 3 * 2.0 ** -140, np.float32))):
+        ctx.begin()
+        got = ctx.gqa_qk(ctx.upload(q), ctx.upload(k))
+        ctx.finish()
+        exact, mag = gqa_exact(q, k, kl)
+        err = np.abs(got.numpy().astype(np.float64) - exact)
+        assert np.all(err <= product_bound(hd, mag))
+
+
+def test_gqa_qk_f32_time_does_not_depend_on_small_values(ctx):
+    """A key channel of 1e-13, one of subnormals and a query row of 1e-30, at
+    the time of ordinary ones."""
+    h, n, d = 9, 1024, 64
+    out, times = ctx.empty((1, h, n, n), np.float32), []
+    for fq, fk in ((1, 1), (1, 1e-13), (1, 1e-38), (1e-30, 1)):
+        q, k = synth.normal(85, (1, h, n, d)), synth.normal(86, (1, 3, n, d))
+        q[:, :, ::32] *= np.float32(fq)
+        k[..., 5] *= np.float32(fk)
+        dq, dk = ctx.upload(q), ctx.upload(k)
+        times.append(median_us(ctx, lambda: ctx.gqa_qk(dq, dk, n, out)))
+    assert max(times[1:]) <= 2 * times[0], times
+
+
 def test_gqa_pv_f32_time_does_not_depend_on_small_values(ctx):
     """A value channel of 1e-12, and one of subnormals, at the time of ordinary
     ones (equal as measured; the bound allows for a shared machine)."""
