@@ -133,53 +133,90 @@ constexpr float kRescaleSlack = 3.0f;
 // 1: 49.0 / 50.0 us for the latter, 32 of 128 x 900 after 4000 88.9 / 91.3.
 constexpr float kFarSlack = 1.0f;
 
-// One query row by one wave with plain f32 products, as k_attention_rows
-// computes it: for rows whose output the split products leave non-finite
-// (inf - inf and 0 * inf between the parts of an infinite operand or value),
-// so that infinities and NaN come out as in unsplit arithmetic.  Lane = key
-// for the scores, lane = head elements lane + 64 t for the values; no LDS.
-// D <= 32 NT.
+// The query rows of `redo` (a bit each, of the 32 from `q` on) by one wave
+// with plain f32 products, as k_attention_rows computes them: for rows whose
+// output the split products leave non-finite (inf - inf and 0 * inf between
+// the parts of an infinite operand or value), so that infinities and NaN come
+// out as in unsplit arithmetic.  Eight rows at a time, which share every read
+// of K and V; lane = key for the scores, lane = head elements lane + 64 t for
+// the values; no LDS.  D <= 32 NT, a multiple of 8, rows on the 16-byte grid;
+// row c sees `keys` + c keys, at most kv_len.  One MI355X, 9 heads of 64 x [2048,
+// 2048] f32 with an infinite value row in each KV head, so in nearly every
+// query's sum: 2.08 ms, 7.84 a row at a time (68.6 us with none).
 template <typename T, int NT>
-__device__ inline void exact_row(const T* __restrict__ qrow, const T* __restrict__ kh,
-                                 const T* __restrict__ vh, T* __restrict__ orow, uint32_t D,
-                                 uint32_t key_end, float scale) {
+__device__ inline void exact_rows(uint32_t redo, const T* __restrict__ q,
+                                  const T* __restrict__ kh, const T* __restrict__ vh,
+                                  T* __restrict__ out, uint32_t D, uint64_t keys, uint32_t kv_len,
+                                  float scale) {
     constexpr int DT = (NT + 1) / 2;
+    constexpr int R = 8;
+    typedef T t4 __attribute__((ext_vector_type(4)));
     const uint32_t lane = threadIdx.x % 64;
-    float o[DT];
+    while (redo != 0) {
+        uint32_t row[R], key_end[R];  // ascending; a short last group repeats its first row
+        uint32_t last = 0;
+        float m[R], l[R], o[R][DT];
 #pragma unroll
-    for (int t = 0; t < DT; ++t) o[t] = 0.0f;
-    float m = -INFINITY, l = 0.0f;
-    for (uint32_t base = 0; base < key_end; base += 64) {
-        float s = -INFINITY;
-        if (base + lane < key_end) {
-            const T* krow = kh + uint64_t(base + lane) * D;
-            float dot = 0.0f;
-            for (uint32_t d = 0; d < D; ++d) dot += to_float(qrow[d]) * to_float(krow[d]);
-            s = dot * scale;
+        for (int i = 0; i < R; ++i) {
+            row[i] = redo != 0 ? uint32_t(__builtin_ctz(redo)) : row[0];
+            redo &= redo - 1;
+            key_end[i] = uint32_t(min(uint64_t(kv_len), keys + row[i]));
+            last = max(last, key_end[i]);
+            m[i] = -INFINITY;
+            l[i] = 0.0f;
+#pragma unroll
+            for (int t = 0; t < DT; ++t) o[i][t] = 0.0f;
         }
-        const float m_new = fmaxf(m, wave_max_dpp(s));
-        const float alpha = m_new > m ? exp_fast(m - m_new) : 1.0f;
-        m = m_new;
-        const float e = s == -INFINITY ? 0.0f : exp_fast(s - m);
-        l = l * alpha + e;
+        for (uint32_t base = 0; base < last; base += 64) {
+            const T* krow = kh + uint64_t(min(base + lane, kv_len - 1)) * D;
+            float e[R];
 #pragma unroll
-        for (int t = 0; t < DT; ++t) o[t] *= alpha;
-        const uint32_t n = min(64u, key_end - base);
-        for (uint32_t j = 0; j < n; ++j) {
-            const float pj = __shfl(e, int(j), 64);
-            const T* vrow = vh + uint64_t(base + j) * D;
+            for (int i = 0; i < R; ++i) e[i] = 0.0f;
+            for (uint32_t d = 0; d < D; d += 4) {
+                const t4 kd = *reinterpret_cast<const t4*>(krow + d);
 #pragma unroll
-            for (int t = 0; t < DT; ++t) {
-                const uint32_t d = lane + 64 * t;
-                if (d < D) o[t] += pj * to_float(vrow[d]);
+                for (int i = 0; i < R; ++i) {
+                    const t4 qd = *reinterpret_cast<const t4*>(q + uint64_t(row[i]) * D + d);
+#pragma unroll
+                    for (int j = 0; j < 4; ++j) e[i] += to_float(T(qd[j])) * to_float(T(kd[j]));
+                }
+            }
+#pragma unroll
+            for (int i = 0; i < R; ++i) {
+                const float s = base + lane < key_end[i] ? e[i] * scale : -INFINITY;
+                const float m_new = fmaxf(m[i], wave_max_dpp(s));
+                const float alpha = m_new > m[i] ? exp_fast(m[i] - m_new) : 1.0f;
+                m[i] = m_new;
+                e[i] = s == -INFINITY ? 0.0f : exp_fast(s - m_new);
+                l[i] = l[i] * alpha + e[i];
+#pragma unroll
+                for (int t = 0; t < DT; ++t) o[i][t] *= alpha;
+            }
+            const uint32_t n = min(64u, last - base);
+            for (uint32_t j = 0; j < n; ++j) {
+                const T* vrow = vh + uint64_t(base + j) * D;
+                float x[DT];
+#pragma unroll
+                for (int t = 0; t < DT; ++t)
+                    x[t] = lane + 64 * t < D ? to_float(vrow[lane + 64 * t]) : 0.0f;
+#pragma unroll
+                for (int i = 0; i < R; ++i) {
+                    const float pj = __int_as_float(
+                        __builtin_amdgcn_readlane(__float_as_int(e[i]), int(j)));
+#pragma unroll
+                    for (int t = 0; t < DT; ++t)  // a key behind the row adds nothing, whatever it holds
+                        o[i][t] += base + j < key_end[i] ? pj * x[t] : 0.0f;
+                }
             }
         }
-    }
-    const float inv = 1.0f / wave_sum_dpp(l);
 #pragma unroll
-    for (int t = 0; t < DT; ++t) {
-        const uint32_t d = lane + 64 * t;
-        if (d < D) orow[d] = from_float<T>(o[t] * inv);
+        for (int i = 0; i < R; ++i) {
+            const float inv = 1.0f / wave_sum_dpp(l[i]);
+            T* orow = out + uint64_t(row[i]) * D;
+#pragma unroll
+            for (int t = 0; t < DT; ++t)
+                if (lane + 64 * t < D) orow[lane + 64 * t] = from_float<T>(o[i][t] * inv);
+        }
     }
 }
 
@@ -208,7 +245,7 @@ constexpr float kAnyShift = 12.0f;
 // -- 22 bits, and the factor 2^12 (kAnyShift), which cancels in the division
 // by the sum, keeps lo's own bits above the f16 subnormals down to
 // probabilities of 2^-15 of the largest.  A query whose output is not finite
-// is computed again by exact_row, whose products are not split.  One MI355X,
+// is computed again by exact_rows, whose products are not split.  One MI355X,
 // 8 heads x [1021, 1021], head size 80: 475 us on k_attention_rows (a dot
 // product a lane on the vector ALUs, uncoalesced key rows), 24.4 us here; 32
 // heads x [4096, 4096]: 12.0 ms, 0.18 ms; head size 256, 8 heads x [570, 570]:
@@ -559,17 +596,12 @@ __global__ __launch_bounds__(64 * QW * KSPLIT) void k_flash_attention(
                 }
             }
             if constexpr (ANY) {
-                // queries with an output that is not finite, in turn, by the
-                // whole wave (after its stores above: same wave, in order)
-                uint64_t redo = __ballot(!finite);
-                redo = (redo | redo >> 32) & 0xffffffffu;
-                while (redo != 0) {
-                    const uint32_t c = __builtin_ctzll(redo);
-                    redo &= redo - 1;
-                    const uint64_t row = uint64_t(bh) * p.q_len + qw0 + c;
-                    exact_row<half_t, NT>(q + row * hd, kh, vh, out + row * hd, hd,
-                                          min(p.kv_len, p.start + qw0 + c + 1), p.scale);
-                }
+                // queries with an output that is not finite, by the whole
+                // wave (after its stores above: same wave, in order)
+                const uint64_t redo = __ballot(!finite);
+                const uint64_t first = (uint64_t(bh) * p.q_len + qw0) * hd;
+                exact_rows<half_t, NT>(uint32_t(redo | redo >> 32), q + first, kh, vh, out + first,
+                                       hd, uint64_t(p.start) + qw0 + 1, p.kv_len, p.scale);
             }
         }
     }
@@ -639,10 +671,13 @@ __global__ __launch_bounds__(256) void k_flash_combine(half_t* __restrict__ out,
 // probabilities are split 16 keys at a time.  Scores, probabilities and sums
 // are f32 throughout.  Two LDS stages where they fit (a step's block is split
 // and stored before the previous one's products, one barrier a step), else one.
-// A query whose output is not finite, or has an element too small for its
-// values' low parts (the matrix cores take bf16 subnormals as zero), is
-// computed again unsplit (exact_row), and so is a query with elements outside
-// 2^-64 .. 2^64, so that the parts lost from a score are below 2^-61 of one.
+// Queries, probabilities and values are scaled (kPartScale), so that no part
+// of theirs is lost; of a key only what is below 2^-126, which changes a score
+// by less than 2^-59 while query elements are below 2^60.  Other queries are
+// computed again unsplit (exact_rows), and so are those whose output is not finite
+// (infinities, NaN, sums of 2^80 or more).  (A score whose partial sums pass -2^104
+// counts as -inf, far inside the f32 rounding of its terms where use_flash
+// lets the scale in.)
 // Bound by matrix and vector work in turn (they do not overlap: 35 % matrix,
 // 34 % vector, ~19 vector operations a score, at 69 % balance of the tiles
 // over the CUs).  One MI355X against v_mfma_f32_32x32x2_f32 in the same
@@ -682,6 +717,7 @@ __global__ __launch_bounds__(64 * QW * KSPLIT) void k_flash_attention_bf16x3(
     __shared__ __align__(16) unsigned char lds[LDS_BYTES];
     __bf16* const kv_lds = reinterpret_cast<__bf16*>(lds);
 
+    const float scale_log2 = p.scale_log2 / kPartScale;  // of the scores, their queries scaled
     const bool by_tile = p.pairs == p.tiles;  // as in k_flash_attention
     const uint32_t per = by_tile ? p.heads : p.pairs;
     const uint32_t major = blockIdx.x / per, minor = blockIdx.x - major * per;
@@ -767,7 +803,7 @@ __global__ __launch_bounds__(64 * QW * KSPLIT) void k_flash_attention_bf16x3(
                 const bool live = (step * KSPLIT + share) * BN + r < p.kv_len;
                 f32x8 vx = vreg[li];
 #pragma unroll
-                for (int e = 0; e < 8; ++e) vx[e] = live ? vx[e] : 0.0f;
+                for (int e = 0; e < 8; ++e) vx[e] = live ? vx[e] * kPartScale : 0.0f;
                 const Bf16x3 kp = split_bf16(kreg[li]), vp = split_bf16(vx);
 #pragma unroll
                 for (int i = 0; i < 3; ++i) {
@@ -788,7 +824,7 @@ __global__ __launch_bounds__(64 * QW * KSPLIT) void k_flash_attention_bf16x3(
             const f32x4 x1 = *reinterpret_cast<const f32x4*>(qrow + 16 * c + 4);
             f32x8 x = __builtin_shufflevector(x0, x1, 0, 1, 2, 3, 4, 5, 6, 7);
 #pragma unroll
-            for (int e = 0; e < 8; ++e) x[e] = q_valid ? x[e] : 0.0f;
+            for (int e = 0; e < 8; ++e) x[e] = q_valid ? x[e] * kPartScale : 0.0f;
             qf[c] = split_bf16(x);
         }
         f32x16 o[NT], low[APART ? NT : 1];
@@ -843,12 +879,6 @@ __global__ __launch_bounds__(64 * QW * KSPLIT) void k_flash_attention_bf16x3(
                         for (int r = 0; r < 16; ++r)
                             if (kt * 32 + 16 * (r >> 3) + (r & 7) > lim) s[kt][r] = -INFINITY;
                 }
-                // scores in log2 units first, so that the largest one's
-                // probability is exactly 1 (2^(t - m) with t == m)
-#pragma unroll
-                for (int kt = 0; kt < KT; ++kt)
-#pragma unroll
-                    for (int r = 0; r < 16; ++r) s[kt][r] *= p.scale_log2;
                 float mx = -INFINITY, my = -INFINITY;
 #pragma unroll
                 for (int kt = 0; kt < KT; ++kt)
@@ -858,10 +888,11 @@ __global__ __launch_bounds__(64 * QW * KSPLIT) void k_flash_attention_bf16x3(
                         my = max3(my, s[kt][r + 2], s[kt][r + 3]);
                     }
                 mx = fmaxf(mx, my);
-                const float mx_log2 = max_halves(mx);
-                if (__any(mx_log2 > m + kRescaleSlack)) {
-                    const float m_new = fmaxf(m, mx_log2);
-                    const float alpha = m_new > m ? __builtin_amdgcn_exp2f(m - m_new) : 1.0f;
+                mx = max_halves(mx);
+                if (__any((mx - m) * scale_log2 > kRescaleSlack)) {
+                    const float m_new = fmaxf(m, mx);
+                    const float alpha =
+                        m_new > m ? __builtin_amdgcn_exp2f((m - m_new) * scale_log2) : 1.0f;
                     m = m_new;
                     l *= alpha;
 #pragma unroll
@@ -872,21 +903,24 @@ __global__ __launch_bounds__(64 * QW * KSPLIT) void k_flash_attention_bf16x3(
                             if constexpr (APART) low[t][r] *= alpha;
                         }
                 }
-                // p = 2^(t - m); a query that has seen no key yet (m = -inf)
-                // has only -inf scores, and p = 0
-                const float neg_m = m == -INFINITY ? 0.0f : -m;
+                // p = 2^((s - m) scale_log2), so that the largest score's is exactly
+                // 1; a query that has seen no key yet (m = -inf) has only -inf
+                // scores, and p = 0
+                const float mm = m == -INFINITY ? 0.0f : m;
                 float la = 0.0f, lb = 0.0f;
 #pragma unroll
                 for (int c = 0; c < BN / 16; ++c) {
                     f32x8 x;
 #pragma unroll
                     for (int e = 0; e < 8; e += 2) {
-                        x[e] = __builtin_amdgcn_exp2f(s[c >> 1][8 * (c & 1) + e] + neg_m);
-                        x[e + 1] = __builtin_amdgcn_exp2f(s[c >> 1][8 * (c & 1) + e + 1] + neg_m);
+                        x[e] = __builtin_amdgcn_exp2f((s[c >> 1][8 * (c & 1) + e] - mm) *
+                                                      scale_log2);
+                        x[e + 1] = __builtin_amdgcn_exp2f((s[c >> 1][8 * (c & 1) + e + 1] - mm) *
+                                                          scale_log2);
                         la += x[e];
                         lb += x[e + 1];
                     }
-                    const Bf16x3 pb = split_bf16(x);
+                    const Bf16x3 pb = split_bf16(x * kPartScale);
                     // O^T += V^T P^T over these 16 keys
 #pragma unroll
                     for (int t = 0; t < NT; ++t) {
@@ -943,8 +977,10 @@ __global__ __launch_bounds__(64 * QW * KSPLIT) void k_flash_attention_bf16x3(
                     const float* src = mg + ((h - 1) * QW * 64 + qw * 64 + lane) * MERGE;
                     const float m2 = src[0];
                     const float m_tot = fmaxf(m, m2);
-                    const float a1 = m_tot > m ? __builtin_amdgcn_exp2f(m - m_tot) : 1.0f;
-                    const float a2 = m_tot > m2 ? __builtin_amdgcn_exp2f(m2 - m_tot) : 1.0f;
+                    const float a1 =
+                        m_tot > m ? __builtin_amdgcn_exp2f((m - m_tot) * scale_log2) : 1.0f;
+                    const float a2 =
+                        m_tot > m2 ? __builtin_amdgcn_exp2f((m2 - m_tot) * scale_log2) : 1.0f;
                     l = l * a1 + src[1] * a2;
 #pragma unroll
                     for (int t = 0; t < NT; ++t)
@@ -958,18 +994,17 @@ __global__ __launch_bounds__(64 * QW * KSPLIT) void k_flash_attention_bf16x3(
         }
 
         if (sub == 0) {
-            const float inv = 1.0f / (l + __shfl_xor(l, 32, 64));  // both halves of the query
-            bool exact = false;  // this lane's half of a query needs exact_row
+            const float inv =  // both halves of the query
+                kProductUnscale / (l + __shfl_xor(l, 32, 64));
+            bool exact = false;  // this lane's half of a query needs exact_rows
             if (q_valid) {
+                float odd = 0.0f;  // the largest query element, then NaN if an output is not finite
 #pragma unroll
                 for (int c = 0; c < DC; ++c)
 #pragma unroll
-                    for (int e = 0; e < 8; ++e) {
-                        const float a = fabsf(qrow[16 * c + e]);
-                        exact |= a != 0.0f && !(a > 0x1p-64f && a < 0x1p64f);
-                    }
-            }
-            if (q_valid) {
+                    for (int e = 0; e < 8; ++e) odd = fmaxf(odd, fabsf(qrow[16 * c + e]));
+                exact = odd >= 0x1p60f;
+                odd = 0.0f;
                 // register r of tile t: element 32t + 8(r / 4) + 4hs + r % 4
                 float* orow = out + (uint64_t(bh) * p.q_len + qi) * D + 4 * hs;
 #pragma unroll
@@ -980,21 +1015,16 @@ __global__ __launch_bounds__(64 * QW * KSPLIT) void k_flash_attention_bf16x3(
 #pragma unroll
                         for (int e = 0; e < 4; ++e) {
                             w[e] = o[t][4 * g + e] * inv;
-                            const float a = fabsf(w[e]);
-                            exact |= a != 0.0f && !(a > 0x1p-96f && a < INFINITY);
+                            odd = __builtin_fmaf(w[e], 0.0f, odd);
                         }
                         *reinterpret_cast<f32x4*>(orow + 32 * t + 8 * g) = w;
                     }
+                exact |= odd != 0.0f;
             }
-            uint64_t redo = __ballot(exact);
-            redo = (redo | redo >> 32) & 0xffffffffu;
-            while (redo != 0) {
-                const uint32_t c = __builtin_ctzll(redo);
-                redo &= redo - 1;
-                const uint64_t row = uint64_t(bh) * p.q_len + qw0 + c;
-                exact_row<float, NT>(q + row * D, kh, vh, out + row * D, D,
-                                     min(p.kv_len, p.start + qw0 + c + 1), p.scale);
-            }
+            const uint64_t redo = __ballot(exact);
+            const uint64_t first = (uint64_t(bh) * p.q_len + qw0) * D;
+            exact_rows<float, NT>(uint32_t(redo | redo >> 32), q + first, kh, vh, out + first, D,
+                                  uint64_t(p.start) + qw0 + 1, p.kv_len, p.scale);
         }
     }
 }
@@ -1919,7 +1949,8 @@ rl_status launch_flash_any(rl_context* ctx, uint64_t heads, const half_t* q, con
 // Which kernel a shape takes: the MFMA kernels for a head size of 32, 64,
 // 96 or 128 and 16-byte aligned buffers (f16: also byte offsets into one KV
 // head, a block past its end included, that fit the 32-bit buffer offsets
-// of its loads); in f16 the padded matrix-core kernel (ANY) for the other
+// of its loads; f32: a scale of 2^-60 or more, below which scores that leave the
+// scaled range of its products could still matter); in f16 the padded matrix-core kernel (ANY) for the other
 // multiples of 8 up to 256 (rows of whole 16-byte pieces); the row kernel
 // otherwise (head sizes up to 512).
 bool use_flash_any(const AttnShape& s, const void* q, const void* k, const void* v,
@@ -1930,11 +1961,12 @@ bool use_flash_any(const AttnShape& s, const void* q, const void* k, const void*
            aligned_to(q, 16) && aligned_to(k, 16) && aligned_to(v, 16) && aligned_to(o, 16);
 }
 template <typename T>
-bool use_flash(const AttnShape& s, const void* q, const void* k, const void* v, const void* o) {
+bool use_flash(const AttnShape& s, float scale, const void* q, const void* k, const void* v,
+               const void* o) {
     const bool shape = s.head_dim % 32 == 0 && s.head_dim <= 128 && aligned_to(q, 16) &&
                        aligned_to(k, 16) && aligned_to(v, 16) && aligned_to(o, 16);
     if constexpr (!std::is_same<T, half_t>::value) {
-        return shape;
+        return shape && scale >= 0x1p-60f;
     } else {
         const uint64_t span = (s.kv_len + uint64_t(kFlashMaxBlockKeys) * kFlashMaxKeySplit) *
                               s.head_dim * sizeof(T);
@@ -2035,7 +2067,7 @@ rl_status attention_entry(rl_context* ctx, const char* name, const rl_buffer* q,
                           DecodeScratch mode = DecodeScratch::kPool) {
     if (rl_status st = validate_attention(q, k, v, s, scale, start, sizeof(T))) return st;
     if (rl_status st = check_output(out, q->len, sizeof(T), "attention")) return st;
-    const bool flash = use_flash<T>(s, q->data, k->data, v->data, out->data);
+    const bool flash = use_flash<T>(s, scale, q->data, k->data, v->data, out->data);
     if (!flash && s.head_dim > 512)
         return fail(RL_ERR_INVALID_SHAPE, "attention head size %llu exceeds 512",
                     (unsigned long long)s.head_dim);

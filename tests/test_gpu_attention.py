@@ -691,3 +691,38 @@ def test_gqa_pv_f32_time_does_not_depend_on_small_values(ctx):
         dv = ctx.upload(v)
         times.append(median_us(ctx, lambda: ctx.gqa_pv(dp, dv, out)))
     assert max(times[1:]) <= 2 * times[0], times
+
+
+@pytest.mark.parametrize("hd,ql", [(64, 33), (64, 300), (32, 3), (128, 70), (96, 17)])
+def test_attention_f32_improbable_large_values(ctx, hd, ql):
+    """Outputs that are one improbable key's value: probabilities of 2^-112 to
+    2^-125 keep all their bits.  The exponent t, from one product of the scale and
+    log2 e and one of that and the score, is off by at most |t| 2^-23; the rest
+    of the path by a few roundings."""
+    n, kl = 14, 150 + ql
+    q = np.zeros((1, 2, ql, hd), np.float32)
+    q[..., 0] = 1
+    t = np.arange(112, 112 + n)
+    k = np.zeros((1, 1, kl, hd), np.float32)
+    k[0, 0, 20:20 + n, 0] = -t * np.log(2.0) * 4
+    v = np.zeros((1, 1, kl, hd), np.float32)
+    v[0, 0, 20 + np.arange(n), np.arange(n)] = 2.0 ** 40 / 3
+    got = run_attention(ctx, q, k, v, 0.25, 150, kl).astype(np.float64)[..., :n]
+    exact, _, _ = attention_exact(q, k, v, 0.25, 150, kl)
+    assert np.all(np.abs(got / exact[..., :n] - 1) <= t * 2.0 ** -23 + 16 * U32)
+
+
+def test_attention_f32_time_does_not_depend_on_small_values(ctx):
+    """Value and key channels of 1e-12, 1e-30 and subnormals and queries of 1e-25,
+    at the time of ordinary ones."""
+    h, n, d = 9, 1024, 64
+    out, times = ctx.empty((1, h, n, d), np.float32), []
+    for fq, fkv in ((1, 1), (1, 1e-12), (1, 1e-30), (1, 1e-38), (1e-25, 1)):
+        q = synth.normal(91, (1, h, n, d))
+        k, v = synth.normal(92, (1, 3, n, d)), synth.normal(93, (1, 3, n, d))
+        q[:, :, ::32] *= np.float32(fq)
+        k[..., 5] *= np.float32(fkv)
+        v[..., 5] *= np.float32(fkv)
+        dq, dk, dv = ctx.upload(q), ctx.upload(k), ctx.upload(v)
+        times.append(median_us(ctx, lambda: ctx.attention(dq, dk, dv, 0.125, 0, n, out)))
+    assert max(times[1:]) <= 2 * times[0], times
