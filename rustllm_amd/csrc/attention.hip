@@ -697,19 +697,25 @@ __global__ __launch_bounds__(64 * QW * KSPLIT) void k_flash_attention_bf16x3(
     constexpr int RD = NT == 3 ? 128 : D;  // elements of an LDS row
     constexpr int SW = RD / 32;            // its chunk order (lds_swizzle)
     constexpr int THREADS = 64 * QW * KSPLIT;
+    // OWN (32-query tiles): no two waves read the same keys, so K goes from
+    // memory into operand registers and only V, for its transpose, through LDS.
+    constexpr bool OWN = QW == 1;
+    static_assert(!OWN || BN == 32, "one key tile a block");
     constexpr int TILE_Q = 32 * QW;
     constexpr int ROW_CHUNKS = RD / 8;     // 8-element chunks of a row
     constexpr int BLOCK_CHUNKS = BN * ROW_CHUNKS;
     constexpr int LOADS = BLOCK_CHUNKS * KSPLIT / THREADS;
     constexpr int PLANE = BN * RD;         // one part of a K or V block
-    constexpr int STAGE = KSPLIT * 6 * PLANE;
-    constexpr int NSTAGE = 2 * STAGE * 2 <= 128 * 1024 ? 2 : 1;
+    constexpr int PLANES = OWN ? 3 : 6;    // of a block in LDS
+    constexpr int STAGE = KSPLIT * PLANES * PLANE;
+    constexpr int NSTAGE = OWN ? 1 : 2 * STAGE * 2 <= 128 * 1024 ? 2 : 1;
     constexpr int MERGE = NT * 16 + 2;     // floats a lane hands over
     // Four waves have the registers to sum the smaller products apart, one
     // rounding of the large sum a slice instead of six: with two key shares
     // the chains are long (32 heads of 128 x 500 queries after 2500 keys, error
     // against 64 bits: 6.7e-7 in one chain, 4.1e-7 apart; f32 products 6.3e-7).
-    constexpr bool APART = QW * KSPLIT == 4;
+    // OWN, whose registers hold K as well, sums each block's products apart.
+    constexpr bool APART = QW * KSPLIT == 4 && !OWN;
     constexpr int LDS_BYTES = NSTAGE * STAGE * 2 > (KSPLIT - 1) * QW * 64 * MERGE * 4
                                   ? NSTAGE * STAGE * 2
                                   : (KSPLIT - 1) * QW * 64 * MERGE * 4;
@@ -768,21 +774,34 @@ __global__ __launch_bounds__(64 * QW * KSPLIT) void k_flash_attention_bf16x3(
         // 8 consecutive elements of a row per chunk; rows past kv_len are not
         // read (they may hold anything): a key past the end loads row
         // kv_len - 1, its score is masked and its value row zeroed
-        f32x8 kreg[LOADS], vreg[LOADS];
+        f32x8 kreg[OWN ? DC : LOADS], vreg[LOADS];
+        auto load_k = [&](uint32_t step) {  // OWN: this lane's operand elements
+            const uint32_t key = (step * KSPLIT + sub) * BN + perm32(col);
+            const float* src = kh + uint64_t(min(key, p.kv_len - 1)) * D + 8 * hs;
+#pragma unroll
+            for (int c = 0; c < DC; ++c) {
+                const f32x4 k0 = *reinterpret_cast<const f32x4*>(src + 16 * c);
+                const f32x4 k1 = *reinterpret_cast<const f32x4*>(src + 16 * c + 4);
+                kreg[c] = __builtin_shufflevector(k0, k1, 0, 1, 2, 3, 4, 5, 6, 7);
+            }
+        };
         auto load_step = [&](uint32_t step) {
 #pragma unroll
             for (int li = 0; li < LOADS; ++li) {
-                const uint32_t chunk = threadIdx.x + THREADS * li;
+                const uint32_t chunk =
+                    OWN ? sub * BLOCK_CHUNKS + lane + 64 * li : threadIdx.x + THREADS * li;
                 const uint32_t c = chunk % BLOCK_CHUNKS;
                 const uint32_t key = (step * KSPLIT + chunk / BLOCK_CHUNKS) * BN + c / ROW_CHUNKS;
                 const uint32_t ch = c % ROW_CHUNKS;
                 if (RD > D && ch >= D / 8) continue;  // head size 96: 12 of 16 chunks
                 const uint64_t at = uint64_t(min(key, p.kv_len - 1)) * D + ch * 8;
-                const f32x4 k0 = *reinterpret_cast<const f32x4*>(kh + at);
-                const f32x4 k1 = *reinterpret_cast<const f32x4*>(kh + at + 4);
+                if constexpr (!OWN) {
+                    const f32x4 k0 = *reinterpret_cast<const f32x4*>(kh + at);
+                    const f32x4 k1 = *reinterpret_cast<const f32x4*>(kh + at + 4);
+                    kreg[li] = __builtin_shufflevector(k0, k1, 0, 1, 2, 3, 4, 5, 6, 7);
+                }
                 const f32x4 v0 = *reinterpret_cast<const f32x4*>(vh + at);
                 const f32x4 v1 = *reinterpret_cast<const f32x4*>(vh + at + 4);
-                kreg[li] = __builtin_shufflevector(k0, k1, 0, 1, 2, 3, 4, 5, 6, 7);
                 vreg[li] = __builtin_shufflevector(v0, v1, 0, 1, 2, 3, 4, 5, 6, 7);
             }
         };
@@ -790,13 +809,14 @@ __global__ __launch_bounds__(64 * QW * KSPLIT) void k_flash_attention_bf16x3(
             __bf16* stage = kv_lds + (step % NSTAGE) * STAGE;
 #pragma unroll
             for (int li = 0; li < LOADS; ++li) {
-                const uint32_t chunk = threadIdx.x + THREADS * li;
+                const uint32_t chunk =
+                    OWN ? sub * BLOCK_CHUNKS + lane + 64 * li : threadIdx.x + THREADS * li;
                 const uint32_t c = chunk % BLOCK_CHUNKS;
                 const uint32_t share = chunk / BLOCK_CHUNKS;
                 const uint32_t r = c / ROW_CHUNKS, ch = c % ROW_CHUNKS;
                 if (RD > D && ch >= D / 8) continue;
-                __bf16* ks = stage + share * 6 * PLANE;
-                __bf16* vs = ks + 3 * PLANE;
+                __bf16* vs = stage + share * PLANES * PLANE;
+                __bf16* ks = vs + 3 * PLANE;
                 const uint32_t kr = (r & ~31u) | perm32(r & 31u);
                 const uint32_t kat = kr * RD + 8 * (ch ^ lds_swizzle<SW>(kr));
                 const uint32_t vat = r * RD + 8 * (ch ^ lds_swizzle<SW>(r));
@@ -804,15 +824,20 @@ __global__ __launch_bounds__(64 * QW * KSPLIT) void k_flash_attention_bf16x3(
                 f32x8 vx = vreg[li];
 #pragma unroll
                 for (int e = 0; e < 8; ++e) vx[e] = live ? vx[e] * kPartScale : 0.0f;
-                const Bf16x3 kp = split_bf16(kreg[li]), vp = split_bf16(vx);
+                const Bf16x3 vp = split_bf16(vx);
 #pragma unroll
-                for (int i = 0; i < 3; ++i) {
-                    *reinterpret_cast<b8*>(ks + i * PLANE + kat) = kp.part[i];
+                for (int i = 0; i < 3; ++i)
                     *reinterpret_cast<b8*>(vs + i * PLANE + vat) = vp.part[i];
+                if constexpr (!OWN) {
+                    const Bf16x3 kp = split_bf16(kreg[li]);
+#pragma unroll
+                    for (int i = 0; i < 3; ++i)
+                        *reinterpret_cast<b8*>(ks + i * PLANE + kat) = kp.part[i];
                 }
             }
         };
         load_step(0);
+        if constexpr (OWN) load_k(0);
 
         // B operand of S^T = K Q^T: lane (col, hs) holds elements
         // 16c + 8hs .. + 7 of its query for every slice c
@@ -837,11 +862,19 @@ __global__ __launch_bounds__(64 * QW * KSPLIT) void k_flash_attention_bf16x3(
             }
         float m = -INFINITY, l = 0.0f;
 
-        store_step(0);  // the previous tile's LDS use ended with a barrier
-        if (NSTAGE == 2 && steps > 1) load_step(1);
-        __syncthreads();
+        if constexpr (!OWN) {
+            store_step(0);  // the previous tile's LDS use ended with a barrier
+            if (NSTAGE == 2 && steps > 1) load_step(1);
+            __syncthreads();
+        }
         for (uint32_t step = 0; step < steps; ++step) {
-            if constexpr (NSTAGE == 2) {
+            if constexpr (OWN) {
+                // the wave's own rows in LDS: ordered within it, no barrier
+                __builtin_amdgcn_fence(__ATOMIC_ACQ_REL, "wavefront");
+                store_step(step);
+                __builtin_amdgcn_fence(__ATOMIC_ACQ_REL, "wavefront");
+                if (step + 1 < steps) load_step(step + 1);
+            } else if constexpr (NSTAGE == 2) {
                 if (step + 1 < steps) {
                     store_step(step + 1);
                     if (step + 2 < steps) load_step(step + 2);
@@ -850,8 +883,8 @@ __global__ __launch_bounds__(64 * QW * KSPLIT) void k_flash_attention_bf16x3(
                 if (step + 1 < steps) load_step(step + 1);
             }
             const uint32_t blk = step * KSPLIT + sub;
-            const __bf16* ks = kv_lds + (step % NSTAGE) * STAGE + sub * 6 * PLANE;
-            const __bf16* vs = ks + 3 * PLANE;
+            const __bf16* vs = kv_lds + (step % NSTAGE) * STAGE + sub * PLANES * PLANE;
+            const __bf16* ks = vs + 3 * PLANE;
             if (blk < blocks && blk * BN < wave_keys) {
                 f32x16 s[KT];
 #pragma unroll
@@ -861,13 +894,19 @@ __global__ __launch_bounds__(64 * QW * KSPLIT) void k_flash_attention_bf16x3(
 #pragma unroll
                     for (int c = 0; c < DC; ++c) {
                         Bf16x3 ka;
+                        if constexpr (OWN) {
+                            ka = split_bf16(kreg[c]);
+                        } else {
 #pragma unroll
-                        for (int i = 0; i < 3; ++i)
-                            ka.part[i] = *reinterpret_cast<const b8*>(ks + i * PLANE +
-                                                                      kt * 32 * RD + koff[c]);
+                            for (int i = 0; i < 3; ++i)
+                                ka.part[i] = *reinterpret_cast<const b8*>(
+                                    ks + i * PLANE + kt * 32 * RD + koff[c]);
+                        }
                         s[kt] = mfma_bf16x3(ka, qf[c], s[kt]);
                     }
                 }
+                if constexpr (OWN)
+                    if (step + 1 < steps) load_k(step + 1);
                 // register r of tile kt holds key
                 // kbase + 32 kt + 16 (r / 8) + 8 hs + r % 8
                 const uint32_t kbase = blk * BN;
@@ -908,8 +947,7 @@ __global__ __launch_bounds__(64 * QW * KSPLIT) void k_flash_attention_bf16x3(
                 // scores, and p = 0
                 const float mm = m == -INFINITY ? 0.0f : m;
                 float la = 0.0f, lb = 0.0f;
-#pragma unroll
-                for (int c = 0; c < BN / 16; ++c) {
+                auto split_p = [&](int c) {  // the probabilities of keys 16 c .. + 15
                     f32x8 x;
 #pragma unroll
                     for (int e = 0; e < 8; e += 2) {
@@ -920,33 +958,55 @@ __global__ __launch_bounds__(64 * QW * KSPLIT) void k_flash_attention_bf16x3(
                         la += x[e];
                         lb += x[e + 1];
                     }
-                    const Bf16x3 pb = split_bf16(x * kPartScale);
-                    // O^T += V^T P^T over these 16 keys
+                    return split_bf16(x * kPartScale);
+                };
+                auto read_v = [&](int c, int t) {  // V^T of those keys, elements 32 t .. + 31
+                    Bf16x3 va;
+#pragma unroll
+                    for (int i = 0; i < 3; ++i) {
+                        const half_t* plane =
+                            reinterpret_cast<const half_t*>(vs + i * PLANE + 16 * c * RD);
+                        const h4 lo = lds_read_transposed(plane + voff[0][t]);
+                        const h4 hi = lds_read_transposed(plane + voff[1][t]);
+                        const h8 w = {lo[0], lo[1], lo[2], lo[3], hi[0], hi[1], hi[2], hi[3]};
+                        va.part[i] = __builtin_bit_cast(b8, w);
+                    }
+                    return va;
+                };
+                // O^T += V^T P^T
+                if constexpr (OWN) {
+                    const Bf16x3 p0 = split_p(0), p1 = split_p(1);
 #pragma unroll
                     for (int t = 0; t < NT; ++t) {
-                        Bf16x3 va;
+                        f32x16 acc;
 #pragma unroll
-                        for (int i = 0; i < 3; ++i) {
-                            const half_t* plane =
-                                reinterpret_cast<const half_t*>(vs + i * PLANE + 16 * c * RD);
-                            const h4 lo = lds_read_transposed(plane + voff[0][t]);
-                            const h4 hi = lds_read_transposed(plane + voff[1][t]);
-                            const h8 w = {lo[0], lo[1], lo[2], lo[3], hi[0], hi[1], hi[2], hi[3]};
-                            va.part[i] = __builtin_bit_cast(b8, w);
-                        }
-                        if constexpr (APART) {
-                            low[t] = mfma_bf16x3_low(va, pb, low[t]);
-                            o[t] = __builtin_amdgcn_mfma_f32_32x32x16_bf16(va.part[0], pb.part[0],
-                                                                           o[t], 0, 0, 0);
-                        } else {
-                            o[t] = mfma_bf16x3(va, pb, o[t]);
+                        for (int r = 0; r < 16; ++r) acc[r] = 0.0f;
+                        acc = mfma_bf16x3(read_v(0, t), p0, acc);
+                        acc = mfma_bf16x3(read_v(1, t), p1, acc);
+#pragma unroll
+                        for (int r = 0; r < 16; ++r) o[t][r] += acc[r];
+                    }
+                } else {
+#pragma unroll
+                    for (int c = 0; c < BN / 16; ++c) {
+                        const Bf16x3 pb = split_p(c);
+#pragma unroll
+                        for (int t = 0; t < NT; ++t) {
+                            const Bf16x3 va = read_v(c, t);
+                            if constexpr (APART) {
+                                low[t] = mfma_bf16x3_low(va, pb, low[t]);
+                                o[t] = __builtin_amdgcn_mfma_f32_32x32x16_bf16(
+                                    va.part[0], pb.part[0], o[t], 0, 0, 0);
+                            } else {
+                                o[t] = mfma_bf16x3(va, pb, o[t]);
+                            }
                         }
                     }
                 }
                 l += la + lb;
             }
-            __syncthreads();
-            if constexpr (NSTAGE == 1) {
+            if constexpr (!OWN) __syncthreads();
+            if constexpr (!OWN && NSTAGE == 1) {
                 if (step + 1 < steps) store_step(step + 1);
                 __syncthreads();
             }
@@ -958,6 +1018,7 @@ __global__ __launch_bounds__(64 * QW * KSPLIT) void k_flash_attention_bf16x3(
 #pragma unroll
                 for (int r = 0; r < 16; ++r) o[t][r] += low[t][r];
         }
+        if constexpr (OWN) __syncthreads();  // before the merge area takes the others' rows
         if constexpr (KSPLIT > 1) {
             // Groups 1.. hand their (max, sum, output) to group 0 through LDS.
             float* mg = reinterpret_cast<float*>(lds);
@@ -1871,7 +1932,8 @@ void launch_flash_split(rl_context* ctx, uint64_t heads, uint32_t nt, const half
     }
 }
 
-// f32: 128-query tiles of two key shares from kWideF32 tile pairs, else
+// f32: up to 32 queries one tile of four shares, each wave with its own keys
+// (OWN); 128-query tiles of two key shares from kWideF32 tile pairs, else
 // 64-query tiles of four shares (two for head sizes 96 and 128, whose blocks
 // leave no LDS for more, and for at most 128 keys); blocks of 32 keys (64 for
 // head size 32 with 128-query tiles).
@@ -1885,16 +1947,28 @@ void launch_flash_f32(rl_context* ctx, dim3 g, const float* q, const float* k, c
 // pairs) 124 / 140 us, 32 of 96 x [1200, 1200] (160) 81 / 106; 32 of 64 x [1000,
 // 1000] (128) 44.7 / 38.9, 15 x [2000, 2000] (120) 77.5 / 63.9.
 constexpr uint64_t kWideF32 = 150;
+// Up to 32 queries, 32-query tiles (OWN) against the 64-query ones, whose second
+// query wave only stages, and the f32 matrix-core kernel's 32-query tiles before
+// them (9 heads over 3 KV heads): 1 query of 128 after 100 keys 12.3 / 15.6 / 13.1
+// us, after 480 25.2 / 40.9 / 30.8; 16 after 1000 42.4 / 76 / 56.4; 32 of 96 after
+// 3300 113 / 207 / 133; 32 of 64 after 360 14.8 / 17.6 / 20.9; 16 of 32 after 480
+// 9.8 / 10.8 / 11.5.
 rl_status launch_flash_f32(rl_context* ctx, uint64_t heads, const float* q, const float* k,
                            const float* v, float* o, AttnParams p) {
     const uint32_t nt = p.head_dim / 32;
+    const bool one_tile = p.q_len <= 32;
     const bool wide = heads * ((ceil_div(p.q_len, 128) + 1) / 2) >= kWideF32;
-    p.tiles = uint32_t(ceil_div(p.q_len, wide ? 128 : 64));
+    p.tiles = one_tile ? 1u : uint32_t(ceil_div(p.q_len, wide ? 128 : 64));
     p.pairs = flash_pairs(ctx, heads, p.tiles);
     const uint64_t grid = heads * p.pairs;
     if (grid > UINT32_MAX) return fail(RL_ERR_INVALID_SHAPE, "attention grid exceeds u32");
     const dim3 g(static_cast<unsigned>(grid));
-    if (wide) {
+    if (one_tile) {
+        if (nt == 1) launch_flash_f32<1, 1, 4, 32>(ctx, g, q, k, v, o, p);
+        else if (nt == 2) launch_flash_f32<2, 1, 4, 32>(ctx, g, q, k, v, o, p);
+        else if (nt == 3) launch_flash_f32<3, 1, 4, 32>(ctx, g, q, k, v, o, p);
+        else launch_flash_f32<4, 1, 4, 32>(ctx, g, q, k, v, o, p);
+    } else if (wide) {
         if (nt == 1) launch_flash_f32<1, 4, 2, 64>(ctx, g, q, k, v, o, p);
         else if (nt == 2) launch_flash_f32<2, 4, 2, 32>(ctx, g, q, k, v, o, p);
         else if (nt == 3) launch_flash_f32<3, 4, 2, 32>(ctx, g, q, k, v, o, p);

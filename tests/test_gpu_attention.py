@@ -726,3 +726,49 @@ def test_attention_f32_time_does_not_depend_on_small_values(ctx):
         dq, dk, dv = ctx.upload(q), ctx.upload(k), ctx.upload(v)
         times.append(median_us(ctx, lambda: ctx.attention(dq, dk, dv, 0.125, 0, n, out)))
     assert max(times[1:]) <= 2 * times[0], times
+
+
+# Up to 32 queries one tile whose waves take their own keys: shares without a
+# block, with a part of one, several each; 33 queries take the other tiles.
+FEW_QUERY_SHAPES = [
+    (1, 3, 1, 1, 1, 8, 64, 0),          # one key: three shares have none
+    (1, 6, 2, 3, 36, 40, 32, 33),       # a block and a part of one
+    (2, 4, 2, 16, 128, 128, 96, 112),   # a block a share, batch 2
+    (1, 4, 4, 32, 129, 160, 128, 97),   # one key more
+    (1, 9, 3, 31, 300, 304, 128, 269),
+    (1, 40, 8, 32, 32, 32, 96, 0),      # a causal square
+    (5, 32, 8, 2, 400, 416, 64, 398),   # 160 heads: before the 128-query rule
+    (1, 9, 3, 17, 1000, 1024, 32, 983),
+    (1, 9, 3, 33, 433, 448, 128, 400),  # two tiles' worth: 64-query tiles
+]
+
+
+@pytest.mark.parametrize("shape", FEW_QUERY_SHAPES)
+def test_attention_f32_few_queries(ctx, shape):
+    test_attention_within_float64_bound(ctx, np.float32, shape)
+
+
+@pytest.mark.parametrize("hd", [96, 128])
+def test_attention_f32_few_queries_cost_less_than_a_tile(ctx, hd):
+    """One query over 481 keys against 64 (0.53 of the time as measured; 0.9 on
+    tiles of 64)."""
+    times = []
+    for ql in (1, 64):
+        kl = 480 + ql
+        q, k, v = (ctx.upload(synth.normal(94, (1, h, n, hd)))
+                   for h, n in ((9, ql), (3, kl), (3, kl)))
+        out = ctx.empty((1, 9, ql, hd), np.float32)
+        times.append(median_us(ctx, lambda: ctx.attention(q, k, v, 0.1, 480, kl, out)))
+    assert times[0] <= 0.75 * times[1], times
+
+
+@pytest.mark.parametrize("power", [-59, -60, -61, -90])
+def test_attention_f32_tiny_scales(ctx, power):
+    """Scales around 2^-60, below which the row kernel takes over, with queries
+    and keys that bring the scores back to ordinary sizes."""
+    hd, ql = 64, 70
+    q = synth.normal(95, (1, 4, ql, hd)) * np.float32(2.0 ** 28)
+    k = synth.normal(96, (1, 2, ql, hd)) * np.float32(2.0 ** (-power - 31))
+    v = synth.normal(97, (1, 2, ql, hd))
+    got = run_attention(ctx, q, k, v, 2.0 ** power, 0, ql)
+    check(got, q, k, v, 2.0 ** power, 0, ql, f"scale 2^{power}")
