@@ -413,6 +413,7 @@ struct FusedSeg {
     FastDiv div;          // packs per row (bias add, row gather) or per head (repeat_kv)
     uint32_t repeats;     // repeat_kv
     uint32_t small_index;
+    uint32_t stream;      // maps, bias adds: streamed loads
     FusedDims outer;      // row gather / scatter
 };
 
@@ -426,6 +427,11 @@ struct FusedSeg {
 // blocks in a run of their own and streamed loads (201 MB in and out of the
 // L2s), 28.2 with plain loads, 28.6 in groups; [4096, 2560] 54.5, 52.5, 49.8; f32
 // [4096, 1536] 58.6, 59.6, 46.9; f32 [2000, 960] 25.3, 22.4, 18.1.
+// An op that shares its input with none has plain loads where other ops share
+// its launch and it reads at most kStreamReadBytes (add, SiLU and mul over four
+// arrays, f16 [8192, 4096]: streamed 87.6 us, plain 79.5; [16384, 8192]: 354, 372),
+// else streamed ones (alone in its launch, reading what the one before wrote:
+// add, SwiGLU, add, f16 [8192, 4096]: streamed 102, plain 112; f32 194, 213).
 struct FusedTable {
     // each group's first block in the fused grid (ascending) at its first op's
     // index, kNoBlock at its other ops
@@ -473,16 +479,28 @@ constexpr uint32_t fused_kind() {
 template <typename TIn, typename TOut, int ARITY, typename Op>
 __device__ inline void fused_map(const FusedSeg& s, uint32_t blk) {
     typedef FusedShape<Op, TIn, TOut> M;
-    map_body<TIn, TOut, map_pack<TIn, TOut>(), M::unroll, ARITY, M::nt_store, M::phased, Op, false>(
-        static_cast<const TIn*>(s.a), static_cast<const TIn*>(s.b), static_cast<TOut*>(s.out),
-        s.n_packs, s.tail, Op{}, blk);
+    const auto body = [&](auto stream) {
+        map_body<TIn, TOut, map_pack<TIn, TOut>(), M::unroll, ARITY, M::nt_store, M::phased, Op,
+                 stream.value>(static_cast<const TIn*>(s.a), static_cast<const TIn*>(s.b),
+                               static_cast<TOut*>(s.out), s.n_packs, s.tail, Op{}, blk);
+    };
+    if (s.stream)
+        body(std::true_type{});
+    else
+        body(std::false_type{});
 }
 
 template <typename T>
 __device__ inline void fused_bias(const FusedSeg& s, uint32_t blk, uint32_t nblk) {
-    broadcast_body<T, 16 / sizeof(T), kFusedBiasUnroll, false>(
-        static_cast<const T*>(s.a), static_cast<const T*>(s.b), static_cast<T*>(s.out),
-        s.n_packs, s.div, blk, nblk);
+    const auto body = [&](auto stream) {
+        broadcast_body<T, 16 / sizeof(T), kFusedBiasUnroll, stream.value>(
+            static_cast<const T*>(s.a), static_cast<const T*>(s.b), static_cast<T*>(s.out),
+            s.n_packs, s.div, blk, nblk);
+    };
+    if (s.stream)
+        body(std::true_type{});
+    else
+        body(std::false_type{});
 }
 
 constexpr int kMoveUnroll = 2;  // packs per thread of the row gather and repeat_kv
@@ -739,6 +757,9 @@ rl_status flush_fused(rl_context* ctx) {
             blocks = uint32_t(ceil_div(slots, 8)) * 8 * w;  // blocks past an op's last do nothing
         }
         t.members[start] = n - start;
+        const uint64_t reads = lead.read[0][1] - lead.read[0][0] + lead.read[1][1] - lead.read[1][0];
+        t.seg[start].stream =
+            n - start == 1 && (ctx->fused_count == 1 || reads > kStreamReadBytes);
         for (uint32_t k = start; k < n; ++k) t.first[k] = k == start ? first : kNoBlock;
         first += blocks;
     }
