@@ -137,19 +137,18 @@ constexpr float kFarSlack = 1.0f;
 // with plain f32 products, as k_attention_rows computes them: for rows whose
 // output the split products leave non-finite (inf - inf and 0 * inf between
 // the parts of an infinite operand or value), so that infinities and NaN come
-// out as in unsplit arithmetic.  Eight rows at a time, which share every read
-// of K and V; lane = key for the scores, lane = head elements lane + 64 t for
+// out as in unsplit arithmetic.  R rows at a time, which share every read
+// of K and V (four where eight would cost the calling kernel registers); lane = key for the scores, lane = head elements lane + 64 t for
 // the values; no LDS.  D <= 32 NT, a multiple of 8, rows on the 16-byte grid;
 // row c sees `keys` + c keys, at most kv_len.  One MI355X, 9 heads of 64 x [2048,
 // 2048] f32 with an infinite value row in each KV head, so in nearly every
 // query's sum: 2.08 ms, 7.84 a row at a time (68.6 us with none).
-template <typename T, int NT>
+template <typename T, int NT, int R>
 __device__ inline void exact_rows(uint32_t redo, const T* __restrict__ q,
                                   const T* __restrict__ kh, const T* __restrict__ vh,
                                   T* __restrict__ out, uint32_t D, uint64_t keys, uint32_t kv_len,
                                   float scale) {
     constexpr int DT = (NT + 1) / 2;
-    constexpr int R = 8;
     typedef T t4 __attribute__((ext_vector_type(4)));
     const uint32_t lane = threadIdx.x % 64;
     while (redo != 0) {
@@ -600,7 +599,7 @@ __global__ __launch_bounds__(64 * QW * KSPLIT) void k_flash_attention(
                 // wave (after its stores above: same wave, in order)
                 const uint64_t redo = __ballot(!finite);
                 const uint64_t first = (uint64_t(bh) * p.q_len + qw0) * hd;
-                exact_rows<half_t, NT>(uint32_t(redo | redo >> 32), q + first, kh, vh, out + first,
+                exact_rows<half_t, NT, 4>(uint32_t(redo | redo >> 32), q + first, kh, vh, out + first,
                                        hd, uint64_t(p.start) + qw0 + 1, p.kv_len, p.scale);
             }
         }
@@ -1084,7 +1083,7 @@ __global__ __launch_bounds__(64 * QW * KSPLIT) void k_flash_attention_bf16x3(
             }
             const uint64_t redo = __ballot(exact);
             const uint64_t first = (uint64_t(bh) * p.q_len + qw0) * D;
-            exact_rows<float, NT>(uint32_t(redo | redo >> 32), q + first, kh, vh, out + first, D,
+            exact_rows<float, NT, 8>(uint32_t(redo | redo >> 32), q + first, kh, vh, out + first, D,
                                   uint64_t(p.start) + qw0 + 1, p.kv_len, p.scale);
         }
     }
