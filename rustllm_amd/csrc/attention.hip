@@ -2026,11 +2026,16 @@ rl_status launch_flash_any(rl_context* ctx, uint64_t heads, const half_t* q, con
 // scaled range of its products could still matter); in f16 the padded matrix-core kernel (ANY) for the other
 // multiples of 8 up to 256 (rows of whole 16-byte pieces); the row kernel
 // otherwise (head sizes up to 512).
-bool use_flash_any(const AttnShape& s, const void* q, const void* k, const void* v,
+// Up to kAnyFewKeys visible keys the row kernel beats the padded one, whose
+// operand setup does not depend on the keys (one MI355X, 9 heads): 1 key, head
+// size 80 6.5 against 8.0 us, 112 6.3 / 9.7, 136 6.6 / 11.1, 256 7.5 / 11.4; 17 keys
+// of 112 8.7 / 9.5; 21 keys of 80 8.7 / 8.3, of 112 9.9 / 9.7, of 136 12.9 / 10.7.
+constexpr uint64_t kAnyFewKeys = 18;
+bool use_flash_any(const AttnShape& s, uint64_t start, const void* q, const void* k, const void* v,
                    const void* o) {
     const uint64_t span = (s.kv_len + uint64_t(kFlashMaxBlockKeys) * kFlashMaxKeySplit) *
                           s.head_dim * sizeof(half_t);
-    return s.head_dim % 8 == 0 && s.head_dim <= 256 && span < (uint64_t(1) << 31) &&
+    return s.head_dim % 8 == 0 && s.head_dim <= 256 && start + s.q_len > kAnyFewKeys && span < (uint64_t(1) << 31) &&
            aligned_to(q, 16) && aligned_to(k, 16) && aligned_to(v, 16) && aligned_to(o, 16);
 }
 template <typename T>
@@ -2280,7 +2285,7 @@ rl_status attention_entry(rl_context* ctx, const char* name, const rl_buffer* q,
         return after_launch(ctx, name);
     }
     if constexpr (std::is_same<T, half_t>::value) {
-        if (use_flash_any(s, qd, kd, vd, od)) {
+        if (use_flash_any(s, start, qd, kd, vd, od)) {
             if (rl_status st = launch_flash_any(ctx, heads, qd, kd, vd, od, p)) return st;
             return after_launch(ctx, name);
         }

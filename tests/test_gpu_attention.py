@@ -772,3 +772,22 @@ def test_attention_f32_tiny_scales(ctx, power):
     v = synth.normal(97, (1, 2, ql, hd))
     got = run_attention(ctx, q, k, v, 2.0 ** power, 0, ql)
     check(got, q, k, v, 2.0 ** power, 0, ql, f"scale 2^{power}")
+
+
+@pytest.mark.parametrize("hd", [8, 80, 136, 256])
+@pytest.mark.parametrize("ql,start", [(1, 0), (1, 17), (18, 0), (1, 18), (19, 0), (3, 30)])
+def test_attention_padded_heads_few_keys(ctx, hd, ql, start):
+    """Both sides of the 18 visible keys from which padded heads leave the row kernel."""
+    test_attention_within_float64_bound(ctx, np.float16,
+                                        (2, 4, 2, ql, start + ql, start + ql + 3, hd, start))
+
+
+def test_attention_padded_heads_one_key_costs_less_than_many(ctx):
+    """One key against 64 (0.6 of the time as measured; 1.0 on the padded kernel)."""
+    times = []
+    for start in (0, 63):
+        q, k, v = (ctx.upload(synth.normal(98, (1, 9, n, 136)).astype(np.float16))
+                   for n in (1, start + 1, start + 1))
+        out = ctx.empty((1, 9, 1, 136), np.float16)
+        times.append(median_us(ctx, lambda: ctx.attention(q, k, v, 0.1, start, start + 1, out)))
+    assert times[0] <= 0.85 * times[1], times
