@@ -1080,3 +1080,5 @@ def test_add_rmsnorm_rows_past_the_streaming_size(ctx, dtype):
         ctx.finish()
         assert np.array_equal(s[pick], s2.numpy()) and np.array_equal(y[pick], y2.numpy())
         assert np.array_equal(s, x + x[::-1])
+        _, ry = o.add_rmsnorm(x[pick], x[::-1][pick], w, 1e-5)
+        check_float(y[pick], ry, f"add_rmsnorm of {rows} rows")
