@@ -1841,13 +1841,13 @@ uint32_t flash_pairs(const rl_context* ctx, uint64_t heads, uint32_t tiles) {
 
 // Key chunks per 128-query tile for the f16 kernel (1 = no split), W the
 // wide tile pairs, steps the longest tile's key steps (two blocks each).
-// One workgroup a CU fits (its LDS), so chunks beyond 256 / W workgroups
+// One workgroup a CU fits (its LDS), so chunks beyond CUs / W workgroups
 // queue behind the first wave.  One MI355X, every launch of a call inside
 // the events, against what the shape took unsplit: with 96 <= W <= 128 and
 // at least 16 steps two chunks (8 heads x [4096, 4096] 45.0 -> 39.5 us on the
 // wide tiles, 15 heads x 2048 queries after 2048 cached keys 61.3 -> 47.8,
 // 32 heads of 128 x 1024 after 3072 105.8 -> 87.6); below 96 pairs only a
-// prefill after cached keys, whose every tile is long, splits, up to 256 / W
+// prefill after cached keys, whose every tile is long, splits, up to CUs / W
 // chunks of two steps or more (15 heads x 512 queries after 3584 keys: 51.1
 // us on 32-query tiles, 25.5 in 8 chunks; 1024 after 3072: 49.1, 34.2 in 4).
 // Causal squares with fewer pairs stay on the 32-query tiles (8 heads of 128
@@ -1867,22 +1867,23 @@ struct FlashChunks {
     bool by_tile;     // workgroups of one tile, not of a pair
     float slack;      // rescaling threshold
 };
-FlashChunks flash_key_chunks(uint64_t heads, uint64_t q_len, uint64_t kv_len, uint64_t start,
-                             uint64_t head_dim) {
+FlashChunks flash_key_chunks(const rl_context* ctx, uint64_t heads, uint64_t q_len,
+                             uint64_t kv_len, uint64_t start, uint64_t head_dim) {
+    const uint64_t cus = uint64_t(ctx->num_cus);
     const uint64_t wide = heads * ((ceil_div(q_len, 128) + 1) / 2);
     const uint64_t bn = head_dim <= 64 ? 128 : 64;
     const uint64_t keys = std::min<uint64_t>(kv_len, start + q_len);  // the longest tile's
     const uint64_t steps = ceil_div(ceil_div(keys, bn), 2);
     if (wide >= kFlashFillBlocks) {
-        const bool tiles_fit = start >= 4 * q_len && heads * ceil_div(q_len, 128) <= 256;
-        if (wide > 128 || steps < 16) return {1, false, kRescaleSlack};
+        const bool tiles_fit = start >= 4 * q_len && heads * ceil_div(q_len, 128) <= cus;
+        if (2 * wide > cus || steps < 16) return {1, false, kRescaleSlack};
         if (tiles_fit) return {1, false, kFarSlack};
         return {2, false, kRescaleSlack};
     }
     if (start == 0 || steps < 16) return {1, false, kRescaleSlack};
-    const uint64_t chunks = std::max<uint64_t>(std::min<uint64_t>({256 / wide, 8, steps / 2}), 1);
+    const uint64_t chunks = std::max<uint64_t>(std::min<uint64_t>({cus / wide, 8, steps / 2}), 1);
     const uint64_t halved =
-        std::min<uint64_t>({256 / (heads * ceil_div(q_len, 128)), 8, steps / 2});
+        std::min<uint64_t>({cus / (heads * ceil_div(q_len, 128)), 8, steps / 2});
     if (start >= 4 * q_len && halved >= 2 && 2 * halved >= chunks)
         return {uint32_t(halved), true, kFarSlack};
     return {uint32_t(chunks), false, kRescaleSlack};
@@ -2248,7 +2249,7 @@ rl_status attention_entry(rl_context* ctx, const char* name, const rl_buffer* q,
             // the partials (not while a graph records, nor for the
             // allocation-free entry).
             const auto [chunks, by_tile, slack] =
-                flash_key_chunks(heads, s.q_len, s.kv_len, start, s.head_dim);
+                flash_key_chunks(ctx, heads, s.q_len, s.kv_len, start, s.head_dim);
             const bool pooled = mode == DecodeScratch::kPool && !ctx->capturing;
             p.slack = pooled ? slack : kRescaleSlack;
             if (chunks > 1 && pooled) {

@@ -912,9 +912,11 @@ bool use_mfma(const GqaShape& s, const void* a, const void* b, const void* o) {
            aligned_to(o, 16);
 }
 
-// f32 QK^T workgroups in one round: two a CU (9 heads of 64 x [2048, 2048]: 51.3
-// us; runs of tiles for 768 workgroups 53.3, 300 60.0).
-constexpr uint64_t kQkResident = 512;
+// f32 QK^T workgroups in one round, per CU: 2 (9 heads of 64 x [2048, 2048]: 51.3
+// us; runs of tiles for 3 a CU 53.3, 1.2 60.0; against 1 a CU, 15 heads x [1025,
+// 1025] of 32 19.7 / 30.6, 64 28.9 / 43.4, 96 38.7 / 58.9, 128 46.5 / 66.0; 9 of 128 x
+// [700, 700] 19.9 / 18.6, 15 of 64 20.0 / 19.2).
+constexpr uint64_t kQkResident = 2;
 
 template <typename T>
 rl_status qk_entry(rl_context* ctx, const char* name, const rl_buffer* q, const rl_buffer* k,
@@ -972,8 +974,9 @@ rl_status qk_entry(rl_context* ctx, const char* name, const rl_buffer* q, const 
             // over several only when the query tiles alone do not fill the
             // resident workgroups.
             const uint64_t base = heads * p.q_tiles;
+            const uint64_t resident = kQkResident * uint64_t(ctx->num_cus);
             const uint64_t groups =
-                std::min<uint64_t>(p.k_tiles, std::max<uint64_t>(1, kQkResident / base));
+                std::min<uint64_t>(p.k_tiles, std::max<uint64_t>(1, resident / base));
             p.k_per_block = uint32_t(ceil_div(p.k_tiles, groups));
             p.k_groups = uint32_t(ceil_div(p.k_tiles, p.k_per_block));
             const uint64_t grid = base * p.k_groups;
