@@ -33,8 +33,11 @@
  *    + softmax, and RoPE -- each reads all it writes first.  For every other
  *    op, and for outputs that overlap an input only in part, the output must
  *    not overlap the inputs.
- *  - f16 is IEEE binary16.  All arithmetic is float32; f16 results are
- *    rounded to nearest even.
+ *  - f16 is IEEE binary16.  All arithmetic is float32, f16 results rounded
+ *    to nearest even; the grouped-query matmuls and the fused attention make
+ *    it of matrix-core products, in f32 accumulation: of the f16 operands, or
+ *    for f32 of three bf16 parts of each operand, which hold all its bits (six
+ *    of their nine products; the others are below 2^-26 of the whole).
  *  - One context per thread; a context is not thread-safe (MetalContext is
  *    !Sync, src/metal/context.rs:14-17).  All work of a context runs in
  *    order on its one stream.
@@ -464,9 +467,11 @@ rl_status rl_embedding_f16(rl_context* ctx, const rl_buffer* weight, uint64_t vo
  * Key j is masked for query i when j > query_start_pos + i.  Checks in the
  * reference's order (head groups as RL_ERR_MODEL_FORMAT, the u32 limits,
  * the scale/mask checks); also rejected: kv_capacity < kv_len and
- * head_dim > 512 when the matrix-core path (f16, head_dim 32/64/96/128)
- * does not apply.  Results differ from the four separate calls by their
- * intermediate roundings: scores and probabilities stay in f32 here.  f16
+ * head_dim > 512.
+ * Results differ from the four separate calls by their
+ * intermediate roundings: scores and the softmax stay in f32 here; the
+ * probabilities of the f16 matrix-core paths are rounded to f16 for their
+ * product with V (to 22 bits for head sizes off the multiples of 32 and above 128).  f16
  * launches with few 128-query tiles and long key ranges (a prefill after
  * cached keys) split each tile's keys over workgroups: f32 partials in a
  * pool block, merged by a second kernel (not while a graph records, where

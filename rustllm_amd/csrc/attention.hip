@@ -10,8 +10,7 @@
 // running (max, sum, output) per query, so the scores never leave the chip.
 //
 // f16 with a head size that is a multiple of 32 (32..128; padded, of 8 up to
-// 256) takes the matrix cores
-// (v_mfma_f32_32x32x16_f16, f32 accumulation): per wave 32 queries,
+// 256) takes the matrix cores (v_mfma_f32_32x32x16_f16, f32 accumulation): per wave 32 queries,
 // S^T = K Q^T so that each lane owns one query column and its row statistics
 // need one cross-lane exchange; the keys of a 32-key tile are read in an
 // order that swaps bits 2 and 3 of the key index, which leaves each lane
@@ -23,10 +22,10 @@
 // two stages deep), so the next block streams in during this one's compute.
 // f32 with the multiples of 32 up to 128 takes the bf16 matrix cores in the
 // same tiling, each f32 operand as three bf16 parts (f32 probabilities).
-// Decode steps (few query
-// rows per KV head) split the keys over many workgroups; other head sizes
-// (f16 off the multiples of 8 or above 256, f32 off those of 32, up to 512)
-// take a one-wave-per-query kernel on the vector ALUs.
+// Decode steps (few query rows per KV head) split the keys over many
+// workgroups; other head sizes (f16 off the multiples of 8 or above 256, f32
+// off those of 32, up to 512) and padded ones with a few visible keys take a
+// one-wave-per-query kernel on the vector ALUs.
 //
 // Arithmetic (both kernels): scores are f32 dot products of the (widened)
 // inputs; x * scale in f32 and masking as attention_scale_mask.metal:21-41
@@ -35,8 +34,9 @@
 // output type.  The reference rounds the scores, the scaled scores and the
 // probabilities to f16 in between; this pass does not, so it is closer to
 // the exact result than the reference's own four calls (the tests bound both
-// against float64).  The MFMA kernel feeds P to the second product as f16
-// (relative error 2^-11 per probability, inside the same bound).
+// against float64).  The f16 MFMA kernel feeds P to the second product as f16
+// (relative error 2^-11 per probability, inside the same bound), for padded
+// heads as two f16 parts.
 #include "common.hpp"
 #include "mfma_layout.hpp"
 
@@ -237,18 +237,21 @@ constexpr float kAnyShift = 12.0f;
 // [4096, 4096], one MI355X).
 //
 // ANY: a head size that is a multiple of 8 but has no kernel of its own (D is
-// then the next multiple of 32, or 192 or 256 above 128): rows are read and
+// then the next multiple of 32, above 128 256): rows are read and
 // written at the run-time size, the padding is zeros in registers and LDS.
-// Those head sizes take f32 probabilities (k_attention_rows did): P enters
-// the second product as the sum of two f16 parts, hi + lo, of 2^(t - m + 12)
-// -- 22 bits, and the factor 2^12 (kAnyShift), which cancels in the division
+// k_attention_rows, which they took before, has f32 probabilities; here P enters
+// the second product as the sum of two f16 parts, hi + lo, of 2^(t - m + 12):
+// 22 bits, and the factor 2^12 (kAnyShift), which cancels in the division
 // by the sum, keeps lo's own bits above the f16 subnormals down to
-// probabilities of 2^-15 of the largest.  A query whose output is not finite
+// probabilities of 2^-15 of the largest; below, in steps of 2^-36 of it.  (A sum
+// of its own for a lo scaled by 2^12 more, steps of 2^-48, cost 10 % at head size
+// 80 and 22 at 136 and above; errors against 64 bits are 2.01e-4 with either and
+// with k_attention_rows, the output's own rounding.)  A query whose output is not finite
 // is computed again by exact_rows, whose products are not split.  One MI355X,
 // 8 heads x [1021, 1021], head size 80: 475 us on k_attention_rows (a dot
-// product a lane on the vector ALUs, uncoalesced key rows), 24.4 us here; 32
-// heads x [4096, 4096]: 12.0 ms, 0.18 ms; head size 256, 8 heads x [570, 570]:
-// 645 us, 39.7 us.
+// product a lane on the vector ALUs, uncoalesced key rows), 17.2 us here; 32
+// heads x [4096, 4096]: 12.0 ms, 0.19 ms; head size 256, 8 heads x [570, 570]:
+// 642 us, 30.1 us.
 template <int NT, int QW, int KSPLIT, int BN, bool PARTIAL = false, bool ANY = false>
 __global__ __launch_bounds__(64 * QW * KSPLIT) void k_flash_attention(
     const half_t* __restrict__ q, const half_t* __restrict__ k, const half_t* __restrict__ v,
@@ -677,13 +680,15 @@ __global__ __launch_bounds__(256) void k_flash_combine(half_t* __restrict__ out,
 // (infinities, NaN, sums of 2^80 or more).  (A score whose partial sums pass -2^104
 // counts as -inf, far inside the f32 rounding of its terms where use_flash
 // lets the scale in.)
-// Bound by matrix and vector work in turn (they do not overlap: 35 % matrix,
-// 34 % vector, ~19 vector operations a score, at 69 % balance of the tiles
-// over the CUs).  One MI355X against v_mfma_f32_32x32x2_f32 in the same
-// tiling (which it replaces): 15 heads of 64 x [3001, 3001] 213 -> 120 us, relative
-// error against 64 bits 3.6e-7 -> 3.0e-7; 32 of 64 x 500 queries after 3000
-// keys 306 -> 99 us; 12 of 128 x [1900, 1900] 185 -> 136 us; 9 x [64, 64]
-// 10.5 -> 8.0 us.  Software-pipelined over the blocks (the next block's scores
+// Bound by the latency between a step's phases at two waves a SIMD and the
+// balance of the tiles over the CUs (69 %): the matrix cores are busy 34 %, the
+// vector ALUs 38 % of the time, ~20 vector operations a score (the two do
+// overlap: 8 MFMAs of 128 ns beside 64 exponentials of 238 take 263 ns in two
+// waves of a SIMD, 273 in one).  One MI355X against v_mfma_f32_32x32x2_f32 (which
+// it replaces; in its own tiling): 15 heads of 64 x [3001, 3001] 241 -> 120.5 us, relative
+// error against 64 bits 3.7e-7 -> 2.9e-7; 32 of 64 x 500 queries after 3000
+// keys 309 -> 113 us; 12 of 128 x [1900, 1900] 237 -> 141 us; 9 x [64, 64]
+// 19.1 -> 7.5 us.  Software-pipelined over the blocks (the next block's scores
 // beside this one's exponentials), or with the two waves of a SIMD splitting at
 // different ends of a step, it was no faster (124 and 133 us for 119).
 template <int NT, int QW, int KSPLIT, int BN>
@@ -1829,8 +1834,8 @@ FlashShape flash_shape(uint64_t heads, uint64_t q_len, uint64_t head_dim) {
 // all heads.  One MI355X, pairs against tiles: f16, 8 heads of 80 x [1021,
 // 1021] (128 pairs) 24.3 / 18.8 us; 15 of 64 x [512, 512] (120) 10.9 / 7.5;
 // 32 of 64 x 100 queries after 1000 keys (64) 21.0 / 11.3; 15 of 64 x [1500,
-// 1500] (360) 22.8 / 19.7; f32, 15 of 64 x [3001, 3001] (180) 238 / 211;
-// 32 of 64 x 200 after 2000 (128) 128 / 66.  Filled: f16, 15 of 64 x [4096,
+// 1500] (360) 22.8 / 19.7; f32 (on the f32 matrix cores, which it had then), 15
+// of 64 x [3001, 3001] (180) 238 / 211; 32 of 64 x 200 after 2000 (128) 128 / 66.  Filled: f16, 15 of 64 x [4096,
 // 4096] (240) 53.2 / 54.4, 32 x [2048, 2048] (256) 32.0 / 32.9, 15 x [900,
 // 900] (225) 14.2 / 14.4.
 uint32_t flash_pairs(const rl_context* ctx, uint64_t heads, uint32_t tiles) {
@@ -1944,8 +1949,8 @@ void launch_flash_f32(rl_context* ctx, dim3 g, const float* q, const float* k, c
               p);
 }
 // 128-query tiles against 64 (one MI355X): 15 heads of 64 x [3001, 3001] (180
-// pairs) 124 / 140 us, 32 of 96 x [1200, 1200] (160) 81 / 106; 32 of 64 x [1000,
-// 1000] (128) 44.7 / 38.9, 15 x [2000, 2000] (120) 77.5 / 63.9.
+// pairs) 132 / 152 us, 32 of 96 x [1200, 1200] (160) 90 / 118; 32 of 64 x [1000,
+// 1000] (128) 48.8 / 45.5, 15 x [2000, 2000] (120) 86 / 76.
 constexpr uint64_t kWideF32 = 150;
 // Up to 32 queries, 32-query tiles (OWN) against the 64-query ones, whose second
 // query wave only stages, and the f32 matrix-core kernel's 32-query tiles before

@@ -47,10 +47,10 @@ __host__ __device__ constexpr int v_stride_tr(int d) {
 // banks (64 banks of 4 bytes; a row is D / 8 chunks).
 template <int NT>
 __device__ inline uint32_t lds_swizzle(uint32_t r) {
+    static_assert(NT == 1 || NT == 2 || NT == 4 || NT == 8, "rows of 4, 8, 16 or 32 chunks");
     if constexpr (NT == 1) return (r >> 2) & 3u;
     else if constexpr (NT == 2) return ((r & 2u) << 1) | ((r >> 2) & 3u);
-    else if constexpr (NT == 4 || NT == 8) return ((r & 3u) << 2) | ((r >> 2) & 3u);
-    else return 0u;
+    else return ((r & 3u) << 2) | ((r >> 2) & 3u);
 }
 
 // ds_read_b64_tr_b16: in each group of 16 lanes, lanes 4j .. 4j + 3 read 8
@@ -77,7 +77,6 @@ __device__ inline h4 lds_read_transposed(const half_t* p) {
 constexpr float kPartScale = 0x1p24f;
 constexpr float kProductUnscale = 0x1p-48f;  // of a sum of products of two scaled values
 typedef __bf16 b8 __attribute__((ext_vector_type(8)));
-typedef __bf16 b4 __attribute__((ext_vector_type(4)));
 typedef __bf16 b2 __attribute__((ext_vector_type(2)));
 typedef float f32x2 __attribute__((ext_vector_type(2)));
 typedef float f32x8 __attribute__((ext_vector_type(8)));

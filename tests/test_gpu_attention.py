@@ -388,7 +388,7 @@ def test_attention_in_a_graph_matches_eager(ctx, dtype):
 
 # ------------------------------- f16 head sizes without a kernel of their own
 
-# Padded to the next multiple of 32 (192 and up: to 256); the last of each
+# Padded to the next multiple of 32 (above 128: to 256); the last of each
 # wide/narrow pair has enough heads and queries for the 128-query tiles.
 PADDED_SHAPES = [
     (1, 2, 1, 33, 40, 48, 8, 7),
