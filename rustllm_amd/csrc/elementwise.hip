@@ -403,7 +403,7 @@ inline unsigned grid_for(uint64_t items, uint64_t per_block) {
 typedef OuterDimsT<kMaxFusedOuterRank, uint32_t> FusedDims;
 
 struct FusedSeg {
-    uint32_t kind;
+    uint32_t kind;  // FusedKind, | kFusedStream
     uint32_t tail;  // map
     const void* a;
     const void* b;
@@ -413,7 +413,6 @@ struct FusedSeg {
     FastDiv div;          // packs per row (bias add, row gather) or per head (repeat_kv)
     uint32_t repeats;     // repeat_kv
     uint32_t small_index;
-    uint32_t stream;      // maps, bias adds: streamed loads
     FusedDims outer;      // row gather / scatter
 };
 
@@ -443,6 +442,7 @@ struct FusedTable {
     FusedSeg seg[kMaxFused];
 };
 constexpr uint32_t kNoBlock = 0xffffffffu;
+constexpr uint32_t kFusedStream = 1u << 31;  // maps, bias adds: streamed loads
 
 // Elements of a slot: a power of two of at least the largest block (4096) and
 // at most an eighth of an XCD's share (so that the XCDs come out even), up to
@@ -477,27 +477,28 @@ constexpr uint32_t fused_kind() {
 }
 
 template <typename TIn, typename TOut, int ARITY, typename Op>
-__device__ inline void fused_map(const FusedSeg& s, uint32_t blk) {
+__device__ inline void fused_map(const FusedSeg& s, bool stream_loads, uint32_t blk) {
     typedef FusedShape<Op, TIn, TOut> M;
     const auto body = [&](auto stream) {
         map_body<TIn, TOut, map_pack<TIn, TOut>(), M::unroll, ARITY, M::nt_store, M::phased, Op,
                  stream.value>(static_cast<const TIn*>(s.a), static_cast<const TIn*>(s.b),
                                static_cast<TOut*>(s.out), s.n_packs, s.tail, Op{}, blk);
     };
-    if (s.stream)
+    if (stream_loads)
         body(std::true_type{});
     else
         body(std::false_type{});
 }
 
 template <typename T>
-__device__ inline void fused_bias(const FusedSeg& s, uint32_t blk, uint32_t nblk) {
+__device__ inline void fused_bias(const FusedSeg& s, bool stream_loads, uint32_t blk,
+                                  uint32_t nblk) {
     const auto body = [&](auto stream) {
         broadcast_body<T, 16 / sizeof(T), kFusedBiasUnroll, stream.value>(
             static_cast<const T*>(s.a), static_cast<const T*>(s.b), static_cast<T*>(s.out),
             s.n_packs, s.div, blk, nblk);
     };
-    if (s.stream)
+    if (stream_loads)
         body(std::true_type{});
     else
         body(std::false_type{});
@@ -547,19 +548,21 @@ __global__ __launch_bounds__(kThreads) void k_fused(FusedTable t) {
         blk = (s8 * 8 + blk % 8) * t.weight[i] + j;
     }
     const FusedSeg& s = t.seg[i];  // read in place from the kernel arguments
-    switch (s.kind) {
-        case kFusedAddF32: fused_map<float, float, 2, AddOp>(s, blk); break;
-        case kFusedMulF32: fused_map<float, float, 2, MulOp>(s, blk); break;
-        case kFusedSiluF32: fused_map<float, float, 1, SiluF32Op>(s, blk); break;
-        case kFusedSwigluF32: fused_map<float, float, 2, SwigluF32Op>(s, blk); break;
-        case kFusedAddF16: fused_map<half_t, half_t, 2, AddOp>(s, blk); break;
-        case kFusedMulF16: fused_map<half_t, half_t, 2, MulOp>(s, blk); break;
-        case kFusedSiluF16: fused_map<half_t, half_t, 1, SiluF16Op>(s, blk); break;
-        case kFusedSwigluF16: fused_map<half_t, half_t, 2, SwigluF16Op>(s, blk); break;
-        case kFusedCastF32F16: fused_map<float, half_t, 1, CopyOp>(s, blk); break;
-        case kFusedCastF16F32: fused_map<half_t, float, 1, CopyOp>(s, blk); break;
-        case kFusedBiasF32: fused_bias<float>(s, blk, nblk); break;  // one tile a block
-        case kFusedBiasF16: fused_bias<half_t>(s, blk, nblk); break;
+    const uint32_t kind = s.kind;
+    const bool st = (kind & kFusedStream) != 0;
+    switch (kind & ~kFusedStream) {
+        case kFusedAddF32: fused_map<float, float, 2, AddOp>(s, st, blk); break;
+        case kFusedMulF32: fused_map<float, float, 2, MulOp>(s, st, blk); break;
+        case kFusedSiluF32: fused_map<float, float, 1, SiluF32Op>(s, st, blk); break;
+        case kFusedSwigluF32: fused_map<float, float, 2, SwigluF32Op>(s, st, blk); break;
+        case kFusedAddF16: fused_map<half_t, half_t, 2, AddOp>(s, st, blk); break;
+        case kFusedMulF16: fused_map<half_t, half_t, 2, MulOp>(s, st, blk); break;
+        case kFusedSiluF16: fused_map<half_t, half_t, 1, SiluF16Op>(s, st, blk); break;
+        case kFusedSwigluF16: fused_map<half_t, half_t, 2, SwigluF16Op>(s, st, blk); break;
+        case kFusedCastF32F16: fused_map<float, half_t, 1, CopyOp>(s, st, blk); break;
+        case kFusedCastF16F32: fused_map<half_t, float, 1, CopyOp>(s, st, blk); break;
+        case kFusedBiasF32: fused_bias<float>(s, st, blk, nblk); break;  // one tile a block
+        case kFusedBiasF16: fused_bias<half_t>(s, st, blk, nblk); break;
         case kFusedGatherF32: fused_gather<float>(s, blk, nblk); break;
         case kFusedGatherF16: fused_gather<half_t>(s, blk, nblk); break;
         case kFusedRepeatF32: fused_repeat<float>(s, blk, nblk); break;
@@ -758,15 +761,15 @@ rl_status flush_fused(rl_context* ctx) {
         }
         t.members[start] = n - start;
         const uint64_t reads = lead.read[0][1] - lead.read[0][0] + lead.read[1][1] - lead.read[1][0];
-        t.seg[start].stream =
-            n - start == 1 && (ctx->fused_count == 1 || reads > kStreamReadBytes);
+        if (n - start == 1 && (ctx->fused_count == 1 || reads > kStreamReadBytes))
+            t.seg[start].kind = kFusedStream;
         for (uint32_t k = start; k < n; ++k) t.first[k] = k == start ? first : kNoBlock;
         first += blocks;
     }
     for (uint32_t i = 0; i < n; ++i) {
         const FusedOp& f = ctx->fused[order[i]];
         FusedSeg& g = t.seg[i];
-        g.kind = f.kind;
+        g.kind |= f.kind;
         g.tail = f.tail;
         g.a = f.a;
         g.b = f.b;
