@@ -249,7 +249,7 @@ constexpr float kAnyShift = 12.0f;
 // with k_attention_rows, the output's own rounding.)  A query whose output is not finite
 // is computed again by exact_rows, whose products are not split.  One MI355X,
 // 8 heads x [1021, 1021], head size 80: 475 us on k_attention_rows (a dot
-// product a lane on the vector ALUs, uncoalesced key rows), 17.2 us here; 32
+// product a lane on the vector ALUs, uncoalesced key rows), 16.9 us here; 32
 // heads x [4096, 4096]: 12.0 ms, 0.19 ms; head size 256, 8 heads x [570, 570]:
 // 642 us, 30.1 us.
 template <int NT, int QW, int KSPLIT, int BN, bool PARTIAL = false, bool ANY = false>
@@ -685,8 +685,8 @@ __global__ __launch_bounds__(256) void k_flash_combine(half_t* __restrict__ out,
 // vector ALUs 38 % of the time, ~20 vector operations a score (the two do
 // overlap: 8 MFMAs of 128 ns beside 64 exponentials of 238 take 263 ns in two
 // waves of a SIMD, 273 in one).  One MI355X against v_mfma_f32_32x32x2_f32 (which
-// it replaces; in its own tiling): 15 heads of 64 x [3001, 3001] 241 -> 120.5 us, relative
-// error against 64 bits 3.7e-7 -> 2.9e-7; 32 of 64 x 500 queries after 3000
+// it replaces; in its own tiling): 15 heads of 64 x [3001, 3001] 240 -> 121 us, relative
+// error against 64 bits 3.6e-7 -> 2.9e-7; 32 of 64 x 500 queries after 3000
 // keys 309 -> 113 us; 12 of 128 x [1900, 1900] 237 -> 141 us; 9 x [64, 64]
 // 19.1 -> 7.5 us.  Software-pipelined over the blocks (the next block's scores
 // beside this one's exponentials), or with the two waves of a SIMD splitting at

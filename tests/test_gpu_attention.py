@@ -63,14 +63,14 @@ SHAPES = [
     (1, 6, 3, 384, 2000, 2048, 32, 1616),   # many key blocks, D 32, ragged last block
     (1, 9, 3, 2048, 2048, 2048, 64, 0),     # 9 heads x 2048: 32-query tiles, 2 key shares
     (1, 6, 2, 1, 2048, 4096, 64, 2047),  # decode step from a half-full cache
-    (1, 2, 1, 33, 40, 40, 48, 7),        # head size off the matrix-core path
+    (1, 2, 1, 33, 40, 40, 48, 7),        # padded head sizes (more in PADDED_SHAPES)
     (1, 2, 2, 17, 17, 20, 80, 0),
     (1, 2, 1, 9, 300, 300, 256, 291),
     # f16: too few 128-query tile pairs, the key steps split over workgroups
     # (partials merged by a second kernel)
-    (1, 15, 5, 512, 4096, 4096, 64, 3584),   # 8 key chunks: prefill after cached keys
+    (1, 15, 5, 512, 4096, 4096, 64, 3584),   # 5 key chunks a tile: prefill after cached keys
     (1, 48, 8, 512, 2048, 2048, 128, 1536),  # 96 tile pairs, D 128: 2 key chunks
-    (1, 6, 2, 256, 4096, 4096, 96, 3840),    # D 96 (register-staged blocks), 8 chunks
+    (1, 6, 2, 256, 4096, 4096, 96, 3840),    # D 96 (LDS rows of 16 chunks), 8 chunks
     (1, 4, 2, 300, 5000, 5000, 32, 4700),    # D 32, ragged query tile and key count
     (2, 4, 4, 200, 4100, 4160, 64, 3900),    # batch 2, cache rows past kv_len hold NaN
 ]
