@@ -251,53 +251,16 @@ def test_ops_over_one_input_share_its_slots(ctx, dtype, n):
     replay_and_compare(ctx, record, outs)
 
 
-# Recorded ops that share no input: `count` in a launch, each over two arrays.
-def own_arrays(ctx, count, shape):
-    x = [ctx.empty(shape, F32) for _ in range(count + 1)]
-    outs = [ctx.empty(shape, F32) for _ in range(count)]
+@pytest.mark.parametrize("count,n", [(1, 1001), (1, 22000003), (3, 20971520), (3, 20971525)])
+def test_ops_over_arrays_of_their_own(ctx, count, n):
+    """Streamed loads alone in a launch and past 160 MB of reads (20971520
+    elements are the most below), plain ones else: the eager result."""
+    values = norm("own", (min(n, 1 << 16),), F32)
+    x = [ctx.upload(np.resize(np.roll(values, i), n)) for i in range(count + 1)]
+    outs = [ctx.empty((n,), F32) for _ in range(count)]
 
     def record():
         for i, op in zip(range(count), (ctx.add, ctx.mul, ctx.swiglu)):
             op(x[i], x[i + 1], outs[i])
 
-    return x, outs, record
-
-
-@pytest.mark.parametrize("count,n", [(1, 1001), (1, 22000003), (3, 20971520), (3, 20971525)])
-def test_ops_over_arrays_of_their_own(ctx, count, n):
-    """Streamed loads alone in a launch and past 160 MB of reads (20971520
-    elements are the most below), plain ones else: the eager result."""
-    x, outs, record = own_arrays(ctx, count, (n,))
-    values = norm("own", (min(n, 1 << 16),), F32)
-    for i, b in enumerate(x):
-        ctx.copy(ctx.upload(np.resize(np.roll(values, i), n)), b)
     replay_and_compare(ctx, record, outs, reps=2)
-
-
-@pytest.mark.parametrize("count", [1, 3])
-def test_large_ops_over_arrays_of_their_own_take_the_eager_time(ctx, count):
-    """0.99 of it as measured (1.07 and 1.05 with plain loads)."""
-    _, outs, record = own_arrays(ctx, count, (16384, 8192))
-    ctx.capture_begin()
-    record()
-    graph = ctx.capture_end()
-
-    def fastest(call):
-        a, b = ctx.event(), ctx.event()
-        times = []
-        for _ in range(8):
-            ctx.begin()
-            ctx.record(a)
-            for _ in range(4):
-                call()
-            ctx.record(b)
-            ctx.finish()
-            times.append(ctx.elapsed_ms(a, b))
-        ctx.destroy_event(a)
-        ctx.destroy_event(b)
-        return min(times)
-
-    eager = fastest(record)
-    recorded = fastest(lambda: ctx.graph_launch(graph))
-    ctx.graph_destroy(graph)
-    assert recorded <= 1.03 * eager, (recorded, eager)
